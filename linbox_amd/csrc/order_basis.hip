@@ -93,10 +93,8 @@ struct Acc {
     }
 };
 
-// Also clears the grid barrier's arrival count for the M_Basis launch that follows.
-__global__ void __launch_bounds__(256) gather_coeff_major(DevView v, size_t count, uint32_t *out, unsigned *bar)
+__global__ void __launch_bounds__(256) gather_coeff_major(DevView v, size_t count, uint32_t *out)
 {
-    if (blockIdx.x == 0 && threadIdx.x == 0) bar[0] = 0;
     const size_t entries = v.rows * v.cols, total = entries * count;
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) {
         const size_t t = i / entries, e = i - t * entries;
@@ -585,53 +583,102 @@ __global__ void __launch_bounds__(kMbThreads) m_basis_kernel(const uint32_t *__r
 
 // ---------------------------------------------------------------------------
 // M_Basis over several workgroups (orders up to kMcMaxOrder: the PM_Basis
-// base case).  Row operations on sigma act on every column alike, so sigma's
-// columns are split over G workgroups: group g keeps columns [g cw, g cw + cw)
-// of every coefficient of sigma, and rows g cw .. of the serie that those
-// columns meet, resident in LDS for the whole call.  Per step each group
-// forms its share of the discrepancy (the sum over its columns), the shares
-// are exchanged through global memory with one grid barrier, and every group
-// then runs the same sort, elimination and bookkeeping on the summed
-// discrepancy (so every group takes the same decisions) and applies the row
-// operations to its own columns.  The steps follow m_basis_kernel and the
-// reference's order-basis.h:346-600; the differences are in how they are
-// computed:
-//  * the shift sort handles one value at a time: the reference's selection
-//    sort places the elements of the smallest remaining value in order of
-//    position, and each element it displaces follows a chain of those
-//    positions, which one pass of the wave resolves;
-//  * each wave keeps its rows of [R | Z] in registers during elimination and
-//    stores a row only when it is that wave's candidate for the next pivot;
-//  * a x - b y takes one Montgomery reduction (a x + b (p - y) < 2^64 for
-//    p < 2^31), and rows carry no scale: every row below pivot j is
-//    multiplied by its entry a_j, so a row's scale is the product of the a_j
-//    of the pivots above it, read from a prefix product at the end.
+// base case).  The steps follow m_basis_kernel and order-basis.h:346-600, but
+// instead of summing the discrepancy from sigma and the serie at each step, the
+// row operations are applied to the serie itself (the residual
+// x^-k sigma.serie, whose lowest coefficient is the discrepancy) and to sigma.
+// Row operations act on every column alike, so the columns are split over G
+// workgroups: group g keeps cs columns of the residual serie (all
+// coefficients) and cj columns of sigma in LDS, and no group needs another's
+// columns except to see the discrepancies.  Those come in blocks of B steps:
+// every group also holds the next B coefficients of the residual in full
+// (the window), runs the B eliminations on it redundantly (so all groups take
+// the same decisions), and the groups exchange the following B coefficients
+// through global memory at one grid barrier per block.
+//
+// What bounds a step is the serial chain of pivots, so the elimination goes in
+// panels of four rows:
+//  * rows are held in registers, kMbPanel rows (one panel) or two panels per
+//    wave, NC lanes to a row, values centred in [-h, h], h = (p-1)/2;
+//  * on its turn a wave runs an in-place, division-free Gauss-Jordan
+//    elimination of its panel (row operations inside the panel), which gives
+//    D and H = D P_C^-1 P for the panel's pivot columns C, and publishes them;
+//  * every other row takes the whole panel in one update with a single
+//    reduction: x <- D x - (x_C) H off C and x_C <- (x_C) H on C.
+// These are column operations on the discrepancy: they leave pivot rows with
+// one nonzero entry and turn a non-pivot row into its combination of the pivot
+// rows times the product of the D's, so no separate combination is carried.
+// The row rank profile and the combinations do not depend on which columns
+// are chosen, so the result is that of a pivot-by-pivot elimination.
+//
+// Per step: the elimination; then, between two barriers, one wave inverts the
+// product of the D's, one sorts the shifts for the next step, and the others
+// form sums over the pivot rows: for the window with the combinations still
+// unscaled (one Montgomery product per entry scales the sum once the inverse
+// is known), and for the group's own columns with the previous step's
+// combinations, so that neither waits for the inverse; then the pivot rows
+// are multiplied by x.
+//
+// Measured at 64 x 32, order 32, p = 998244353: 553 us per base case
+// against 922 us for the form before it (discrepancies summed from sigma, a grid
+// barrier per step, pivot-by-pivot elimination of [R | Z]), and PM_Basis at order
+// 4096 84.6 ms against 132.4 ms (8 x 4 at order 512: 4.8 against 6.1 ms, 128 x 32
+// at order 128: 3.3 against 6.7 ms).  A step takes about 39 k cycles: eight panels at
+// 3.3 k each (a lone wave issues an instruction every five cycles at best, and a
+// panel is some 400 of them with three LDS hand-offs), 5 k for the inverse and the
+// sums, 5 k for scaling and shifting, and a quarter of the 12 k of an exchange.
 constexpr int kMcMaxOrder = 32;
 constexpr int kMcMaxGroups = 64;
-constexpr int kMcLdsWords = 36864;  // dynamic LDS words (the static arrays take the rest of the 160 KiB)
-constexpr unsigned kMcSpinLimit = 1u << 24;  // polls of the grid barrier before it reports a failure
+constexpr int kMcLdsWords = 38400;  // dynamic LDS words (the static arrays take 9.3 of the other 10 KiB)
+constexpr unsigned kMcSpinLimit = 1u << 24;  // polls of a wait before it reports a failure
+constexpr int kMbPanel = 4;          // rows per panel
+constexpr int kMcMaxBlock = 4;       // steps per exchange
+constexpr int kMcSumWaves = kMbWaves - 2;  // waves 0 and 1 invert and sort meanwhile
+constexpr int kMcMaxTasks = 4;       // window tiles per wave (cols_split sees to it)
 
-// a x - b y mod p on Montgomery forms, ny = p - y (odd p < 2^31)
-__device__ __forceinline__ uint32_t amb1(uint32_t a, uint32_t x, uint32_t b, uint32_t ny, uint32_t p, uint32_t pinv)
-{
-    const uint64_t t = (uint64_t)a * x + (uint64_t)b * ny;
-    const uint32_t q = (uint32_t)t * pinv;
-    const uint32_t r = (uint32_t)((t + (uint64_t)q * p) >> 32);
-    return r >= p ? r - p : r;
-}
+// Constants of one odd prime below 2^31 for arithmetic on centred values.
+struct Centred {
+    uint32_t p, pinv, h, one;  // p^-1 mod 2^32, (p-1)/2, 2^32 mod p
+    int32_t c8[7];             // 2^(8d) mod p, centred
 
-// All groups of the grid meet here for the `count`-th time.  bar[0] counts
-// arrivals, bar[1] is set when a poll limit runs out (the host reports the
-// call as failed, and later barriers no longer wait).  The shares exchanged
-// through the barrier are written and read with agent-scope atomics.
-__device__ __forceinline__ void grid_barrier(unsigned *bar, unsigned count)
+    __device__ __forceinline__ int32_t from(uint32_t x) const { return (int32_t)(x > h ? x - p : x); }
+    __device__ __forceinline__ uint32_t canonical(int32_t x) const
+    {
+        return (uint32_t)x + ((uint32_t)(x >> 31) & p);
+    }
+    // t 2^-32 mod p, centred, for -p <= t >> 32 < p: with m = t p^-1 mod 2^32 the low
+    // words of t and m p agree, so the high words' difference is exact; h + it lies in [0, 2p)
+    __device__ __forceinline__ int32_t redc(int64_t t) const
+    {
+        const int32_t hi = (int32_t)(t >> 32), m = (int32_t)((uint32_t)t * pinv);
+        uint32_t u = (uint32_t)hi + ((uint32_t)(hi >> 31) & p) + h;
+        u -= (uint32_t)mulhi_s32(m, (int32_t)p);
+        return (int32_t)(csub(u, p) - h);
+    }
+    __device__ __forceinline__ int32_t mul(int32_t x, int32_t y) const { return redc((int64_t)x * y); }
+    // x - y of centred values, centred
+    __device__ __forceinline__ int32_t sub(int32_t x, int32_t y) const
+    {
+        const int32_t d = x - y;  // in [-(p-1), p-1]
+        uint32_t u = (uint32_t)d + h;
+        u += (uint32_t)((int32_t)u >> 31 & (int32_t)p) & (uint32_t)(d >> 31);
+        return (int32_t)(csub(u, p) - h);
+    }
+};
+
+// All groups of the grid meet here: bar[0] counts arrivals and is awaited to
+// reach `target`; bar[1] is set when a poll limit runs out (the host reports the
+// call as failed, and later barriers no longer wait).  What the groups exchange is
+// written and read with agent-scope atomics, which go past the caches, so the
+// barrier only waits for the stores (no write-back or invalidation of an L2).
+__device__ __forceinline__ void grid_barrier(unsigned *bar, unsigned target)
 {
+    __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (threadIdx.x == 0) {
-        __hip_atomic_fetch_add(bar, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned target = count * gridDim.x;
+        __hip_atomic_fetch_add(bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         unsigned polls = 0;
-        while (__hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
+        while ((int)(__hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - target) < 0) {
             // the failure flag only matters once a limit ran out: read it now and then
             if ((polls & 255) == 255 && __hip_atomic_load(bar + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
             if (++polls == kMcSpinLimit) {
@@ -640,445 +687,775 @@ __device__ __forceinline__ void grid_barrier(unsigned *bar, unsigned count)
             }
             __builtin_amdgcn_s_sleep(1);
         }
-        __atomic_thread_fence(__ATOMIC_ACQUIRE);
     }
     __syncthreads();
 }
 
-// sum of x[j] y[j*ystride], len terms, on two independent accumulators
-__device__ __forceinline__ void dot2(AccSmall &a0, AccSmall &a1, const uint32_t *x, const uint32_t *y, int ystride,
-                                     int len, uint32_t f62)
+// i / d for 0 <= i < 2^20, d > 0, given r = 1 / (float)d: (i + 1/2) r is at least
+// 1/(2d) away from an integer, more than the products' rounding
+__device__ __forceinline__ int quot(int i, float r) { return (int)(((float)i + 0.5f) * r); }
+
+// Montgomery product of canonical words by 32-bit multiplications, whose latency is
+// half that of a 64-bit multiply-add: x y - m p with m = x y p^-1 mod 2^32
+__device__ __forceinline__ uint32_t mont_pos(uint32_t x, uint32_t y, const Centred &K)
 {
-    int j = 0;
-    for (; j + 3 < len; j += 4) {
-        const uint32_t x0 = x[j], x1 = x[j + 1], x2 = x[j + 2], x3 = x[j + 3];
-        const uint32_t y0 = y[j * ystride], y1 = y[(j + 1) * ystride], y2 = y[(j + 2) * ystride],
-                       y3 = y[(j + 3) * ystride];
-        a0.add2(x0, y0, x1, y1, f62);
-        a1.add2(x2, y2, x3, y3, f62);
-    }
-    for (; j < len; ++j) a0.add1(x[j], y[j * ystride], f62);
+    const uint32_t m = x * y * K.pinv, r = __umulhi(x, y) - __umulhi(m, K.p), s = r + K.p;
+    return s < r ? s : r;
 }
 
-__device__ __forceinline__ uint32_t sum2(const AccSmall &a0, const AccSmall &a1, uint32_t p, uint64_t mu)
+// Sums over an operation's pivot rows for a tile of 16 of its non-pivot rows and
+// 16 columns, on INT8 matrix instructions: out[r] is the sum for row
+// 4 (lane >> 4) + r and this lane's column, as redc returns it.  A word's four
+// balanced digits are four neighbouring bytes of the inner dimension, so the words
+// themselves are the A operand, and with the other word's digits in reverse,
+// shifted by e bytes, one 64-deep product gives the digit products of one
+// anti-diagonal for 16 pivots: seven products per 16 pivots, of which 16/28 is
+// needed, against no repacking into digit planes.  The sums stay below
+// 64 * 4 * 2^14, so the diagonals recombine in 64 bits without a reduction.
+// x: combinations, xs words per non-pivot row (up to the next multiple of 32 pivots
+// other words of the LDS may be read, and count for nothing); col: this lane's
+// column of M; poff: the pivot rows' offsets (any up to that multiple).
+// On 64-bit multiply-adds with four rows per thread these sums were bound by LDS
+// reads (each word read once per lane that needed it).
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ void tile_sums(int32_t (&out)[4], const int32_t *x, int xs, const int32_t *col,
+                                          const int *poff, int rank, int lane, const Centred &K)
 {
-    return csub(a0.get(p, mu, 0) + a1.get(p, mu, 0), p);
-}
-
-// G = gridDim.x groups of kMbThreads threads; ROWS >= m / kMbWaves rows of the
-// elimination per wave.  S: serie, coefficient-major S[(t*m + j)*n + c]; part:
-// 2 x G x m x n words of exchanged discrepancy shares; bar: the grid barrier's
-// two words, zero at launch.  Dynamic LDS, in words: W (order+1) x m x cw
-// (W[(l*m + phys)*cw + jj], coefficient l of sigma's column g*cw+jj in
-// physical row phys), Sg order x cw x n (serie rows of the group's columns),
-// V m x (2n+1) (row r of the discrepancy under elimination, [R_r | Z_r],
-// logical order), D m x n (discrepancy before elimination, by physical row).
-// out_count: coefficients of sigma written (zero above the degree); 0 writes
-// degree+1 of them.
-template <int ROWS>
-__global__ void __launch_bounds__(kMbThreads) m_basis_cols_kernel(
-    const uint32_t *__restrict__ S, DevView out, uint64_t *__restrict__ shift_io, uint64_t *__restrict__ deg_out,
-    uint32_t *__restrict__ part, unsigned *__restrict__ bar, int order, int m, int n, int cw, int out_count,
-    uint32_t p, uint64_t mu, uint32_t f62, uint32_t pinv, uint32_t r2m, uint32_t one)
-{
-    const int G = gridDim.x, g = blockIdx.x, j0 = g * cw;
-    const int cols = m - j0 < cw ? m - j0 : cw;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int mn = m * n, vs = 2 * n + 1, cst = m * cw;  // cst: words per coefficient of the group's W
-    extern __shared__ uint32_t dyn[];
-    uint32_t *W = dyn;
-    uint32_t *Sg = W + (order + 1) * cst;
-    uint32_t *V = Sg + order * cw * n;
-    uint32_t *D = V + m * vs;
-    __shared__ uint64_t shift[kMbMaxM], degree[kMbMaxM], tmp64[kMbMaxM], tmp64b[kMbMaxM];
-    __shared__ int rowmap[kMbMaxM], tmpmap[kMbMaxM], oldrow[kMbMaxM], pivot_of[kMbMaxM], comp[kMbMaxM],
-        cidx[kMbMaxM], was_piv[kMbMaxM], qtab[kMbMaxM], piv_s[kMbMaxN], piv_c[kMbMaxN];
-    __shared__ uint32_t pref[kMbMaxN + 1], rinv[kMbMaxM], piv_a[kMbMaxN];  // pivots: row, column, entry
-    __shared__ int s_maxdeg, s_nc, s_npub, s_turn;
-
-    for (int i = tid; i < (order + 1) * cst; i += kMbThreads) {
-        const int q = i / cw, jj = i - q * cw, ph = q % m, l = q / m;
-        W[i] = (l == 0 && ph == j0 + jj) ? 1u : 0u;
-    }
-    for (int i = tid; i < order * cw * n; i += kMbThreads) {
-        const int q = i / n, c = i - q * n, jj = q % cw, t = q / cw;
-        Sg[i] = jj < cols ? S[((size_t)t * m + j0 + jj) * n + c] : 0u;
-    }
-    for (int i = tid; i < m; i += kMbThreads) {
-        rowmap[i] = i;
-        shift[i] = shift_io[i];
-        degree[i] = 0;
-        was_piv[i] = 0;
-    }
-    if (tid == 0) {
-        s_maxdeg = 0;
-        pref[0] = one;
-    }
-    __syncthreads();
-    unsigned nbar = 0;  // grid barriers passed (the same count in every group)
-    const uint64_t below = (1ull << lane) - 1;
-
-    for (int k = 0; k < order; ++k) {
-        const int maxdeg = s_maxdeg, lim = k < maxdeg ? k : maxdeg;
-        // ---- 1. selection sort of the shift (order-basis.h:388-399), one value at a time ----
-        if (wave == 0) {
-            const bool v0 = lane < m, v1 = lane + 64 < m;
-            uint64_t k0 = v0 ? shift[lane] : 0, k1 = v1 ? shift[lane + 64] : 0;
-            int o0 = lane, o1 = lane + 64;
-            for (int start = 0; start < m - 1;) {
-                const bool a0 = v0 && lane >= start, a1 = v1 && lane + 64 >= start;
-                uint64_t lo = ~(uint64_t)0, hi = 0;
-                if (a0) { lo = k0; hi = k0; }
-                if (a1) { lo = k1 < lo ? k1 : lo; hi = k1 > hi ? k1 : hi; }
-                lo = __ockl_wfred_min_u64(lo);
-                hi = __ockl_wfred_max_u64(hi);
-                if (lo == hi) break;  // what remains holds one value: every later swap is the identity
-                // the smallest value's positions q_0 < q_1 < ... (c of them): step start+j
-                // swaps positions start+j and q_j, since the value's elements not yet placed
-                // never move and q_j >= start+j
-                const bool m0 = a0 && k0 == lo, m1 = a1 && k1 == lo;
-                const uint64_t b0 = __ballot(m0), b1 = __ballot(m1);
-                const int n0 = __popcll(b0), end = start + n0 + __popcll(b1);
-                const int r0 = __popcll(b0 & below), r1 = n0 + __popcll(b1 & below);
-                if (m0) qtab[r0] = lane;
-                if (m1) qtab[r1] = lane + 64;
-                __builtin_amdgcn_s_waitcnt(0);
-                __builtin_amdgcn_wave_barrier();
-                // destination: start+rank for the value's elements; an element displaced
-                // from x in [start, end) goes to q_{x-start}, and on while that is below end
-                auto dest = [&](int x, bool isv, int rk) -> int {
-                    if (isv) return start + rk;
-                    if (x < start || x >= end) return x;
-                    int y = qtab[x - start];
-                    while (y < end) y = qtab[y - start];
-                    return y;
-                };
-                const int d0 = v0 ? dest(lane, m0, r0) : lane;
-                const int d1 = v1 ? dest(lane + 64, m1, r1) : lane + 64;
-                __builtin_amdgcn_s_waitcnt(0);
-                __builtin_amdgcn_wave_barrier();
-                if (v0) { tmp64[d0] = k0; tmpmap[d0] = o0; }
-                if (v1) { tmp64[d1] = k1; tmpmap[d1] = o1; }
-                __builtin_amdgcn_s_waitcnt(0);
-                __builtin_amdgcn_wave_barrier();
-                if (v0) { k0 = tmp64[lane]; o0 = tmpmap[lane]; }
-                if (v1) { k1 = tmp64[lane + 64]; o1 = tmpmap[lane + 64]; }
-                __builtin_amdgcn_s_waitcnt(0);
-                __builtin_amdgcn_wave_barrier();
-                start = end;
+    i32x4 acc[7];
+#pragma unroll
+    for (int d = 0; d < 7; ++d) acc[d] = i32x4{0, 0, 0, 0};
+    const int kg = (lane >> 4) * 4;
+    const int32_t *xr = x + (lane & 15) * xs + kg;
+    for (int b0 = 0; b0 < rank; b0 += 32) {
+        // 32 pivots' words at a time, all loads first
+        int4 po[2];
+        i32x4 a[2];
+        int32_t w[2][4];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) po[h] = *reinterpret_cast<const int4 *>(poff + b0 + 16 * h + kg);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) a[h] = *reinterpret_cast<const i32x4 *>(xr + b0 + 16 * h);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            w[h][0] = col[po[h].x];
+            w[h][1] = col[po[h].y];
+            w[h][2] = col[po[h].z];
+            w[h][3] = col[po[h].w];
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            uint32_t rev[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (b0 + 16 * h + kg + j >= rank) w[h][j] = 0;  // a's words there are arbitrary
+                rev[j] = __builtin_bswap32((uint32_t)w[h][j] + 0x80808080u) ^ 0x80808080u;
+                a[h][j] = (int)(((uint32_t)a[h][j] + 0x80808080u) ^ 0x80808080u);
             }
-            // gather by origin (all lanes read before any lane writes)
-            uint64_t dg0 = 0, dg1 = 0;
-            int rm0 = 0, rm1 = 0;
-            if (v0) { dg0 = degree[o0]; rm0 = rowmap[o0]; }
-            if (v1) { dg1 = degree[o1]; rm1 = rowmap[o1]; }
+#pragma unroll
+            for (int d = 0; d < 7; ++d) {
+                i32x4 bv;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    bv[j] = (int)(d <= 3 ? rev[j] >> (8 * (3 - d)) : rev[j] << (8 * (d - 3)));
+                acc[d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[h], bv, acc[d], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        int64_t t = 0;
+#pragma unroll
+        for (int d = 0; d < 7; ++d) t += (int64_t)acc[d][r] * K.c8[d];
+        out[r] = K.redc(t);
+    }
+}
+
+// Geometry of one launch, the same in every group.
+struct ColsShape {
+    int order, m, n;
+    int cs, cj;  // residual serie and sigma columns per group
+    int B;       // steps per block
+    int rs;      // words per row of M
+    int xs;      // words per row of the combinations: min(m, n) rounded up to 16, and four more
+    int xm;      // their rows: m rounded up to a multiple of 16
+    int xb;      // 1: combinations of two steps are kept (B > 1), 0: of one
+};
+
+// G = gridDim.x groups of kMbThreads threads.  NC lanes hold a row of the
+// discrepancy (n <= NC), PPW panels per wave (m <= 64 PPW).  part: 2 x m x (B n)
+// words of exchanged coefficients; bar: the grid barrier's two words, bar[0]
+// at bar_base when the launch begins.  Dynamic LDS: H (a vector of four words
+// per panel and lane), the combinations X of one or two steps (per non-pivot row, one word
+// per pivot), the panels' diagonals, and M: per physical row the
+// window (coefficient t of the block at t*n + column), the group's residual
+// columns and its sigma columns.  out_count: coefficients of sigma written
+// (zero above the degree); 0 writes degree+1 of them.
+template <int NC, int PPW>
+__global__ void __launch_bounds__(kMbThreads) m_basis_cols_kernel(DevView serie, DevView out,
+                                                                  uint64_t *__restrict__ shift_io,
+                                                                  uint64_t *__restrict__ deg_out, int32_t *part,
+                                                                  unsigned *__restrict__ bar, unsigned bar_base,
+                                                                  ColsShape C, int out_count, Centred K)
+{
+    constexpr int RPR = 64 / NC;             // rows per register
+    constexpr int PR = kMbPanel / RPR;       // registers per panel
+    constexpr int NREG = PPW * PR;
+    const int order = C.order, m = C.m, n = C.n, rs = C.rs, xs = C.xs;
+    const int G = gridDim.x, c0 = blockIdx.x * C.cs, j0 = blockIdx.x * C.cj;
+    const int ncs = c0 < n ? (n - c0 < C.cs ? n - c0 : C.cs) : 0;  // this group's serie columns
+    const int ncj = j0 < m ? (m - j0 < C.cj ? m - j0 : C.cj) : 0;  // and sigma columns
+    const int tid0 = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid0 >> 6);
+    const int npan = (m + kMbPanel - 1) / kMbPanel;
+    const int os = C.B * n, oj = os + C.cs * order;  // columns of M: window, residual, sigma
+    const uint32_t p = K.p, npinv = 0u - K.pinv;
+    // The thread's index as a value the compiler cannot look through: used in each
+    // phase, it keeps lane conditions from being hoisted out of the step loop,
+    // where they would fill the scalar registers and spill.
+    auto fresh_tid = [&]() -> int {
+        int t = tid0;
+        asm volatile("" : "+v"(t));
+        return t;
+    };
+
+    extern __shared__ int4 dyn4[];
+    int4 *H = dyn4;                              // [panel][NC]
+    int32_t *X = (int32_t *)(H + npan * NC);     // [step & xb][non-pivot row][xs], a word per pivot
+    int32_t *Dz = X + (1 + C.xb) * C.xm * xs;    // [panel][NC]
+    int32_t *M = Dz + npan * NC;                 // [physical row][rs]
+    __shared__ int4 pcol[kMbMaxM / kMbPanel];    // 4 x pivot columns of a panel, in H's slot order
+    __shared__ int pbits[kMbMaxM / kMbPanel];     // its pivot rows, one bit each
+    __shared__ uint32_t pdet[kMbMaxM / kMbPanel]; // its D
+    __shared__ uint64_t shift[kMbMaxM], degree[kMbMaxM], tmp64[kMbMaxM], tmp64b[kMbMaxM];
+    __shared__ int rowmap[2][kMbMaxM], tmpmap[kMbMaxM], qtab[kMbMaxM];
+    __shared__ __align__(16) int poff[2][kMbMaxN];  // M offsets of pivot rows,
+    __shared__ __align__(16) int noff[2][kMbMaxM + 16];  // and of the other rows
+    __shared__ int op_rank[2], op_lim[2];
+    __shared__ int bidx[kMbMaxN];      // pivot index of a column, -1 without one
+    __shared__ int32_t col_e[kMbMaxN];  // product of the D's of the panels before the column's
+    __shared__ uint32_t s_e;   // product of the D's of the panels booked
+    __shared__ int32_t s_inv[2];
+    __shared__ int s_book;     // panels booked
+    __shared__ int s_maxdeg;
+    __shared__ unsigned s_pub;  // panels published | rank << 8 | (rank == n) << 16
+
+    // ---- initial state ----
+    {
+        const int tid = tid0;
+        for (int i = tid; i < m * ncj * (order + 1); i += kMbThreads) {
+            const int q = i / (order + 1), l = i - q * (order + 1), ph = q / ncj, jj = q - ph * ncj;
+            M[ph * rs + oj + jj * (order + 1) + l] = (l == 0 && ph == j0 + jj) ? 1 : 0;
+        }
+        for (int i = tid; i < m * ncs * order; i += kMbThreads) {
+            const int q = i / order, t = i - q * order, ph = q / ncs, cc = q - ph * ncs;
+            M[ph * rs + os + cc * order + t] = K.from(serie.base[view_index(serie, (size_t)ph * n + c0 + cc, t)]);
+        }
+        const int b0 = C.B < order ? C.B : order;
+        for (int i = tid; i < m * n; i += kMbThreads) {
+            const int ph = i / n, c = i - ph * n;
+            for (int t = 0; t < b0; ++t) M[ph * rs + t * n + c] = K.from(serie.base[view_index(serie, i, t)]);
+        }
+        for (int i = tid; i < m; i += kMbThreads) {
+            rowmap[0][i] = i;
+            shift[i] = shift_io[i];
+            degree[i] = 0;
+        }
+        if (tid < 2 * (kMbMaxM + 16)) noff[0][tid] = 0;
+        if (tid < 2 * kMbMaxN) poff[0][tid] = 0;
+        if (tid < kMbMaxN) bidx[tid] = -1;
+        if (tid < kMbMaxM / kMbPanel) pbits[tid] = 0;
+        if (tid == 0) {
+            s_maxdeg = 0;
+            op_lim[0] = 0;
+            s_pub = 0;
+            s_book = 0;
+        }
+    }
+    __syncthreads();
+
+    // Selection sort of the shift (order-basis.h:388-399), one value at a time, by
+    // one wave: the reference's sort places the elements of the smallest remaining
+    // value in order of position, and each element it displaces follows a chain of
+    // those positions, which one pass of the wave resolves.  shift, degree and
+    // rmap are permuted alike.
+    auto sort_rows = [&](int *rmap, int lane) {
+        const uint64_t below = (1ull << lane) - 1;
+        const bool v0 = lane < m, v1 = lane + 64 < m;
+        uint64_t k0 = v0 ? shift[lane] : 0, k1 = v1 ? shift[lane + 64] : 0;
+        int o0 = lane, o1 = lane + 64;
+        for (int start = 0; start < m - 1;) {
+            const bool a0 = v0 && lane >= start, a1 = v1 && lane + 64 >= start;
+            uint64_t lo = ~(uint64_t)0, hi = 0;
+            if (a0) { lo = k0; hi = k0; }
+            if (a1) { lo = k1 < lo ? k1 : lo; hi = k1 > hi ? k1 : hi; }
+            lo = __ockl_wfred_min_u64(lo);
+            hi = __ockl_wfred_max_u64(hi);
+            if (lo == hi) break;  // what remains holds one value: every later swap is the identity
+            // the smallest value's positions q_0 < q_1 < ... (c of them): step start+j
+            // swaps positions start+j and q_j, since the value's elements not yet placed
+            // never move and q_j >= start+j
+            const bool m0 = a0 && k0 == lo, m1 = a1 && k1 == lo;
+            const uint64_t b0 = __ballot(m0), b1 = __ballot(m1);
+            const int n0 = __popcll(b0), end = start + n0 + __popcll(b1);
+            const int r0 = __popcll(b0 & below), r1 = n0 + __popcll(b1 & below);
+            if (m0) qtab[r0] = lane;
+            if (m1) qtab[r1] = lane + 64;
             __builtin_amdgcn_s_waitcnt(0);
             __builtin_amdgcn_wave_barrier();
-            if (v0) { shift[lane] = k0; degree[lane] = dg0; rowmap[lane] = rm0; }
-            if (v1) { shift[lane + 64] = k1; degree[lane + 64] = dg1; rowmap[lane + 64] = rm1; }
-            // rows to sum: those that were not pivots at the previous step
-            int base = 0;
-            for (int h = 0; h < m; h += 64) {
-                const int r = h + lane;
-                const bool need = r < m && !was_piv[h == 0 ? rm0 : rm1];
-                const uint64_t bal = __ballot(need);
-                const int idx = base + __popcll(bal & below);
-                if (r < m) cidx[r] = need ? idx : -1;
-                if (need) comp[idx] = r;
-                base += __popcll(bal);
+            // destination: start+rank for the value's elements; an element displaced
+            // from x in [start, end) goes to q_{x-start}, and on while that is below end
+            auto dest = [&](int x, bool isv, int rk) -> int {
+                if (isv) return start + rk;
+                if (x < start || x >= end) return x;
+                int y = qtab[x - start];
+                while (y < end) y = qtab[y - start];
+                return y;
+            };
+            const int d0 = v0 ? dest(lane, m0, r0) : lane;
+            const int d1 = v1 ? dest(lane + 64, m1, r1) : lane + 64;
+            __builtin_amdgcn_s_waitcnt(0);
+            __builtin_amdgcn_wave_barrier();
+            if (v0) { tmp64[d0] = k0; tmpmap[d0] = o0; }
+            if (v1) { tmp64[d1] = k1; tmpmap[d1] = o1; }
+            __builtin_amdgcn_s_waitcnt(0);
+            __builtin_amdgcn_wave_barrier();
+            if (v0) { k0 = tmp64[lane]; o0 = tmpmap[lane]; }
+            if (v1) { k1 = tmp64[lane + 64]; o1 = tmpmap[lane + 64]; }
+            __builtin_amdgcn_s_waitcnt(0);
+            __builtin_amdgcn_wave_barrier();
+            start = end;
+        }
+        // gather by origin (all lanes read before any lane writes)
+        uint64_t dg0 = 0, dg1 = 0;
+        int rm0 = 0, rm1 = 0;
+        if (v0) { dg0 = degree[o0]; rm0 = rmap[o0]; }
+        if (v1) { dg1 = degree[o1]; rm1 = rmap[o1]; }
+        __builtin_amdgcn_s_waitcnt(0);
+        __builtin_amdgcn_wave_barrier();
+        if (v0) { shift[lane] = k0; degree[lane] = dg0; rmap[lane] = rm0; }
+        if (v1) { shift[lane + 64] = k1; degree[lane + 64] = dg1; rmap[lane + 64] = rm1; }
+    };
+    if (wave == 1) sort_rows(rowmap[0], tid0 & 63);
+    __syncthreads();
+    unsigned nbar = 0;
+    // without an exchange nothing else keeps group 0 from writing the shift before
+    // another group has read it
+    if (G > 1 && order <= C.B) grid_barrier(bar, bar_base + ++nbar * (unsigned)G);
+
+    // Column u (-1: none) of the non-pivot rows of a tile minus the tile's sums, which
+    // are of unscaled combinations: times the inverse of the D's.
+    auto apply_tile = [&](const int32_t (&sum)[4], int ob, int i0, int nn, int u, int lane) {
+        const int i = i0 + 4 * (lane >> 4);
+        const int32_t inv = s_inv[ob];
+        const int4 no = *reinterpret_cast<const int4 *>(&noff[ob][i]);
+        const int off[4] = {no.x, no.y, no.z, no.w};
+        int32_t old[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) old[r] = M[off[r] + (u < 0 ? 0 : u)];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) old[r] = K.sub(old[r], K.mul(sum[r], inv));
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (u >= 0 && i + r < nn) M[off[r] + u] = old[r];
+    };
+    // The group's own columns under the operation of step kk: non-pivot rows -=
+    // combination . pivot rows (:509-517), one tile per wave at a time, tiles
+    // [t, count) by nt waves.  Residual coefficients up to kk are zero from here on;
+    // sigma has op_lim+1 coefficients.
+    auto own_update = [&](int kk, bool residual, int t, int nt, int lane) {
+        const int ob = kk & 1, rank = __builtin_amdgcn_readfirstlane(op_rank[ob]),
+                  lim = __builtin_amdgcn_readfirstlane(op_lim[ob]), nn = m - rank, len = order - kk - 1;
+        const int vs = residual ? ncs * len : 0, vt = vs + ncj * (lim + 1);
+        if (!rank || !nn || !vt) return;
+        const int nct = (vt + 15) >> 4, ntile = nct * ((nn + 15) >> 4);
+        for (int i = t, rq = 0, ct = t; i < ntile; i += nt, ct += nt) {
+            while (ct >= nct) ct -= nct, ++rq;
+            const int v = 16 * ct + (lane & 15), vc = v < vt ? v : 0;
+            int u;
+            if (vc < vs) {
+                const int cc = ncs > 1 ? quot(vc, 1.0f / (float)len) : 0;
+                u = os + cc * order + kk + 1 + (vc - cc * len);
+            } else {
+                const int jj = quot(vc - vs, 1.0f / (float)(lim + 1));
+                u = oj + jj * (order + 1) + (vc - vs - jj * (lim + 1));
             }
-            if (lane == 0) s_nc = base;
+            int32_t sum[4];
+            tile_sums(sum, X + ((ob & C.xb) * C.xm + 16 * rq) * xs, xs, M + u, poff[ob], rank, lane, K);
+            apply_tile(sum, ob, 16 * rq, nn, v < vt ? u : -1, lane);
         }
-        __syncthreads();
-        // ---- 2. this group's share of the discrepancy (order-basis.h:416-456) ----
-        const int nc = s_nc, slot = (int)(nbar & 1);
-        for (int o = tid; o < nc * n; o += kMbThreads) {
-            const int i = o / n, c = o - i * n, ph = rowmap[comp[i]];
-            AccSmall acc0, acc1;
-            for (int l = 0; l <= lim; ++l)
-                dot2(acc0, acc1, W + l * cst + ph * cw, Sg + (k - l) * cw * n + c, n, cols, f62);
-            const uint32_t v = sum2(acc0, acc1, p, mu);
-            if (G == 1) V[comp[i] * vs + c] = v;
-            else __hip_atomic_store(part + (slot * G + g) * mn + o, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (G > 1 && nc) grid_barrier(bar, ++nbar);
-        else __syncthreads();
-        // the summed discrepancy, its Montgomery form in V, an empty Z part; rows
-        // that were pivots at the previous step keep theirs: x.sigma_t has the same
-        // discrepancy (:446-456).  One row per wave, one column per lane.
-        for (int r = wave; r < m; r += kMbWaves) {
-            const int ph = rowmap[r];
-            const bool wp = was_piv[ph] != 0;
-            if (lane < n) {
-                uint32_t v;
-                if (wp) {
-                    v = D[ph * n + lane];
-                } else if (G == 1) {
-                    v = V[r * vs + lane];
-                } else {
-                    // plain loads, eight in flight: the grid barrier's acquire fence has
-                    // invalidated this CU's caches
-                    const uint32_t *q = part + slot * G * mn + cidx[r] * n + lane;
-                    uint64_t sum = 0;
-                    int h = 0;
-                    for (; h + 16 <= G; h += 16) {
-                        uint32_t t[16];
+    };
+    // Pivot rows of a step times x (:573-580): words [lo, hi) of their rows of M move up
+    // by `step` words.  A wave takes rows b and b + kMbWaves and reads kShiftChunks x 64
+    // words of each, from the top down, before it writes any of them, so its writes
+    // reach only words already read.  What enters an own residual column is a dead
+    // coefficient; sigma's columns get a zero at the bottom.
+    constexpr int kShiftChunks = 2, kShiftWords = 64 * kShiftChunks;
+    typedef int32_t ShiftWords[2][kShiftChunks];
+    auto shift_read = [&](ShiftWords &v, const int *po, int rank, int b, int lo, int top, int step, int lane) {
 #pragma unroll
-                        for (int j = 0; j < 16; ++j) t[j] = q[(h + j) * mn];
+        for (int r = 0; r < 2; ++r)
 #pragma unroll
-                        for (int j = 0; j < 16; ++j) sum += t[j];
-                    }
-                    for (; h + 8 <= G; h += 8) {
-                        uint32_t t[8];
-#pragma unroll
-                        for (int j = 0; j < 8; ++j) t[j] = q[(h + j) * mn];
-#pragma unroll
-                        for (int j = 0; j < 8; ++j) sum += t[j];
-                    }
-                    for (; h < G; ++h) sum += q[h * mn];
-                    v = red64(sum, p, mu);
-                }
-                D[ph * n + lane] = v;
-                V[r * vs + lane] = mont(v, r2m, p, pinv);
-                V[r * vs + n + lane] = 0;
+            for (int c = 0; c < kShiftChunks; ++c) {
+                const int w = top - 64 * (c + 1) + lane;
+                v[r][c] = b + r * kMbWaves < rank && w >= lo ? M[po[b + r * kMbWaves] + w - step] : 0;
             }
-        }
-        for (int i = tid; i < m; i += kMbThreads) pivot_of[i] = -1;
-        if (tid == 0) {
-            s_npub = 0;
-            s_turn = 0;
-        }
-        __syncthreads();
-        // ---- 3. row rank profile and combinations (the PLUQ of :470-488) ----
-        // Wave w holds rows r0 = w*ROWS .. r0+ROWS-1 of [R | Z] in registers (lane j: words
-        // j and j+64).  Waves take turns in order: on its turn wave w runs through its own
-        // rows, each against the pivots before it, publishes each pivot's vector as it finds
-        // it (s_npub) and then hands the turn on (s_turn).  Until its turn a wave applies to
-        // its rows every pivot already published, so the waves below apply a block's pivots
-        // while it is still being eliminated.  Every row below a pivot meets it once, in pivot
-        // order, as in a pivot-by-pivot elimination.  Pivot vector j: [R_s | Z_s (j words) |
-        // -scale_s | 0 ...]; a row below it becomes a [R_r | Z_r] - b [pivot vector],
-        // a = R_s[c_j], b = R_r[c_j].  The counters are workgroup-scope release/acquire
-        // words in LDS; a wait that runs past its poll limit raises the failure flag, and
-        // every later wait in the call then gives up at once.
-        const int r0 = wave * ROWS;
-        uint32_t x0[ROWS], x1[ROWS];
+    };
+    auto shift_write = [&](const ShiftWords &v, const int *po, int rank, int b, int lo, int top, int lane) {
 #pragma unroll
-        for (int u = 0; u < ROWS; ++u) {
-            const int r = r0 + u;
-            x0[u] = r < m && lane < n ? V[r * vs + lane] : 0u;
-            x1[u] = 0u;
-        }
-        // applies pivots [applied, upto) to this wave's rows
-        int applied = 0;
-        auto apply_to = [&](int upto) {
-            for (; applied < upto; ++applied) {
-                const int j = applied, s = piv_s[j], c0 = piv_c[j];
-                const uint32_t a = piv_a[j];
-                const int wdt = n + j + 1;
-                const uint32_t y0 = lane < wdt ? V[s * vs + lane] : 0u, ny0 = p - y0;
-                // the rows' updates are independent: straight-line code lets their
-                // multiply chains overlap
-                if (wdt > 64) {
-                    const uint32_t y1 = lane + 64 < wdt ? V[s * vs + lane + 64] : 0u, ny1 = p - y1;
+        for (int r = 0; r < 2; ++r)
 #pragma unroll
-                    for (int u = 0; u < ROWS; ++u) {
-                        const uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)x0[u], c0);
-                        x0[u] = amb1(a, x0[u], b, ny0, p, pinv);
-                        x1[u] = amb1(a, x1[u], b, ny1, p, pinv);
-                    }
-                } else {
-#pragma unroll
-                    for (int u = 0; u < ROWS; ++u) {
-                        const uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)x0[u], c0);
-                        x0[u] = amb1(a, x0[u], b, ny0, p, pinv);
-                    }
-                }
+            for (int c = 0; c < kShiftChunks; ++c) {
+                const int w = top - 64 * (c + 1) + lane;
+                if (b + r * kMbWaves < rank && w >= lo) M[po[b + r * kMbWaves] + w] = v[r][c];
             }
-        };
-        if (r0 < m) {
-            unsigned polls = 0;
-            bool mine = false;
-            for (;;) {
-                // the turn first: once it is this wave's, every pivot of the waves
-                // before it is published and counted below
-                const int turn = __hip_atomic_load(&s_turn, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-                const int pub = __hip_atomic_load(&s_npub, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-                apply_to(pub);
-                if (pub == n) break;  // every pivot found: these rows hold no new one
-                if (turn >= wave) {
-                    mine = true;
-                    break;
-                }
-                // the failure flag (global memory) only matters once a poll limit
-                // ran out somewhere: read it now and then, not on every poll
-                if ((polls & 255) == 255 && __hip_atomic_load(bar + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                    break;
-                if (++polls == kMcSpinLimit) {
-                    __hip_atomic_store(bar + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(1);
+    };
+    auto shift_rows = [&](int kk, int lo, int hi, int step, int lane) {
+        const int rank = __builtin_amdgcn_readfirstlane(op_rank[kk & 1]);
+        for (int b = wave; b < rank; b += 2 * kMbWaves)
+            for (int top = hi; top > lo; top -= kShiftWords) {
+                ShiftWords v;
+                shift_read(v, poff[kk & 1], rank, b, lo, top, step, lane);
+                __builtin_amdgcn_wave_barrier();
+                shift_write(v, poff[kk & 1], rank, b, lo, top, lane);
+                __builtin_amdgcn_wave_barrier();
             }
-            if (mine) {
-                int j = applied;
-                uint32_t aprod = pref[j];  // the scale of the next pivot row
+    };
+    const int own_lo = os + 1, own_hi = oj + ncj * (order + 1);
+    auto own_zero = [&](int kk, int lane) {
+        const int rank = __builtin_amdgcn_readfirstlane(op_rank[kk & 1]);
+        for (int b = wave; b < rank; b += kMbWaves)
+            for (int jj = lane; jj < ncj; jj += 64) M[poff[kk & 1][b] + oj + jj * (order + 1)] = 0;
+    };
+    auto own_shift = [&](int kk, int lane) {
+        shift_rows(kk, own_lo, own_hi, 1, lane);
+        own_zero(kk, lane);
+    };
+
+    for (int k0 = 0; k0 < order; k0 += C.B) {
+        const int bk = order - k0 < C.B ? order - k0 : C.B;  // steps of this block
+        for (int b = 0; b < bk; ++b) {
+            const int k = k0 + b, kb = k & 1;
+            const int *rmap = rowmap[kb];
+            int32_t *Xk = X + (kb & C.xb) * C.xm * xs;
+            {
+                const int lane = fresh_tid() & 63, col = lane & (NC - 1), half = lane / NC;
+                // ---- rows of the discrepancy in shift order ----
+                int32_t x[NREG];
 #pragma unroll
-                for (int u = 0; u < ROWS; ++u) {
-                    const int r = r0 + u;
-                    const uint64_t bal = __ballot(r < m && lane < n && x0[u] != 0);
-                    if (bal) {
-                        const int c0 = (int)__builtin_ctzll(bal), wdt = n + j + 1;
-                        const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)x0[u], c0);
-                        const uint32_t y0 = lane == wdt - 1 ? p - aprod : x0[u];
-                        const uint32_t y1 = lane + 64 == wdt - 1 ? p - aprod : x1[u];
-                        if (lane < wdt) V[r * vs + lane] = y0;
-                        if (lane + 64 < wdt) V[r * vs + lane + 64] = y1;
-                        const uint32_t next = mont(aprod, a, p, pinv);
-                        if (lane == 0) {
-                            piv_s[j] = r;
-                            piv_c[j] = c0;
-                            piv_a[j] = a;
-                            pivot_of[r] = j;
-                            pref[j + 1] = next;
-                            __hip_atomic_store(&s_npub, j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+                for (int q = 0; q < PPW; ++q) {
+                    const int r0 = (wave * PPW + q) * kMbPanel;
+#pragma unroll
+                    for (int g = 0; g < PR; ++g) {
+                        const int r = r0 + g * RPR + half;
+                        x[q * PR + g] = r < m && col < n ? M[rmap[r] * rs + b * n + col] : 0;
+                    }
+                }
+                // ---- row rank profile and combinations (the PLUQ of :470-488) ----
+                const int hb4 = (lane & ~(NC - 1)) << 2;
+                int applied = 0;
+                unsigned state = 0;
+                uint64_t used = 0;  // columns of the panels applied
+                // Wave 0, whose rows are the first to be finished, books the panels as it takes
+                // them in: the places of their pivots, their columns' factors (the product of the
+                // D's before them) and their rows.
+                uint32_t e_run = K.one;
+                int rk_run = 0;
+                auto book = [&](int P, const int4 &cc, bool inc) {
+                    const int bits = __builtin_amdgcn_readfirstlane(pbits[P]);
+                    const uint32_t det = (uint32_t)__builtin_amdgcn_readfirstlane((int)pdet[P]);
+                    if (inc && half == 0) {
+                        // the row of this column's slot (slots: rows 0, 2, 1, 3 with two rows a register)
+                        const int c4 = col << 2;
+                        // an unused slot repeats a used one's column: its row has no bit
+                        constexpr int s1 = RPR == 2 ? 2 : 1, s2 = RPR == 2 ? 1 : 2;
+                        const int u = cc.x == c4 && (bits & 1)           ? 0
+                                      : cc.y == c4 && (bits >> s1 & 1) ? s1
+                                      : cc.z == c4 && (bits >> s2 & 1) ? s2
+                                                                       : 3;
+                        bidx[col] = rk_run + __popc(bits & ((1 << u) - 1));
+                        col_e[col] = K.from(e_run);
+                    }
+                    if (lane < kMbPanel && bits >> lane & 1)
+                        poff[kb][rk_run + __popc(bits & ((1 << lane) - 1))] = rmap[P * kMbPanel + lane] * rs;
+                    rk_run += __popc(bits);
+                    e_run = mont(e_run, det, p, npinv);
+                };
+                // takes every published panel in; returns whether the elimination is over
+                // (no unused column left) once at least `want` panels are in.  A panel's
+                // words are written before the count in s_pub and one wave's LDS accesses
+                // are done in order, so words read after a count that covers them are theirs.
+                auto advance = [&](int want) -> bool {
+                    unsigned polls = 0;
+                    for (;;) {
+                        state = __hip_atomic_load(&s_pub, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+                        // the next panel's words, read along with the count (by the wave whose
+                        // turn is next: the others would only load the LDS)
+                        int4 cc, hv;
+                        int32_t dz;
+                        auto fetch = [&]() {
+                            cc = pcol[applied];
+                            hv = H[applied * NC + col];
+                            dz = Dz[applied * NC + col];
+                        };
+                        const bool early = applied + 1 == want && applied < npan;
+                        if (early) fetch();
+                        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+                        state = (unsigned)__builtin_amdgcn_readfirstlane((int)state);
+                        const int pub = (int)(state & 255u);
+                        if (!early && applied < pub) fetch();
+                        while (applied < pub) {
+                            // a panel without pivots has no column (-1)
+                            if (__builtin_amdgcn_readfirstlane(cc.x) >= 0) {
+                                const int a0 = hb4 + cc.x, a1 = hb4 + cc.y, a2 = hb4 + cc.z, a3 = hb4 + cc.w;
+                                int32_t z[NREG][4];
+#pragma unroll
+                                for (int g = 0; g < NREG; ++g) {
+                                    z[g][0] = __builtin_amdgcn_ds_bpermute(a0, x[g]);
+                                    z[g][1] = __builtin_amdgcn_ds_bpermute(a1, x[g]);
+                                    z[g][2] = __builtin_amdgcn_ds_bpermute(a2, x[g]);
+                                    z[g][3] = __builtin_amdgcn_ds_bpermute(a3, x[g]);
+                                }
+                                used |= __ballot(dz == 0);
+#pragma unroll
+                                for (int g = 0; g < NREG; ++g) {
+                                    // five products of centred values: the high word is below p in size
+                                    int64_t t = (int64_t)dz * x[g], t1 = (int64_t)z[g][1] * hv.y;
+                                    t += (int64_t)z[g][0] * hv.x;
+                                    t1 += (int64_t)z[g][2] * hv.z;
+                                    t += (int64_t)z[g][3] * hv.w;
+                                    x[g] = K.redc(t + t1);
+                                }
+                                if (wave == 0) book(applied, cc, dz == 0);
+                            }
+                            if (wave == 0 && lane == 0) s_book = applied + 1;
+                            if (++applied < pub) fetch();
                         }
-                        const uint32_t ny0 = p - y0, ny1 = p - y1;
-#pragma unroll
-                        for (int v = u + 1; v < ROWS; ++v) {
-                            const uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)x0[v], c0);
-                            x0[v] = amb1(a, x0[v], b, ny0, p, pinv);
-                            if (wdt > 64) x1[v] = amb1(a, x1[v], b, ny1, p, pinv);
+                        if (state >> 16) return true;
+                        if (pub >= want) return false;
+                        // the failure flag (global memory) only matters once a poll limit
+                        // ran out somewhere: read it now and then, not on every poll
+                        if ((polls & 255) == 255 &&
+                            __hip_atomic_load(bar + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                            return true;
+                        if (++polls == kMcSpinLimit) {
+                            __hip_atomic_store(bar + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            return true;
                         }
-                        aprod = next;
-                        ++j;
+                        // the wave whose turn is next polls without a pause
+                        if (pub + 1 < want) __builtin_amdgcn_s_sleep(1);
                     }
+                };
+                int mine = 0, found = 0;  // rows of this wave, pivots among them
+                int prank[PPW], prow[PPW];  // pivots before the panel, its pivot rows
+                bool over = false;
+#pragma unroll
+                for (int q = 0; q < PPW; ++q) {
+                    const int P = wave * PPW + q, r0 = P * kMbPanel;
+                    prank[q] = n;
+                    prow[q] = 0;
+                    if (r0 < m) mine += m - r0 < kMbPanel ? m - r0 : kMbPanel;
+                    if (r0 >= m || over) continue;
+                    over = advance(P);
+                    if (over) continue;
+                    __builtin_amdgcn_s_setprio(3);
+                    // Gauss-Jordan on a canonical copy of the panel; at column c of the pivot in
+                    // row u the pivot vector and row u read dcur, the other rows 0 (the panel's
+                    // inverse takes the place of its pivot columns).  One wave's serial chain:
+                    // what counts is the number of instructions.
+                    const int rank0 = (int)(state >> 8 & 255u);
+                    uint32_t y[PR];
+#pragma unroll
+                    for (int g = 0; g < PR; ++g) y[g] = K.canonical(x[q * PR + g]);
+                    uint32_t dcur = K.one;
+                    uint64_t freec = ~used;  // n <= NC, and words beyond column n are zero
+                    int pc[kMbPanel] = {-1, -1, -1, -1}, c_any = -1;
+                    bool inc = false;  // this lane's column is a pivot column of the panel
+                    unsigned rowbits = 0;
+#pragma unroll
+                    for (int u = 0; u < kMbPanel; ++u) {
+                        const int gu = u / RPR, hu = u % RPR;
+                        uint64_t bal = __ballot(y[gu] != 0);
+                        if constexpr (RPR == 2) bal = (hu ? bal >> 32 : bal & 0xffffffffu) & (uint32_t)freec;
+                        else bal &= freec;
+                        if (bal == 0) continue;
+                        const int c = RPR == 2 ? __builtin_ctz((uint32_t)bal) : (int)__builtin_ctzll(bal);
+                        uint32_t bl[PR], bh[PR];
+#pragma unroll
+                        for (int g = 0; g < PR; ++g) {
+                            bl[g] = (uint32_t)__builtin_amdgcn_readlane((int)y[g], c);
+                            bh[g] = RPR == 2 ? (uint32_t)__builtin_amdgcn_readlane((int)y[g], 32 + c) : bl[g];
+                        }
+                        const uint32_t a = hu ? bh[gu] : bl[gu];
+                        const bool isc = col == c;
+                        uint32_t yr = y[gu];
+                        if constexpr (RPR == 2) {
+                            // the row's half in both halves of the wave
+                            const auto sw = __builtin_amdgcn_permlane32_swap(y[gu], y[gu], false, false);
+                            yr = hu == 0 ? (uint32_t)sw[0] : (uint32_t)sw[1];
+                        }
+                        const uint32_t ny = p - (isc ? dcur : yr);
+#pragma unroll
+                        for (int g = 0; g < PR; ++g) {
+                            uint32_t am = a, bv = bl[g], at = 0;
+                            if constexpr (RPR == 2) bv = half ? bh[g] : bl[g];
+                            if (g == gu) {  // the pivot row is scaled, not updated
+                                const bool isp = half == hu;
+                                am = isp ? dcur : a;
+                                bv = isp ? 0u : bv;
+                                at = isp ? dcur : 0u;
+                            }
+                            const uint32_t xin = isc ? at : y[g];
+                            const uint64_t t = (uint64_t)am * xin + (uint64_t)bv * ny;
+                            const uint32_t qq = (uint32_t)t * npinv;
+                            y[g] = csub((uint32_t)((t + (uint64_t)qq * p) >> 32), p);
+                        }
+                        dcur = mont(dcur, a, p, npinv);
+                        pc[u] = c_any = c << 2;
+                        rowbits |= 1u << u;
+                        inc = inc || isc;
+                        freec &= ~(1ull << c);
+                    }
+                    const unsigned cnt = (unsigned)__popc(rowbits), rk = (unsigned)rank0 + cnt;
+                    // slots of rows without a pivot: H zero, any column
+#pragma unroll
+                    for (int u = 0; u < kMbPanel; ++u) pc[u] = pc[u] < 0 ? c_any : pc[u];
+                    int32_t hv[PR];
+#pragma unroll
+                    for (int g = 0; g < PR; ++g) {
+                        const int32_t v = K.from(y[g]);
+                        hv[g] = rowbits >> (g * RPR + half) & 1 ? (inc ? v : -v) : 0;
+                    }
+                    int32_t *hp = reinterpret_cast<int32_t *>(H + P * NC + col);
+                    if constexpr (RPR == 2) {  // slots: rows 0, 2 of the lower half, 1, 3 of the upper
+                        *reinterpret_cast<int2 *>(hp + 2 * half) = make_int2(hv[0], hv[1]);
+                    } else {
+                        *reinterpret_cast<int4 *>(hp) = make_int4(hv[0], hv[1], hv[2], hv[3]);
+                    }
+                    Dz[P * NC + col] = inc ? 0 : K.from(dcur);  // both halves write the same word
+                    if (lane == 0) {
+                        pcol[P] = RPR == 2 ? make_int4(pc[0], pc[2], pc[1], pc[3])
+                                           : make_int4(pc[0], pc[1], pc[2], pc[3]);
+                        pbits[P] = (int)rowbits;
+                        pdet[P] = dcur;
+                        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+                        __hip_atomic_store(&s_pub, (unsigned)(P + 1) | rk << 8 | (rk == (unsigned)n ? 1u << 16 : 0u),
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    }
+                    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+                    __builtin_amdgcn_s_setprio(0);
+                    found += (int)cnt;
+                    prank[q] = rank0;
+                    prow[q] = (int)rowbits;
                 }
-                applied = j;
-                if (lane == 0) __hip_atomic_store(&s_turn, wave + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+                // the non-pivot rows take the remaining panels, and their combinations
+                // (times the product of all D's) go to X
+                if (wave == 0 || mine > found) advance(npan);
+                if (wave == 0 && lane == 0) s_e = e_run;
+                if (mine > found) {
+                    // wait for the last panel's booking
+                    for (unsigned polls = 0; wave != 0 && polls < kMcSpinLimit; ++polls) {
+                        const int bk_n = __hip_atomic_load(&s_book, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        if (__builtin_amdgcn_readfirstlane(bk_n) >= applied) break;
+                        if ((polls & 255) == 255 &&
+                            __hip_atomic_load(bar + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                            break;
+                    }
+                    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+                    const int bc = col < n ? bidx[col] : -1;
+                    const int32_t ce = col_e[col];
+#pragma unroll
+                    for (int q = 0; q < PPW; ++q)
+#pragma unroll
+                        for (int g = 0; g < PR; ++g) {
+                            const int v = g * RPR + half, r = (wave * PPW + q) * kMbPanel + v;
+                            if (r < m && !(prow[q] >> v & 1)) {
+                                // its place: the rows above it less the pivots among them
+                                const int i = r - prank[q] - __popc(prow[q] & ((1 << v) - 1));
+                                const int32_t z = K.mul(x[q * PR + g], ce);
+                                if (bc >= 0) Xk[i * xs + bc] = z;
+                                if (col == 0) noff[kb][i] = rmap[r] * rs;
+                            }
+                        }
+                }
             }
-        }
-        __syncthreads();
-        const int rank = s_npub;
-        // a non-pivot row's scale is the product of the entries of the pivots above it;
-        // its combination is Z / scale: plain inverse s^-1 = mont(montpow(scale, p-2), 1)
-        if (tid < 2 * 64) {
-            const uint64_t pm0 = __ballot(lane < m && pivot_of[lane] >= 0);
-            const uint64_t pm1 = __ballot(lane + 64 < m && pivot_of[lane + 64] >= 0);
-            const int r = tid;
-            if (r < m && pivot_of[r] < 0) {
-                const int cnt = wave == 0 ? __popcll(pm0 & below) : __popcll(pm0) + __popcll(pm1 & below);
-                uint32_t x = one, bp = pref[cnt];
+            __syncthreads();
+            // ---- the inverse, the next order, and the sums over the pivot rows ----
+            const int rank = __builtin_amdgcn_readfirstlane((int)(s_pub >> 8 & 255u));
+            const int nn = m - rank;
+            const int wc = rank && nn ? (bk - b - 1) * n : 0, w0 = (b + 1) * n;
+            const int wct = (wc + 15) >> 4, wtile = wct * ((nn + 15) >> 4);
+            const float rwct = 1.0f / (float)(wct ? wct : 1);
+            int32_t sum[kMcMaxTasks][4];
+            if (wave == 0) {
+                // s^(p-2), s the product of the D's: both products of a bit in every step, so that
+                // their chains overlap
+                uint32_t v = K.one, sq = s_e;
                 for (uint32_t e = p - 2; e; e >>= 1) {
-                    if (e & 1) x = mont(x, bp, p, pinv);
-                    bp = mont(bp, bp, p, pinv);
+                    const uint32_t f = e & 1 ? sq : K.one;
+                    v = mont_pos(v, f, K);
+                    sq = mont_pos(sq, sq, K);
                 }
-                rinv[r] = mont(x, 1u, p, pinv);
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < ROWS; ++u) {
-            const int r = r0 + u;
-            if (r < m && pivot_of[r] < 0) {
-                const uint32_t inv = rinv[r];
-                if (lane >= n && lane < n + rank) V[r * vs + lane] = mont(x0[u], inv, p, pinv);
-                if (lane + 64 < n + rank) V[r * vs + lane + 64] = mont(x1[u], inv, p, pinv);
-            }
-        }
-        // Qt: pivot rows first, then the others, each in increasing order
-        static_assert(kMbMaxM <= 2 * 64 && kMbThreads >= 2 * 64, "two ballots cover every row");
-        if (tid < 2 * 64) {
-            const uint64_t b0 = __ballot(lane < m && pivot_of[lane] < 0);
-            const uint64_t b1 = __ballot(lane + 64 < m && pivot_of[lane + 64] < 0);
-            const int r = tid;
-            if (r < m) {
-                int pos = pivot_of[r];
-                if (pos < 0) pos = rank + (wave == 0 ? __popcll(b0 & below) : __popcll(b0) + __popcll(b1 & below));
-                oldrow[pos] = r;
-                tmpmap[pos] = rowmap[r];
-                tmp64[pos] = shift[r];
-                tmp64b[pos] = degree[r];
-                was_piv[rowmap[r]] = pivot_of[r] >= 0;
-            }
-        }
-        __syncthreads();
-        for (int i = tid; i < m; i += kMbThreads) {
-            rowmap[i] = tmpmap[i];
-            shift[i] = tmp64[i];
-            degree[i] = tmp64b[i];
-        }
-        __syncthreads();
-        // ---- 4. this group's columns: non-pivot rows -= combination . pivot rows (:509-517) ----
-        {
-            const int nrows = m - rank, per_l = nrows * cw, total = (lim + 1) * per_l;
-            for (int o = tid; o < total; o += kMbThreads) {
-                const int l = o / per_l, rem = o - l * per_l, q = rem / cw, jj = rem - q * cw, si = rank + q;
-                const uint32_t *y = V + oldrow[si] * vs + n;
-                const uint32_t *w = W + l * cst + jj;
-                AccSmall acc0, acc1;
-                int t = 0;
-                for (; t + 3 < rank; t += 4) {
-                    const uint32_t w0 = w[rowmap[t] * cw], w1 = w[rowmap[t + 1] * cw], w2 = w[rowmap[t + 2] * cw],
-                                   w3 = w[rowmap[t + 3] * cw];
-                    acc0.add2(y[t], w0, y[t + 1], w1, f62);
-                    acc1.add2(y[t + 2], w2, y[t + 3], w3, f62);
+                if (fresh_tid() == 0) {
+                    s_inv[kb] = K.from(v);
+                    op_rank[kb] = rank;
                 }
-                for (; t < rank; ++t) acc0.add1(y[t], w[rowmap[t] * cw], f62);
-                const uint32_t sub = sum2(acc0, acc1, p, mu);
-                uint32_t *dst = W + l * cst + rowmap[si] * cw + jj;
-                const uint32_t v = *dst;
-                *dst = v >= sub ? v - sub : v + (p - sub);
-            }
-        }
-        __syncthreads();
-        // ---- pivot rows times x (:573-580); degrees and shifts (:546-566) ----
-        for (int o = tid; o < rank * cw; o += kMbThreads) {
-            const int t = o / cw, jj = o - t * cw;
-            uint32_t *col = W + rowmap[t] * cw + jj;
-            // eight coefficients at a time from the top: a block's writes reach only
-            // coefficients already read
-            for (int top = lim; top >= 0; top -= 8) {
-                uint32_t v[8];
+            } else if (wave == 1) {
+                // Qt: pivot rows first, then the others, each in increasing order; degrees
+                // and shifts (:546-566); then the next step's order
+                const int lane = fresh_tid() & 63;
+                const uint64_t below = (1ull << lane) - 1;
+                const uint64_t pm0 = __ballot(lane < m && pbits[lane >> 2] >> (lane & 3) & 1);
+                const uint64_t pm1 = __ballot(lane + 64 < m && pbits[(lane >> 2) + 16] >> (lane & 3) & 1);
+                const int maxdeg = s_maxdeg, np0 = __popcll(pm0);
+                uint64_t dm = 0;
+                for (int h = 0; h < m; h += 64) {
+                    const int r = h + lane;
+                    if (r < m && (h ? pm1 : pm0) >> lane & 1) dm = degree[r] > dm ? degree[r] : dm;
+                }
+                dm = __ockl_wfred_max_u64(dm);
+                int *next = rowmap[kb ^ 1];
+                for (int h = 0; h < m; h += 64) {
+                    const int r = h + lane;
+                    if (r < m) {
+                        const uint64_t word = h ? pm1 : pm0;
+                        const bool isp = word >> lane & 1;
+                        const int bel = __popcll(word & below) + (h ? np0 : 0);
+                        const int pos = isp ? bel : rank + r - bel;
+                        const uint64_t d = degree[r];
+                        tmp64[pos] = shift[r] + (isp ? 1 : 0);
+                        tmp64b[pos] = isp ? d + 1 : (d < dm ? dm : d);
+                        next[pos] = rmap[r];
+                    }
+                }
+                __builtin_amdgcn_s_waitcnt(0);
+                __builtin_amdgcn_wave_barrier();
+                for (int r = lane; r < m; r += 64) {
+                    shift[r] = tmp64[r];
+                    degree[r] = tmp64b[r];
+                }
+                const uint64_t md64 = (uint64_t)maxdeg > dm + 1 ? (uint64_t)maxdeg : dm + 1;
+                const int md = (int)(md64 < (uint64_t)order ? md64 : (uint64_t)order);
+                if (lane == 0) s_maxdeg = md;
+                __builtin_amdgcn_s_waitcnt(0);
+                __builtin_amdgcn_wave_barrier();
+                if (k + 1 < order) sort_rows(next, lane);
+            } else {
+                const int lane = fresh_tid() & 63;
 #pragma unroll
-                for (int u = 0; u < 8; ++u)
-                    if (top - u >= 0) v[u] = col[(top - u) * cst];
-#pragma unroll
-                for (int u = 0; u < 8; ++u)
-                    if (top - u >= 0) col[(top - u + 1) * cst] = v[u];
+                for (int q = 0; q < kMcMaxTasks; ++q) {
+                    const int i = wave - 2 + q * kMcSumWaves;
+                    if (i < wtile) {
+                        const int rq = quot(i, rwct), w = 16 * (i - rq * wct) + (lane & 15);
+                        tile_sums(sum[q], Xk + 16 * rq * xs, xs, M + w0 + (w < wc ? w : 0), poff[kb], rank, lane, K);
+                    }
+                }
+                // the own columns' tiles begin at the waves the window leaves idle
+                if (b > 0) own_update(k - 1, true, kMbWaves - 1 - wave, kMcSumWaves, lane);
             }
-            col[0] = 0;
-        }
-        if (wave == kMbWaves - 1) {
-            uint64_t dm = 0;
-            for (int i = lane; i < rank; i += 64) dm = degree[i] > dm ? degree[i] : dm;
-            dm = __ockl_wfred_max_u64(dm);
-            for (int i = lane; i < m; i += 64) {
-                if (i < rank) {
-                    degree[i]++;
-                    shift[i]++;
-                } else if (degree[i] < dm) {
-                    degree[i] = dm;
+            __syncthreads();
+            // ---- scaled sums from the window; pivot rows times x ----
+            {
+                const int tid = fresh_tid(), lane = tid & 63;
+                const int whi = bk * n;
+                if (b > 0 && rank <= 2 * kMbWaves && whi - w0 <= kShiftWords && own_hi - own_lo <= kShiftWords) {
+                    // both shifts in one round of reads and one of writes
+                    const int rank1 = __builtin_amdgcn_readfirstlane(op_rank[kb ^ 1]);
+                    ShiftWords vw, vo;
+                    if (rank1 <= 2 * kMbWaves) {
+                        shift_read(vw, poff[kb], rank, wave, w0, whi, n, lane);
+                        shift_read(vo, poff[kb ^ 1], rank1, wave, own_lo, own_hi, 1, lane);
+                        __builtin_amdgcn_wave_barrier();
+                        shift_write(vw, poff[kb], rank, wave, w0, whi, lane);
+                        shift_write(vo, poff[kb ^ 1], rank1, wave, own_lo, own_hi, lane);
+                        __builtin_amdgcn_wave_barrier();
+                        own_zero(k - 1, lane);
+                    } else {
+                        shift_rows(k, w0, whi, n, lane);
+                        own_shift(k - 1, lane);
+                    }
+                } else {
+                    shift_rows(k, w0, whi, n, lane);
+                    if (b > 0) own_shift(k - 1, lane);
+                }
+                if (wave >= 2) {
+#pragma unroll
+                    for (int q = 0; q < kMcMaxTasks; ++q) {
+                        const int i = wave - 2 + q * kMcSumWaves;
+                        if (i < wtile) {
+                            const int rq = quot(i, rwct), w = 16 * (i - rq * wct) + (lane & 15);
+                            apply_tile(sum[q], kb, 16 * rq, nn, w < wc ? w0 + w : -1, lane);
+                        }
+                    }
+                }
+                if (tid < kMbMaxN) bidx[tid] = -1;
+                if (tid < kMbMaxM / kMbPanel) pbits[tid] = 0;
+                if (tid == 0) {
+                    s_pub = 0;
+                    s_book = 0;
+                    if (b + 1 < bk) op_lim[kb ^ 1] = k + 1 < s_maxdeg ? k + 1 : s_maxdeg;
                 }
             }
-            if (lane == 0) {
-                const uint64_t md = (uint64_t)maxdeg > dm + 1 ? (uint64_t)maxdeg : dm + 1;
-                s_maxdeg = (int)(md < (uint64_t)order ? md : (uint64_t)order);
+            __syncthreads();
+        }
+        // ---- the block's last operation on the own columns ----
+        const int kl = k0 + bk - 1;
+        const bool more = kl + 1 < order;
+        own_update(kl, more, wave, kMbWaves, fresh_tid() & 63);
+        __syncthreads();
+        own_shift(kl, fresh_tid() & 63);
+        __syncthreads();
+        if (!more) break;
+        // ---- the next block's window ----
+        const int tid = fresh_tid();
+        const int nb = order - kl - 1 < C.B ? order - kl - 1 : C.B;  // its steps
+        const int cn = ncs * nb;
+        const float rcn = 1.0f / (float)(cn ? cn : 1), rcs = 1.0f / (float)(ncs ? ncs : 1);
+        if (G > 1) {
+            int32_t *px = part + (size_t)(nbar & 1) * m * os;
+            for (int i = tid; i < m * cn; i += kMbThreads) {
+                const int ph = quot(i, rcn), rem = i - ph * cn, t = quot(rem, rcs), cc = rem - t * ncs;
+                __hip_atomic_store(px + ph * os + t * n + c0 + cc, M[ph * rs + os + cc * order + kl + 1 + t],
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            grid_barrier(bar, bar_base + ++nbar * (unsigned)G);
+            const int wn = nb * n;
+            const float rwn = 1.0f / (float)wn;
+            for (int i0 = tid; i0 < m * wn; i0 += 8 * kMbThreads) {
+                int32_t v[8];  // eight loads in flight
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int i = i0 + u * kMbThreads, ph = quot(i, rwn), w = i - ph * wn;
+                    v[u] = i < m * wn ? __hip_atomic_load(px + ph * os + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                      : 0;
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int i = i0 + u * kMbThreads, ph = quot(i, rwn), w = i - ph * wn;
+                    if (i < m * wn) M[ph * rs + w] = v[u];
+                }
+            }
+        } else {
+            for (int i = tid; i < m * cn; i += kMbThreads) {
+                const int ph = quot(i, rcn), rem = i - ph * cn, t = quot(rem, rcs), cc = rem - t * ncs;
+                M[ph * rs + t * n + cc] = M[ph * rs + os + cc * order + kl + 1 + t];
             }
         }
+        if (tid == 0) op_lim[(kl + 1) & 1] = kl + 1 < s_maxdeg ? kl + 1 : s_maxdeg;
         __syncthreads();
     }
     // sigma.resize(max_degree+1), shift2 = shift (:592-597)
     const int md = s_maxdeg;
     const int cnt = out_count ? out_count : md + 1;
-    for (int o = tid; o < cnt * m * cols; o += kMbThreads) {
-        const int q = o / cols, l = q / m, jj = o - q * cols, i = q - l * m;
-        const uint32_t v = l <= md ? W[l * cst + rowmap[i] * cw + jj] : 0u;
+    const int *rmap = rowmap[order & 1];
+    for (int o = tid0; o < m * ncj * cnt; o += kMbThreads) {
+        const int q = o / cnt, l = o - q * cnt, i = q / ncj, jj = q - i * ncj;
+        const uint32_t v = l <= md ? K.canonical(M[rmap[i] * rs + oj + jj * (order + 1) + l]) : 0u;
         out.base[view_index(out, (size_t)i * m + j0 + jj, l)] = v;
     }
-    if (g == 0) {
-        for (int i = tid; i < m; i += kMbThreads) shift_io[i] = shift[i];
-        if (tid == 0) *deg_out = (uint64_t)md;
+    if (blockIdx.x == 0) {
+        for (int i = tid0; i < m; i += kMbThreads) shift_io[i] = shift[i];
+        if (tid0 == 0) *deg_out = (uint64_t)md;
     }
 }
 
@@ -1102,9 +1479,11 @@ size_t pm_level_bytes(size_t m, size_t n, size_t order)
 }
 
 struct MbScratch {
-    uint32_t *S, *W, *part;
+    uint32_t *S, *W;
+    int32_t *part;
     uint64_t *shift, *deg;
     unsigned *bar;  // grid barrier: arrivals, then the failure flag
+    unsigned arrivals;  // of the launches queued so far
 };
 
 struct PmRun {
@@ -1138,16 +1517,12 @@ DevView polfirst_view(uint32_t *base, size_t rows, size_t cols, size_t stor, siz
     return v;
 }
 
-size_t mc_lds_words(size_t m, size_t n, size_t order, size_t cw)
+size_t mc_lds_words(const ColsShape &C)
 {
-    return cw * ((order + 1) * m + order * n) + m * n + m * (n + 1) + m * n;
+    const size_t nc = C.n <= 32 ? 32 : 64, npan = ((size_t)C.m + kMbPanel - 1) / kMbPanel;
+    return npan * nc * 5 + (size_t)(1 + C.xb) * C.xm * C.xs + (size_t)C.m * C.rs;
 }
 
-// Column split of m_basis_cols_kernel: *G groups of *cw columns, or *G = 0 for
-// the one-workgroup kernel (orders above kMcMaxOrder, or LDS too small for one
-// column).  By default about m^2 n / 8192 groups (at most 16): the work each
-// group repeats (sort and elimination) against the work it shares out.
-// LBX_MBASIS_GROUPS=N asks for N groups, 0 for the one-workgroup kernel.
 // The grid of m_basis_cols_kernel must fit on the device at once: one group
 // per CU (its LDS takes most of a CU's 160 KiB).
 lbx_status mc_check_groups(int G)
@@ -1158,24 +1533,39 @@ lbx_status mc_check_groups(int G)
     return G <= cus ? LBX_OK : LBX_ERR_UNSUPPORTED;
 }
 
-void cols_split(size_t m, size_t n, size_t order, int *G, int *cw)
+// Column split of m_basis_cols_kernel over the returned number of groups, or 0
+// for the one-workgroup kernel (orders above kMcMaxOrder, or no split fits).
+// By default about m^2 n / 4096 groups (at most 32), so that a group's own
+// columns cost no more per step than its window; more where the LDS of fewer
+// groups would not hold their columns.  Blocks of kMcMaxBlock steps where they
+// fit, shorter ones otherwise.  LBX_MBASIS_GROUPS=N asks for N groups, 0 for the
+// one-workgroup kernel.
+int cols_split(size_t m, size_t n, size_t order, ColsShape *C)
 {
-    *G = 0;
-    *cw = 0;
-    if (order > (size_t)kMcMaxOrder) return;
-    size_t target = std::min<size_t>(16, std::max<size_t>(1, m * m * n / 8192));
+    if (order > (size_t)kMcMaxOrder) return 0;
+    size_t target = std::min<size_t>(32, std::max<size_t>(1, m * m * n / 4096));
     if (const char *e = getenv("LBX_MBASIS_GROUPS")) {
         const long want = atol(e);
-        if (want <= 0) return;
-        target = (size_t)want;
+        if (want <= 0) return 0;
+        target = std::min<size_t>((size_t)want, (size_t)kMcMaxGroups);
     }
-    size_t w = (m + target - 1) / target;
-    while (w > 0 && mc_lds_words(m, n, order, w) > (size_t)kMcLdsWords) --w;
-    if (!w) return;
-    const size_t groups = (m + w - 1) / w;
-    if (groups > (size_t)kMcMaxGroups) return;
-    *G = (int)groups;
-    *cw = (int)w;
+    for (int B = std::min<int>(kMcMaxBlock, (int)order); B > 0; B >>= 1)
+        for (size_t g = target; g <= (size_t)kMcMaxGroups; ++g) {
+            C->order = (int)order;
+            C->m = (int)m;
+            C->n = (int)n;
+            C->cs = (int)((n + g - 1) / g);
+            C->cj = (int)((m + g - 1) / g);
+            C->B = B;
+            C->rs = (int)((size_t)B * n + C->cs * order + C->cj * (order + 1)) | 1;  // odd: rows start in distinct banks
+            C->xs = (int)((std::min(m, n) + 15) & ~(size_t)15) + 4;
+            C->xm = (int)((m + 15) & ~(size_t)15);
+            C->xb = B > 1;
+            const size_t tiles = ((size_t)(B - 1) * n + 15) / 16 * ((m + 15) / 16);
+            if (mc_lds_words(*C) <= (size_t)kMcLdsWords && tiles <= (size_t)(kMcSumWaves * kMcMaxTasks))
+                return (int)std::max((n + C->cs - 1) / C->cs, (m + C->cj - 1) / C->cj);
+        }
+    return 0;
 }
 
 // T = a_top . b_top (m x m coefficient matrices: coefficient ta of a, tb of b);
@@ -1221,40 +1611,37 @@ lbx_status run_m_basis(PmRun &R, const DevView &serie, const DevView &sigma, siz
                        size_t out_count)
 {
     const size_t m = R.m, n = R.n;
-    const size_t g = serie.rows * serie.cols * order;
-    hipLaunchKernelGGL(gather_coeff_major, dim3(grid_for(g)), dim3(256), 0, R.s, serie, order, R.mb.S, R.mb.bar);
-    LBX_TRY_HIP(hipGetLastError());
     uint64_t mu = ~(uint64_t)0 / R.p;
     const uint32_t r32 = (uint32_t)(((uint64_t)1 << 32) % R.p), r64 = (uint32_t)((uint64_t)r32 * r32 % R.p);
     uint32_t f62 = (uint32_t)(((uint64_t)1 << 62) % R.p);
     const bool mont_ok = R.p < (1u << 31) && (R.p & 1);
     uint32_t pinv = 0, r2m = 0, one = 1;
     if (mont_ok) {
-        uint32_t inv = R.p;  // Newton iteration for p^-1 mod 2^32
-        for (int i = 0; i < 5; ++i) inv *= 2u - R.p * inv;
-        pinv = 0u - inv;
+        pinv = 0u - inv_mod32(R.p);
         one = r32;
-        r2m = (uint32_t)((uint64_t)r32 * r32 % R.p);
+        r2m = r64;
     }
-    int G = 0, cw = 0;
-    if (mont_ok) cols_split(m, n, order, &G, &cw);
+    ColsShape C;
+    const int G = mont_ok ? cols_split(m, n, order, &C) : 0;
     if (G > 0) {
-        const size_t lds = mc_lds_words(m, n, order, (size_t)cw) * 4;
-        // rows of the elimination per wave: m / 16, rounded up to 2, 4 or 8
-        const void *kern = m <= 2 * (size_t)kMbWaves   ? (const void *)m_basis_cols_kernel<2>
-                           : m <= 4 * (size_t)kMbWaves ? (const void *)m_basis_cols_kernel<4>
-                                                       : (const void *)m_basis_cols_kernel<8>;
+        const size_t lds = mc_lds_words(C) * 4;
+        const void *kern = n <= 32 ? (m <= 64 ? (const void *)m_basis_cols_kernel<32, 1>
+                                              : (const void *)m_basis_cols_kernel<32, 2>)
+                                   : (m <= 64 ? (const void *)m_basis_cols_kernel<64, 1>
+                                              : (const void *)m_basis_cols_kernel<64, 2>);
         LBX_TRY_HIP(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        const uint32_t *S = R.mb.S;
-        DevView out = sigma;
+        Centred K{R.p, inv_mod32(R.p), (R.p - 1) / 2, one, {}};
+        for (int d = 0; d < 7; ++d) {
+            const uint32_t c = (uint32_t)(((uint64_t)1 << (8 * d)) % R.p);
+            K.c8[d] = (int32_t)(c > K.h ? c - R.p : c);
+        }
+        DevView in = serie, out = sigma;
         uint64_t *shift_io = R.mb.shift;
-        uint32_t *part = R.mb.part;
-        unsigned *bar = R.mb.bar;
-        int order_i = (int)order, m_i = (int)m, n_i = (int)n, oc = (int)out_count;
-        uint32_t p = R.p;
-        void *args[] = {&S,   &out, &shift_io, &deg, &part, &bar,  &order_i, &m_i, &n_i, &cw,
-                        &oc,  &p,   &mu,       &f62, &pinv, &r2m, &one};
-        // Every group waits for the others at each step, so all G must become
+        int32_t *part = R.mb.part;
+        unsigned *bar = R.mb.bar, bar_base = R.mb.arrivals;
+        int oc = (int)out_count;
+        void *args[] = {&in, &out, &shift_io, &deg, &part, &bar, &bar_base, &C, &oc, &K};
+        // Every group waits for the others at each exchange, so all G must become
         // resident.  G <= 64 groups of one CU each fit on the device together,
         // and groups still queued behind other streams' work are dispatched as
         // that work drains (the barrier's poll limit bounds the wait), so an
@@ -1263,8 +1650,13 @@ lbx_status run_m_basis(PmRun &R, const DevView &serie, const DevView &sigma, siz
         // before and after every base case.
         LBX_TRY(mc_check_groups(G));
         LBX_TRY_HIP(hipLaunchKernel(kern, dim3(G), dim3(kMbThreads), args, lds, R.s));
+        const unsigned blocks = (unsigned)((order + C.B - 1) / C.B);
+        if (G > 1) R.mb.arrivals += (unsigned)G * std::max(blocks - 1, 1u);
         return LBX_OK;
     }
+    const size_t g = serie.rows * serie.cols * order;
+    hipLaunchKernelGGL(gather_coeff_major, dim3(grid_for(g)), dim3(256), 0, R.s, serie, order, R.mb.S);
+    LBX_TRY_HIP(hipGetLastError());
     // staged words: enough for every coefficient of a step, at most kMbStageWords
     const size_t need = std::max((order + 1) * (m * m + m * n), m * m);
     const int stage = (int)std::min(need, (size_t)kMbStageWords);
@@ -1387,7 +1779,7 @@ lbx_status order_basis(lbx_ctx *ctx, uint32_t p, lbx_polmat *sigma, const lbx_po
     StreamOrder stream_order(ctx, s);
     const size_t base_order = divide ? std::min(order, kMbThreshold) : order;
     const size_t b_S = align256(m * n * base_order * 4), b_W = align256((base_order + 1) * m * m * 4);
-    const size_t b_part = align256(2 * (size_t)kMcMaxGroups * m * n * 4);
+    const size_t b_part = align256(2 * (size_t)kMcMaxBlock * m * n * 4);
     const size_t b_sh = align256(m * 8), b_small = 256;
     const size_t arena = divide ? pm_level_bytes(m, n, order) : 0;
     void *scratch = nullptr;
@@ -1396,7 +1788,7 @@ lbx_status order_basis(lbx_ctx *ctx, uint32_t p, lbx_polmat *sigma, const lbx_po
     PmRun R{ctx, p, m, n, method, s, {}, base + b_S + b_W + b_part + b_sh + 2 * b_small, 0, arena};
     R.mb.S = (uint32_t *)base;
     R.mb.W = (uint32_t *)(base + b_S);
-    R.mb.part = (uint32_t *)(base + b_S + b_W);
+    R.mb.part = (int32_t *)(base + b_S + b_W);
     R.mb.shift = (uint64_t *)(base + b_S + b_W + b_part);
     R.mb.deg = (uint64_t *)(base + b_S + b_W + b_part + b_sh);
     R.mb.bar = (unsigned *)(base + b_S + b_W + b_part + b_sh + b_small);

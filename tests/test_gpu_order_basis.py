@@ -235,3 +235,29 @@ def test_errors(ctx):
     with pytest.raises(LinboxError) as e:  # m*n above 4096
         ob.M_Basis(PolynomialMatrix(128, 128, 3), large, 2, [0] * 128)
     assert e.value.status == 11
+
+
+@pytest.mark.parametrize("m,n,order,p", [
+    (64, 32, 32, FFT_P),        # full panels, four blocks of steps and more
+    (61, 31, 31, 2013265921),   # ragged panel, columns and last block; 31-bit prime
+    (64, 33, 9, 2147483647),    # one row per register, largest odd prime of the split kernel
+    (65, 32, 8, FFT_P),         # two panels per wave, two blocks
+    (128, 32, 6, FFT_P),        # the widest split
+    (117, 35, 5, FFT_P),        # one step per block
+    (64, 64, 5, 97),            # as many columns as rows
+    (40, 1, 32, FFT_P), (3, 2, 4, 3), (5, 2, 1, FFT_P)])
+def test_base_case_blocks(ctx, m, n, order, p):
+    """M_Basis over several workgroups at the edges of its panels (4 rows), lane groups
+    (32 or 64 columns), waves, row tiles (16) and blocks of steps (4): random series, and
+    series whose discrepancies lose rows and columns inside a panel."""
+    rng = np.random.default_rng(7 * m + n + order)
+    shift = [int(x) for x in rng.integers(0, 3, m)]
+    serie = rand(rng, p, m * n * order)
+    compare(ctx, "m", p, m, n, serie, order, shift)
+    F = serie.reshape(m, n, order).astype(np.uint64)
+    F[1 % m] = 0                                   # a zero row in the first panel
+    F[m - 1] = (F[0] * 2 + F[m // 2]) % p          # a dependent row in the last
+    if n > 2:
+        F[:, 1] = (F[:, 0] + F[:, n - 1] * 5) % p  # a dependent column
+    F[m // 3:2 * m // 3, :, 0] = 0                 # rows that enter one step later
+    compare(ctx, "m", p, m, n, F.astype(np.uint32).reshape(-1), order, [0] * m)
