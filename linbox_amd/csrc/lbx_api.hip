@@ -343,6 +343,23 @@ struct Pipe {
     lbx_status end(size_t n) { return on ? pipeline_end(ctx, s, n) : LBX_OK; }
 };
 
+// Whether a matfirst or matrowfirst operand is moved into polfirst scratch
+// before its transforms (and such a result written through it).  The transform
+// kernels take an entry's coefficients one stride apart, a 64-byte sector for
+// every word, unless a group holds 16 or more neighbouring entries (2^13 words
+// a group: up to 2^9 points); the tiled copy reads and writes whole lines, at
+// the price of one more pass and one more launch.  Measured (copied against
+// direct, us): 64^3 at 2^11 points, 2^22 words an operand: 151 / 226 matfirst,
+// 163 / 205 matrowfirst; 96x48x80 at 2^12: the inverse's tail alone 231 direct;
+// 32^3 at 2^11, 2^20 words: 83 / 83 and 100 / 79; 128^3 at 2^9, 2^22 words:
+// 154 / 162 and 167 / 157; smaller operands lose the launches (16^3 at 2^11:
+// 56 / 49 and 70 / 47).
+bool copies_to_polfirst(const DevView &v, size_t entries, size_t count, unsigned L)
+{
+    return v.layout != LBX_POLFIRST && entries < ((size_t)1 << 32) && L >= 10 &&
+           count >= ((size_t)1 << 21) / entries + 1;
+}
+
 // Forward transforms, pointwise products and inverse transform of one
 // single-prime product on device views.  deg+1 coefficients of c are written.
 // Every device buffer is taken from the workspace before the first launch.
@@ -420,8 +437,33 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
     }
 
     // ---- launches ----
+    // operands stored by coefficient become polfirst in the buffer that their
+    // transform's output takes afterwards: in place for whole transforms, and
+    // in the point blocks for split ones (when one chunk's head has read it all
+    // before the tail writes them); rows are 16-byte multiples for the copy
+    const auto load_polfirst = [&](DevView &v, size_t entries, bool one_chunk, void *blocks, void *hat) -> lbx_status {
+        const size_t stor = split ? (v.size + 3) & ~(size_t)3 : N;
+        if (!copies_to_polfirst(v, entries, v.size, L) || v.size > N || stor > N || !one_chunk) return LBX_OK;
+        const DevView pf{(uint32_t *)(split ? blocks : hat), LBX_POLFIRST, v.rows, v.cols, stor, 0, v.size};
+        LBX_TRY_HIP(launch_copy(v, pf, entries, v.size, 0, 0, s));
+        v = pf;
+        return LBX_OK;
+    };
+    LBX_TRY(load_polfirst(a, m * k, rpc >= mpad || !split, al, ahat));
+    LBX_TRY(load_polfirst(b, k * n, rpc >= npad || !split, bl, bhat));
+    // the result likewise leaves through the product's own buffer, free once
+    // the inverse transform has read it
+    DevView out = c;
+    if (copies_to_polfirst(c, m * n, count, L) && count <= N && (!split || cchunk >= m * n)) {
+        const size_t stor = split ? std::min((count + 3) & ~(size_t)3, N) : N;
+        out = DevView{(uint32_t *)(split ? cmat : chat), LBX_POLFIRST, m, n, stor, 0, count};
+    }
+    const auto store_result = [&]() -> lbx_status {
+        if (out.base != c.base) LBX_TRY_HIP(launch_copy(out, c, m * n, count, 0, 0, s));
+        return LBX_OK;
+    };
     if (mid) {
-        const DevView &sm = mid->small_left ? a_in : b_in;
+        const DevView sm = mid->small_left ? a : b;
         const size_t se = mid->small_left ? m * k : k * n;
         LBX_TRY_HIP(launch_reverse_gather(sm, se, mid->hdeg, (uint32_t *)rev, s));
         const DevView rv{(uint32_t *)rev, LBX_POLFIRST, sm.rows, sm.cols, mid->hdeg, 0, mid->hdeg};
@@ -489,11 +531,12 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
             LBX_TRY(ip.handoff(chunk));
             {
                 KernelTimer kt(ctx, ip.consumer(), "kernel dit_tail", timing);
-                LBX_TRY_HIP(launch_ntt_inverse_tail(buf, ne, L, BL, twc, p, c, e0, count, 1, ip.consumer()));
+                LBX_TRY_HIP(launch_ntt_inverse_tail(buf, ne, L, BL, twc, p, out, e0, count, 1, ip.consumer()));
             }
             LBX_TRY(ip.done(chunk));
         }
         LBX_TRY(ip.end(chunk));
+        LBX_TRY(store_result());
         st.mark("inverse FFT_DIT");
         return LBX_OK;
     }
@@ -525,8 +568,9 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
     }
     {
         KernelTimer kt(ctx, s, "kernel dit", timing);
-        LBX_TRY_HIP(launch_ntt_inverse((uint32_t *)chat, m * n, L, twc, p, c, count, 1, s));
+        LBX_TRY_HIP(launch_ntt_inverse((uint32_t *)chat, m * n, L, twc, p, out, count, 1, s));
     }
+    LBX_TRY(store_result());
     st.mark("inverse FFT_DIT");
     return LBX_OK;
 }

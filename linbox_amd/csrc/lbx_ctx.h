@@ -273,6 +273,9 @@ void batch_release(lbx_ctx *ctx);
 lbx_status batch_products(lbx_ctx *ctx, const lbx_job *jobs, size_t njobs, hipStream_t s);
 // Whether the plain form takes point-major operands (split transforms) for m x k x n.
 bool plain_point_major(size_t m, size_t k, size_t n);
+// Whether a view of `entries` x `count` coefficients that is not polfirst goes
+// through a polfirst copy in a product with 2^L points.
+bool copies_to_polfirst(const DevView &v, size_t entries, size_t count, unsigned L);
 // The pointwise form LBX_METHOD_AUTO resolves to for m x k x n at 2^L points.
 int choose_method(int method, size_t m, size_t k, size_t n, unsigned L);
 

@@ -222,6 +222,10 @@ enum TwFormat : int { kTwShoup = 0, kTwMont = 1 };
 // The pow_w twiddle table of root w of order 2^L (N-1 entries) computed on
 // the device, identical to the host-built one of the same format.
 hipError_t launch_build_twiddles(uint2 *tw, uint32_t p, unsigned L, uint32_t w, TwFormat fmt, hipStream_t s);
+// dst(e, start + i) = src(e, beg + i) for i < cnt, between any two layouts
+// (copy.hip; entries < 2^32).
+hipError_t launch_copy(const DevView &src, const DevView &dst, size_t entries, size_t cnt, size_t beg, size_t start,
+                       hipStream_t s);
 // view(e, t) = value for t0 <= t < t0+count (a graph-safe fill, no memset node).
 hipError_t launch_fill(const DevView &out, size_t entries, size_t t0, size_t count, uint32_t value, hipStream_t s);
 // view(e, t) = in[e*stride + t] for t < count.

@@ -409,9 +409,10 @@ struct FpLayout {
 // mod p_i for j < i), then c = sum_i v_i beta_i mod p with beta_i = prod_{j<i}
 // p_j mod p, written to the output view.  Every value is a 32-bit word: v_i <
 // p_i < 2^31 and Shoup products take any 32-bit multiplicand.  WIDE (p >= 2^31):
-// the Shoup remainder x*w - q*p < 2p and the sum are held in 64 bits.
+// the Shoup remainder x*w - q*p < 2p and the sum are held in 64 bits.  `out`
+// may be res[0]'s own storage.
 template <int RM, bool WIDE>
-__global__ void __launch_bounds__(256) few_primes_crt_kernel(const uint32_t *__restrict__ res, size_t entries,
+__global__ void __launch_bounds__(256) few_primes_crt_kernel(const uint32_t *res, size_t entries,
                                                              size_t size, const uint32_t *__restrict__ K, int r,
                                                              uint32_t p, DevView out)
 {
@@ -673,8 +674,23 @@ lbx_status mp_product(lbx_ctx *ctx, const uint32_t *Pw, int nl, const DevView &a
                 LBX_TRY_HIP(hipGetLastError());
             }
             LBX_TRY(ensure(ctx, "mp_rc", (size_t)r * m * n * sc * 4, &rc));
+            // every prime's product reads the operands: those stored by
+            // coefficient become polfirst once, for all of them (a copy that
+            // there is no memory for is left to the products)
+            const auto as_polfirst = [&](const DevView &v, size_t entries, const char *slot) -> DevView {
+                const size_t stor = (v.size + 3) & ~(size_t)3;
+                void *buf;
+                if (fp->reduce || !copies_to_polfirst(v, entries, v.size, lpts)) return v;
+                if (ensure(ctx, slot, entries * stor * 4, &buf) != LBX_OK) {
+                    (void)hipGetLastError();
+                    return v;
+                }
+                const DevView pf{(uint32_t *)buf, LBX_POLFIRST, v.rows, v.cols, stor, 0, v.size};
+                return launch_copy(v, pf, entries, v.size, 0, 0, s) == hipSuccess ? pf : v;
+            };
+            const DevView a1 = as_polfirst(a, m * k, "mp_ra"), b1 = as_polfirst(b, k * n, "mp_rb");
             for (int i = 0; i < r; ++i) {
-                DevView va = a, vb = b;
+                DevView va = a1, vb = b1;
                 if (fp->reduce) {
                     va = DevView{(uint32_t *)ra + (size_t)i * m * k * sa, LBX_POLFIRST, m, k, sa, 0, sa};
                     vb = DevView{(uint32_t *)rb + (size_t)i * k * n * sb, LBX_POLFIRST, k, n, sb, 0, sb};
@@ -687,14 +703,19 @@ lbx_status mp_product(lbx_ctx *ctx, const uint32_t *Pw, int nl, const DevView &a
                 else
                     LBX_TRY(fft_prime_product(ctx, fp->primes[i], lpts, va, vb, vc, m, k, n, sc, method, s));
             }
+            // a result stored by coefficient is recombined polfirst, in the place
+            // of the first prime's residues, and copied out in one pass
+            DevView cv = c;
+            if (copies_to_polfirst(c, m * n, sc, lpts)) cv = DevView{(uint32_t *)rc, LBX_POLFIRST, m, n, sc, 0, sc};
             const dim3 grid(grid_of(m * n * sc, 256));
             if (Pw[0] >= (1u << 31))
                 hipLaunchKernelGGL((few_primes_crt_kernel<kFewMaxPrimes, true>), grid, dim3(256), 0, s,
-                                   (const uint32_t *)rc, m * n, sc, fp->d_const, r, Pw[0], c);
+                                   (const uint32_t *)rc, m * n, sc, fp->d_const, r, Pw[0], cv);
             else
                 hipLaunchKernelGGL((few_primes_crt_kernel<kFewMaxPrimes, false>), grid, dim3(256), 0, s,
-                                   (const uint32_t *)rc, m * n, sc, fp->d_const, r, Pw[0], c);
+                                   (const uint32_t *)rc, m * n, sc, fp->d_const, r, Pw[0], cv);
             LBX_TRY_HIP(hipGetLastError());
+            if (cv.base != c.base) LBX_TRY_HIP(launch_copy(cv, c, m * n, sc, 0, 0, s));
             return LBX_OK;
         }
     }

@@ -307,17 +307,18 @@ __device__ __forceinline__ void mfma_tile_lds(const uint4 *__restrict__ lA, cons
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) const void global_cvoid;
 
-// Global -> LDS copy of `chunks` 16-byte chunks (a multiple of 256) with the
+// Global -> LDS copy of `chunks` 16-byte chunks (a multiple of 64) with the
 // row swizzle, using global_load_lds_dwordx4: each wave instruction fills 64
 // consecutive LDS chunks (1 KiB at M0 + 16*lane) with no register staging, so
 // every load of the copy is in flight at once.  Lane i of a wave's j-th
 // instruction fills LDS chunk P = 64*(4j + wave) + i, i.e. row r = P / cpr,
 // swizzled column P % cpr, which holds global chunk r*cpr + ((P % cpr) ^ (r & 15)).
+// NW waves share the copy (P = 64*(NW*j + wave) + i).
+template <int NW = 4>
 __device__ __forceinline__ void copy_lds(const uint4 *__restrict__ g, uint4 *l, int chunks, int cpr, int wave,
                                          int lane)
 {
-    for (int j = 0; j * 256 < chunks; ++j) {
-        const int base = 64 * (4 * j + wave);
+    for (int base = 64 * wave; base < chunks; base += 64 * NW) {
         const int P = base + lane;
         const int r = P / cpr, c = P - r * cpr;
         __builtin_amdgcn_global_load_lds((global_cvoid *)(g + r * cpr + (c ^ (r & 15))), (lds_void *)(l + base), 16,
@@ -366,7 +367,7 @@ __global__ void __launch_bounds__(256, 2) pw_mfma_lds_kernel(const uint8_t *__re
     }
 }
 
-// A in registers, B in LDS: for mpad in {32, 64, 128}, k <= 128 and a B block
+// A in registers, B in LDS: for mpad in {32, 64, 96, 128}, k <= 128 and a B block
 // of at most 64 KiB.  Each wave multiplies one 32-row band of A, which it
 // loads straight into registers (64 VGPRs at k = 128); only B, which every
 // wave needs, goes through LDS, whole, with one LDS-direct copy.  A point
@@ -374,8 +375,10 @@ __global__ void __launch_bounds__(256, 2) pw_mfma_lds_kernel(const uint8_t *__re
 // flight together; two groups per CU overlap one's loads with the other's
 // multiplies.  With nrt = mpad/32 < 4 bands, wave w takes band w % nrt and
 // every (4/nrt)-th column block from w / nrt.
-template <int KC>
-__global__ void __launch_bounds__(256, 2) pw_mfma_rega_kernel(const uint8_t *__restrict__ Al,
+// Three bands (mpad = 96) take groups of three waves, one band each: 96x48x80 at
+// 2^12 points 88 us, against 107 us in the LDS form above.
+template <int KC, int NW>
+__global__ void __launch_bounds__(64 * NW, 2) pw_mfma_rega_kernel(const uint8_t *__restrict__ Al,
                                                               const uint8_t *__restrict__ Bl,
                                                               uint32_t *__restrict__ Cmat, int m, int n, int mpad,
                                                               int npad, size_t npts, uint32_t p, MfmaConst mc)
@@ -386,12 +389,12 @@ __global__ void __launch_bounds__(256, 2) pw_mfma_rega_kernel(const uint8_t *__r
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, lg = lane >> 4;
     const int a_chunks = mpad * cpr, b_chunks = npad * cpr;
     const int nrt = mpad / 32, ncb = npad / 32;
-    const int band = wave % nrt, cb0 = wave / nrt, cbs = 4 / nrt;
+    const int band = wave % nrt, cb0 = wave / nrt, cbs = NW / nrt;
     for (size_t t = blockIdx.x; t < npts; t += gridDim.x) {
         const uint4 *gA = reinterpret_cast<const uint4 *>(Al) + t * (size_t)a_chunks;
         const uint4 *gB = reinterpret_cast<const uint4 *>(Bl) + t * (size_t)b_chunks;
         __syncthreads();  // the previous point is done with lB
-        copy_lds(gB, lB, b_chunks, cpr, wave, lane);
+        copy_lds<NW>(gB, lB, b_chunks, cpr, wave, lane);
         v4i a[2][KC][4];
 #pragma unroll
         for (int sub = 0; sub < 2; ++sub)
@@ -709,13 +712,15 @@ hipError_t launch_pointwise_mfma(const uint8_t *Al, const uint8_t *Bl, uint32_t 
     if (npts > 0x7fffffff) return hipErrorInvalidValue;
     const size_t a_bytes = limb_block_bytes(m, k);
     const int cus = device_cus();
-    if ((mpad == 32 || mpad == 64 || mpad == 128) && kchunks <= 2 && npad * kchunks * 256 <= 65536) {
+    if (mpad <= 128 && kchunks <= 2 && npad * kchunks * 256 <= 65536) {
         const size_t lds = npad * kchunks * 256;
         const size_t grid = npts < (size_t)cus * 2 ? npts : (size_t)cus * 2;
-        auto k = kchunks == 1 ? pw_mfma_rega_kernel<1> : pw_mfma_rega_kernel<2>;
+        const int nw = mpad == 96 ? 3 : 4;
+        auto k = nw == 3 ? (kchunks == 1 ? pw_mfma_rega_kernel<1, 3> : pw_mfma_rega_kernel<2, 3>)
+                         : (kchunks == 1 ? pw_mfma_rega_kernel<1, 4> : pw_mfma_rega_kernel<2, 4>);
         hipError_t e = hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(256), lds, s, Al, Bl, Cmat, (int)m, (int)n, (int)mpad,
+        hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(64 * nw), lds, s, Al, Bl, Cmat, (int)m, (int)n, (int)mpad,
                            (int)npad, npts, p, mc);
         return hipGetLastError();
     }

@@ -554,3 +554,48 @@ def test_mul_plain_point_major(ctx, monkeypatch):
         say("plain point-major chunked", p, m, k, n, sa, sb)
         got = gpu_mul(ctx, p, m, k, n, a, sa, b, sb, lbx.METHOD_PLAIN_U64)
         assert np.array_equal(got.reshape(-1), ref)
+
+
+@pytest.mark.parametrize("p,m,k,n,sa,sb,layouts", [
+    # a, b and the result on both sides of the 2^21-word line of the polfirst copies
+    (998244353, 64, 64, 64, 513, 512, ("matfirst", "matfirst", "matfirst")),
+    (2013265921, 64, 64, 64, 510, 514, ("matrowfirst", "matrowfirst", "matrowfirst")),
+    # odd entry counts (no 16-byte rows), an operand that fills the transform
+    (469762049, 63, 65, 61, 1024, 1, ("matfirst", "matfirst", "matrowfirst")),
+    (998244353, 7, 300, 5, 1021, 1000, ("matrowfirst", "matfirst", "matfirst")),
+    # whole transforms (plain form), three FFT primes, and one word above 2^31
+    (167772161, 9, 16, 100, 3001, 4000, ("matfirst", "matfirst", "matfirst")),
+    (268435399, 32, 48, 40, 1400, 1300, ("matfirst", "matrowfirst", "matfirst")),
+    (4294967291, 33, 64, 40, 1000, 900, ("matfirst", "matrowfirst", "matrowfirst")),
+    # 65..96 rows of A
+    (998244353, 65, 64, 33, 520, 400, ("polfirst", "matfirst", "matfirst")),
+    (2013265921, 96, 128, 130, 300, 280, ("matfirst", "matfirst", "polfirst")),
+])
+def test_mul_layouts_large(ctx, monkeypatch, p, m, k, n, sa, sb, layouts):
+    """Large operands in each layout, as windows of larger storage, and with
+    split transforms in several chunks, against the polfirst product of the
+    same operands; that one is checked by evaluation at a random point."""
+    rng = np.random.default_rng(m * k * n + sa)
+    a, b = rand(rng, p, m * k * sa).reshape(m * k, sa), rand(rng, p, k * n * sb).reshape(k * n, sb)
+    dom = PolynomialMatrixMulDomain(p, ctx)
+    ref = PolynomialMatrix(m, n, sa + sb - 1)
+    dom.mul(ref, PolynomialMatrix.from_polfirst(a, m, k), PolynomialMatrix.from_polfirst(b, k, n))
+    ref = ref.to_polfirst()
+    x = int(rng.integers(1, p))
+    assert check_by_evaluation(a, b, ref, p, m, k, n, sa, sb, sa + sb - 1, [x])
+
+    def stored(x, rows, cols, layout, off):
+        big = np.zeros((rows * cols, x.shape[1] + 7), np.uint32)
+        big[:, off:off + x.shape[1]] = x
+        M = PolynomialMatrix.from_polfirst(big, rows, cols, layout)
+        return M, M.at(off, off + x.shape[1] - 1)
+
+    for chunk in (None, 1 << 22):
+        if chunk:
+            monkeypatch.setenv("LBX_CHUNK_BYTES", str(chunk))
+        say("layouts large", p, m, k, n, sa, sb, layouts, chunk)
+        C, Cv = stored(np.full((m * n, sa + sb - 1), 7, np.uint32), m, n, layouts[2], 3)
+        dom.mul(Cv, stored(a, m, k, layouts[0], 4)[1], stored(b, k, n, layouts[1], 5)[1])
+        got = C.to_polfirst()
+        assert np.array_equal(got[:, 3:3 + sa + sb - 1], ref)
+        assert not got[:, :3].any() and not got[:, 3 + sa + sb - 1:].any()  # the rest of the storage is kept
