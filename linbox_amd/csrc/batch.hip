@@ -600,15 +600,6 @@ lbx_status run_batch_plan(lbx_ctx *ctx, const std::vector<lbx_job> &bj, const st
     return LBX_OK;
 }
 
-lbx_status batch_products(lbx_ctx *ctx, const lbx_job *jobs, size_t njobs, hipStream_t s)
-{
-    std::vector<lbx_job> bj(jobs, jobs + njobs);
-    std::vector<unsigned> Ls(njobs);
-    for (size_t i = 0; i < njobs; ++i)
-        if (!batchable(jobs[i], &Ls[i])) return LBX_ERR_UNSUPPORTED;
-    return run_batch_plan(ctx, bj, Ls, s);
-}
-
 }  // namespace lbx
 
 using namespace lbx;

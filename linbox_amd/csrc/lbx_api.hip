@@ -214,17 +214,19 @@ private:
 };
 
 // AUTO picks the INT8 form where it measured faster on gfx950 (both forms are
-// bit-exact): for large products (m*k*n >= 2^18) and for short transforms
-// (at most 2^9 points); in between, the split transforms the INT8 form needs
-// cost more than the VALU pointwise they replace (16^3 at 2^14 points: 0.25 ms
-// INT8, 0.08 ms plain; 32^3 at 2^13: 0.20 vs 0.13 ms; 64^3 at 2^11: 0.14 vs
-// 0.16 ms; 16^3 at 2^9: 0.032 vs 0.036 ms).  MFMA tiles are 32x32 with a
-// 64-deep inner step, so every dimension must be at least 16.
+// bit-exact): for large products.  Below, the split transforms and the seven
+// launches it needs cost more than the VALU pointwise they replace (plain /
+// INT8, us: 32^3 at 2^8 points 27 / 36, at 2^13 116 / 177; 48^3 at 2^13 311 /
+// 304; 64^2x32 at 2^11 91 / 97, at 2^13 347 / 291; 64^3 at 2^6 33 / 43, at 2^8
+// 45 / 44, at 2^10 91 / 81, at 2^13 616 / 427; 96^3 at 2^8 99 / 65).  MFMA tiles
+// are 32x32 with a 64-deep inner step, so every dimension must be at least 16,
+// and an inner dimension below 32 is mostly padding (100x17x100 at 2^13: 557 / 719).
 int choose_method(int method, size_t m, size_t k, size_t n, unsigned L)
 {
     if (method == LBX_METHOD_PLAIN_U64 || method == LBX_METHOD_INT8_MFMA) return method;
     if (m < 16 || n < 16 || k < 16) return LBX_METHOD_PLAIN_U64;
-    const bool big = (double)m * k * n >= (double)(1u << 18) || L <= 9;
+    const double mkn = (double)m * k * n, two17 = (double)(1u << 17);
+    const bool big = mkn >= 4 * two17 || (mkn >= 2 * two17 && L >= 8) || (mkn >= two17 && k >= 32 && L >= 13);
     return big ? LBX_METHOD_INT8_MFMA : LBX_METHOD_PLAIN_U64;
 }
 
@@ -360,6 +362,22 @@ bool copies_to_polfirst(const DevView &v, size_t entries, size_t count, unsigned
            count >= ((size_t)1 << 21) / entries + 1;
 }
 
+lbx_status multi_prime(MultiProduct &mp, unsigned i, uint32_t p, const MidSpec *mid, Workspace &ws, hipStream_t s)
+{
+    uint32_t w;
+    LBX_TRY(primitive_root(p, mp.L, &w));
+    const uint32_t wi = invroot(p, mp.L, w);
+    const uint2 *twf, *twi = nullptr;
+    LBX_TRY(ws.twiddle_table(p, mp.L, w, kTwMont, &twf, s));
+    LBX_TRY(ws.twiddle_table(p, mp.L, mid ? w : wi, kTwShoup, &mp.twc[i], s));
+    if (mid) LBX_TRY(ws.twiddle_table(p, mp.L, wi, kTwMont, &twi, s));
+    mp.p[i] = p;
+    mp.twa[i] = mid && !mid->small_left ? twi : twf;
+    mp.twb[i] = mid && mid->small_left ? twi : twf;
+    mp.pc[i] = plain_const(p, invmod_h((uint32_t)(((size_t)1 << mp.L) % p), p));
+    return LBX_OK;
+}
+
 // Forward transforms, pointwise products and inverse transform of one
 // single-prime product on device views.  deg+1 coefficients of c are written.
 // Every device buffer is taken from the workspace before the first launch.
@@ -371,6 +389,12 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
     Workspace &ws = ws_in ? *ws_in : ctx_ws;
     const size_t N = (size_t)1 << L;
     if (L > (unsigned)kMaxLog) return LBX_ERR_UNSUPPORTED;
+    method = choose_method(method, m, k, n, L);
+    const bool int8 = method == LBX_METHOD_INT8_MFMA;
+    const bool split = L >= 8 && L <= (unsigned)kMaxLdsLog && (int8 || plain_point_major(m, k, n));
+    // whole transforms of both operands in one launch (a middle product's
+    // reversal included)
+    const bool fused = !split && !int8 && L >= 1 && L <= (unsigned)kMaxLdsLog;
     uint32_t w;
     LBX_TRY(primitive_root(p, L, &w));
     const uint32_t wi = invroot(p, L, w);
@@ -389,12 +413,9 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
         LBX_TRY(ws.twiddle_table(p, L, wi, kTwMont, &twfi, s));
         (mid->small_left ? twb : twa) = twfi;
         const size_t se = mid->small_left ? m * k : k * n;
-        LBX_TRY(ws.get("mid_rev", se * mid->hdeg * 4, &rev));
+        if (!fused) LBX_TRY(ws.get("mid_rev", se * mid->hdeg * 4, &rev));
     }
     const uint32_t inv_n = invmod_h((uint32_t)(N % p), p);
-    method = choose_method(method, m, k, n, L);
-    const bool int8 = method == LBX_METHOD_INT8_MFMA;
-    const bool split = L >= 8 && L <= (unsigned)kMaxLdsLog && (int8 || plain_point_major(m, k, n));
 
     // ---- buffers ----
     void *al = nullptr, *bl = nullptr, *cmat = nullptr, *scr = nullptr, *ahat = nullptr, *bhat = nullptr,
@@ -462,7 +483,7 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
         if (out.base != c.base) LBX_TRY_HIP(launch_copy(out, c, m * n, count, 0, 0, s));
         return LBX_OK;
     };
-    if (mid) {
+    if (mid && !fused) {
         const DevView sm = mid->small_left ? a : b;
         const size_t se = mid->small_left ? m * k : k * n;
         LBX_TRY_HIP(launch_reverse_gather(sm, se, mid->hdeg, (uint32_t *)rev, s));
@@ -540,6 +561,36 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
         st.mark("inverse FFT_DIT");
         return LBX_OK;
     }
+    if (fused) {
+        MultiProduct mp{};
+        mp.r = 1;
+        mp.L = L;
+        mp.m = m, mp.k = k, mp.n = n;
+        mp.a = a, mp.b = b, mp.c = out;
+        mp.rev_a = mid && mid->small_left ? mid->hdeg : 0;
+        mp.rev_b = mid && !mid->small_left ? mid->hdeg : 0;
+        mp.ahat = (uint32_t *)ahat, mp.bhat = (uint32_t *)bhat, mp.chat = (uint32_t *)chat;
+        mp.count = count;
+        mp.p[0] = p, mp.twa[0] = twa, mp.twb[0] = twb, mp.twc[0] = twc;
+        mp.pc[0] = plain_const(p, inv_n);
+        {
+            KernelTimer kt(ctx, s, "kernel dif", timing);
+            LBX_TRY_HIP(launch_multi_forward(mp, s));
+        }
+        st.mark("direct FFT_DIF");
+        {
+            KernelTimer kt(ctx, s, "kernel pw_plain", timing);
+            LBX_TRY_HIP(launch_multi_pointwise(mp, s));
+        }
+        st.mark("Pointwise mult");
+        {
+            KernelTimer kt(ctx, s, "kernel dit", timing);
+            LBX_TRY_HIP(launch_multi_inverse(mp, s));
+        }
+        LBX_TRY(store_result());
+        st.mark("inverse FFT_DIT");
+        return LBX_OK;
+    }
     {
         KernelTimer kt(ctx, s, "kernel dif a", timing);
         LBX_TRY_HIP(launch_ntt_forward(a, m * k, L, twa, p, (uint32_t *)ahat, s));
@@ -561,8 +612,9 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
     } else {
         {
             KernelTimer kt(ctx, s, "kernel pw_plain", timing);
+            const PlainConst pc = plain_const(p, inv_n);
             LBX_TRY_HIP(launch_pointwise_plain((const uint32_t *)ahat, (const uint32_t *)bhat, (uint32_t *)chat, m, k,
-                                               n, N, p, inv_n, s));
+                                               n, N, 1, &p, &pc, s));
         }
         st.mark("Pointwise mult");
     }
@@ -587,8 +639,9 @@ lbx_status constant_product(lbx_ctx *ctx, uint32_t p, const DevView &a, const De
     LBX_TRY(ws.get("chat", m * n * 4, &chat));
     LBX_TRY_HIP(launch_gather(a, m * k, 1, (uint32_t *)ahat, 1, s));
     LBX_TRY_HIP(launch_gather(b, k * n, 1, (uint32_t *)bhat, 1, s));
-    LBX_TRY_HIP(launch_pointwise_plain((const uint32_t *)ahat, (const uint32_t *)bhat, (uint32_t *)chat, m, k, n, 1,
-                                       p, 1, s));
+    const PlainConst pc = plain_const(p, 1);
+    LBX_TRY_HIP(launch_pointwise_plain((const uint32_t *)ahat, (const uint32_t *)bhat, (uint32_t *)chat, m, k, n, 1, 1,
+                                       &p, &pc, s));
     LBX_TRY_HIP(launch_scatter((const uint32_t *)chat, 1, m * n, 1, c, s));
     return LBX_OK;
 }

@@ -248,6 +248,10 @@ struct MidSpec {
 lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView &a, const DevView &b,
                              const DevView &c, size_t m, size_t k, size_t n, size_t count, int method,
                              hipStream_t s, const MidSpec *mid = nullptr, Workspace *ws = nullptr);
+// Fills entry i of a MultiProduct's per-prime constants: p, the scale 2^-L and
+// the twiddle tables of its root of order 2^L (mid: the small operand with w,
+// the other with w^-1, the inverse with w).
+lbx_status multi_prime(MultiProduct &mp, unsigned i, uint32_t p, const MidSpec *mid, Workspace &ws, hipStream_t s);
 // Product (mid == nullptr; c holds sa+sb-1 coefficients) or midproduct with
 // 2^L points over Z/PZ (P of nl little-endian limbs) through FFT primes and
 // CRT (matpoly-mult-fft-multiprecision.inl:141-277, 427-520).
@@ -267,10 +271,6 @@ lbx_status noalloc_attach(int device);
 void mp_release(lbx_ctx *ctx);
 // Frees the batch plans (graphs, descriptors) cached in a context.
 void batch_release(lbx_ctx *ctx);
-// Independent polfirst products with device operands through the batch
-// kernels, the context lock held; LBX_ERR_UNSUPPORTED (nothing launched) when a
-// job is outside their range.
-lbx_status batch_products(lbx_ctx *ctx, const lbx_job *jobs, size_t njobs, hipStream_t s);
 // Whether the plain form takes point-major operands (split transforms) for m x k x n.
 bool plain_point_major(size_t m, size_t k, size_t n);
 // Whether a view of `entries` x `count` coefficients that is not polfirst goes

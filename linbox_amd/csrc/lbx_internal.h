@@ -121,11 +121,40 @@ hipError_t launch_ntt_inverse_tail(const uint32_t *in, size_t entries, unsigned 
                                    uint32_t p, const DevView &out, size_t out_first, size_t count, uint32_t scale,
                                    hipStream_t s);
 
+// ---- plain products by several primes at once (multi.hip) ----
+// The entry-major plain form of one or more products A_i B_i mod p_i of the
+// same shape at the same length 2^L, L <= kMaxLdsLog, in three launches: the
+// forward transforms of both operands for every prime, the pointwise
+// products, and the inverse transforms.  At most kMultiPrimes primes, whose
+// constants travel in the kernel arguments.
+constexpr int kMultiPrimes = 32;
+struct MultiProduct {
+    unsigned r, L;
+    size_t m, k, n;
+    // operands of prime i: the views at base + i * stride words (0: every prime
+    // reads the same words); rev_x != 0: the first rev_x coefficients reversed
+    // (zero beyond the view), as the small operand of a middle product
+    DevView a, b;
+    size_t astride, bstride;
+    size_t rev_a, rev_b;
+    uint32_t *ahat, *bhat, *chat;  // r x (m k, k n, m n) rows of 2^L words
+    DevView c;                     // result of prime i at base + i * cstride: count coefficients
+    size_t cstride, count;
+    uint32_t p[kMultiPrimes];
+    const uint2 *twa[kMultiPrimes], *twb[kMultiPrimes], *twc[kMultiPrimes];  // Montgomery, Montgomery, Shoup tables
+    PlainConst pc[kMultiPrimes];                                           // with the scale 2^-L
+};
+hipError_t launch_multi_forward(const MultiProduct &mp, hipStream_t s);
+hipError_t launch_multi_pointwise(const MultiProduct &mp, hipStream_t s);
+hipError_t launch_multi_inverse(const MultiProduct &mp, hipStream_t s);
+
 // ---- pointwise stage (pointwise.hip) ----
 // C[e'][t] = scale * sum_q A[i*k+q][t] B[q*n+j][t] mod p at every point t < npts,
-// all operands polfirst with row stride npts (e' = i*n+j).
+// all operands polfirst with row stride npts (e' = i*n+j); r such products, of
+// primes p[i] with constants pc[i], one after the other in each buffer.
 hipError_t launch_pointwise_plain(const uint32_t *A, const uint32_t *B, uint32_t *C, size_t m, size_t k,
-                                  size_t n, size_t npts, uint32_t p, uint32_t scale, hipStream_t s);
+                                  size_t n, size_t npts, unsigned r, const uint32_t *p, const PlainConst *pc,
+                                  hipStream_t s);
 
 // Bytes of one point's limb block for an operand with `rows` rows and inner
 // dimension kdim (rows padded to 32, inner dimension to 64, four planes).

@@ -21,6 +21,7 @@
 // The reference picks ~23-bit primes for fgemm on doubles (:162-164); the
 // primes here are 31-bit because every step is 32-bit integer arithmetic.
 // Products are unique, so the output is identical.
+#include <algorithm>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -475,22 +476,65 @@ unsigned grid_of(size_t total, unsigned block)
     return (unsigned)(g < 8192 ? (g ? g : 1) : 8192);
 }
 
-// The r per-prime products c_i = a_i b_i (polfirst, contiguous; operand i at
-// a + i*astride) as one call of the batch kernels, when the pointwise form
-// this shape takes is their plain one: a few launches in place of r separate
-// products.  LBX_ERR_UNSUPPORTED (nothing launched) otherwise.
-lbx_status primes_as_batch(lbx_ctx *ctx, const std::vector<uint32_t> &primes, const uint32_t *a, size_t astride,
-                           const uint32_t *b, size_t bstride, uint32_t *c, size_t m, size_t k, size_t n, size_t sa,
-                           size_t sb, unsigned lpts, int method, hipStream_t s)
-{
-    if (sa + sb <= 2 || choose_method(method, m, k, n, lpts) != LBX_METHOD_PLAIN_U64) return LBX_ERR_UNSUPPORTED;
-    std::vector<lbx_job> jobs(primes.size());
-    for (size_t i = 0; i < primes.size(); ++i)
-        jobs[i] = lbx_job{primes[i], m, k, n, sa, sb, a + i * astride, b + i * bstride, c + i * m * n * (sa + sb - 1)};
-    return batch_products(ctx, jobs.data(), jobs.size(), s);
-}
+// The r products c_i = a_i b_i mod p_i of one shape (operand i of a at the view
+// a + i * astride words, b alike; c_i polfirst with sc coefficients, one after
+// the other).  Where the pointwise form is the plain one on whole transforms,
+// all primes go through three launches, in chunks of primes whose transforms
+// fit kMultiWords words of scratch (larger products fill the chip prime by
+// prime); a prime by itself otherwise.  Measured (us), one prime at a time /
+// chunks of 2^24 / 2^25 / 2^26 / 2^27 words: 14 primes of 32^3 at 2^11 points
+// 950 / 668 / 617 / 580 / 583; 3 primes of 16^3 at 2^11 78 / 46 / 45 / 45 / 46; 3 of
+// 32^3 at 2^13 372 / 372 / 373 / 371 / 373.
+constexpr size_t kMultiWords = (size_t)1 << 26;
 
-constexpr int kBatchMinPrimes = 6;
+lbx_status prime_products(lbx_ctx *ctx, const std::vector<uint32_t> &primes, const DevView &a, size_t astride,
+                          const DevView &b, size_t bstride, uint32_t *c, size_t m, size_t k, size_t n, size_t sc,
+                          unsigned L, int method, hipStream_t s, const MidSpec *mid)
+{
+    const size_t r = primes.size();
+    if (choose_method(method, m, k, n, L) != LBX_METHOD_PLAIN_U64 || plain_point_major(m, k, n) || L < 1 ||
+        L > (unsigned)kMaxLdsLog) {
+        for (size_t i = 0; i < r; ++i) {
+            DevView va = a, vb = b;
+            va.base += i * astride;
+            vb.base += i * bstride;
+            const DevView vc{c + i * m * n * sc, LBX_POLFIRST, m, n, sc, 0, sc};
+            if (!mid && a.size + b.size <= 2 && sc == 1)
+                LBX_TRY(constant_product(ctx, primes[i], va, vb, vc, m, k, n, s));
+            else
+                LBX_TRY(fft_prime_product(ctx, primes[i], L, va, vb, vc, m, k, n, sc, method, s, mid));
+        }
+        return LBX_OK;
+    }
+    const size_t N = (size_t)1 << L, words = (m * k + k * n + m * n) * N;
+    const size_t chunk = std::min<size_t>({std::max<size_t>(kMultiWords / words, 1), r, (size_t)kMultiPrimes});
+    CtxWorkspace ws(ctx);
+    MultiProduct mp{};
+    mp.L = L;
+    mp.m = m, mp.k = k, mp.n = n;
+    mp.astride = astride, mp.bstride = bstride;
+    mp.rev_a = mid && mid->small_left ? mid->hdeg : 0;
+    mp.rev_b = mid && !mid->small_left ? mid->hdeg : 0;
+    mp.cstride = m * n * sc;
+    mp.count = sc;
+    void *ahat, *bhat, *chat;
+    LBX_TRY(ws.get("ahat", chunk * m * k * N * 4, &ahat));
+    LBX_TRY(ws.get("bhat", chunk * k * n * N * 4, &bhat));
+    LBX_TRY(ws.get("chat", chunk * m * n * N * 4, &chat));
+    mp.ahat = (uint32_t *)ahat, mp.bhat = (uint32_t *)bhat, mp.chat = (uint32_t *)chat;
+    for (size_t i0 = 0; i0 < r; i0 += chunk) {
+        mp.r = (unsigned)std::min(chunk, r - i0);
+        mp.a = a, mp.b = b;
+        mp.a.base += i0 * astride;
+        mp.b.base += i0 * bstride;
+        mp.c = DevView{c + i0 * mp.cstride, LBX_POLFIRST, m, n, sc, 0, sc};
+        for (unsigned i = 0; i < mp.r; ++i) LBX_TRY(multi_prime(mp, i, primes[i0 + i], mid, ws, s));
+        LBX_TRY_HIP(launch_multi_forward(mp, s));
+        LBX_TRY_HIP(launch_multi_pointwise(mp, s));
+        LBX_TRY_HIP(launch_multi_inverse(mp, s));
+    }
+    return LBX_OK;
+}
 
 lbx_status get_plan(lbx_ctx *ctx, const uint32_t *Pw, int nl, size_t k, size_t minsz, unsigned lpts, MpPlan **out)
 {
@@ -641,7 +685,6 @@ lbx_status mp_product(lbx_ctx *ctx, const uint32_t *Pw, int nl, const DevView &a
     // product: s = max_rowdeg+1 coefficients when given, else sa+sb-1 (mul_crtla :150-152;
     // three-primes.inl:69-73); with fewer than sa+sb-1 the cyclic product mod x^pts - 1
     const size_t sa = a.size, sb = b.size, sc = mid ? c.size : (count ? count : sa + sb - 1);
-    const bool full = !mid && sc == sa + sb - 1;
     unsigned lpts = 0;
     size_t pts = 1;
     while (pts < sc) {  // mul_crtla :151-154
@@ -689,20 +732,13 @@ lbx_status mp_product(lbx_ctx *ctx, const uint32_t *Pw, int nl, const DevView &a
                 return launch_copy(v, pf, entries, v.size, 0, 0, s) == hipSuccess ? pf : v;
             };
             const DevView a1 = as_polfirst(a, m * k, "mp_ra"), b1 = as_polfirst(b, k * n, "mp_rb");
-            for (int i = 0; i < r; ++i) {
-                DevView va = a1, vb = b1;
-                if (fp->reduce) {
-                    va = DevView{(uint32_t *)ra + (size_t)i * m * k * sa, LBX_POLFIRST, m, k, sa, 0, sa};
-                    vb = DevView{(uint32_t *)rb + (size_t)i * k * n * sb, LBX_POLFIRST, k, n, sb, 0, sb};
-                }
-                DevView vc{(uint32_t *)rc + (size_t)i * m * n * sc, LBX_POLFIRST, m, n, sc, 0, sc};
-                if (mid)
-                    LBX_TRY(fft_prime_product(ctx, fp->primes[i], lpts, va, vb, vc, m, k, n, sc, method, s, mid));
-                else if (sa + sb <= 2 && sc == 1)
-                    LBX_TRY(constant_product(ctx, fp->primes[i], va, vb, vc, m, k, n, s));
-                else
-                    LBX_TRY(fft_prime_product(ctx, fp->primes[i], lpts, va, vb, vc, m, k, n, sc, method, s));
+            DevView va = a1, vb = b1;
+            if (fp->reduce) {
+                va = DevView{(uint32_t *)ra, LBX_POLFIRST, m, k, sa, 0, sa};
+                vb = DevView{(uint32_t *)rb, LBX_POLFIRST, k, n, sb, 0, sb};
             }
+            LBX_TRY(prime_products(ctx, fp->primes, va, fp->reduce ? m * k * sa : 0, vb, fp->reduce ? k * n * sb : 0,
+                                   (uint32_t *)rc, m, k, n, sc, lpts, method, s, mid));
             // a result stored by coefficient is recombined polfirst, in the place
             // of the first prime's residues, and copied out in one pass
             DevView cv = c;
@@ -733,24 +769,9 @@ lbx_status mp_product(lbx_ctx *ctx, const uint32_t *Pw, int nl, const DevView &a
     hipLaunchKernelGGL(residues, dim3(grid_of(k * n * sb, 256)), dim3(256), 0, s, b, nl, k * n, sb, plan->d_const, r,
                        (uint32_t *)rb);
     LBX_TRY_HIP(hipGetLastError());
-    // many primes (multiword moduli): the products as one batch; a new shape
-    // builds and caches a batch plan (graph capture), which pays off here
-    lbx_status bst = LBX_ERR_UNSUPPORTED;
-    if (full && r >= kBatchMinPrimes)
-        bst = primes_as_batch(ctx, plan->primes, (const uint32_t *)ra, m * k * sa, (const uint32_t *)rb, k * n * sb,
-                              (uint32_t *)rc, m, k, n, sa, sb, lpts, method, s);
-    if (bst != LBX_ERR_UNSUPPORTED) LBX_TRY(bst);
-    for (int i = 0; i < r && bst == LBX_ERR_UNSUPPORTED; ++i) {
-        DevView va{(uint32_t *)ra + (size_t)i * m * k * sa, LBX_POLFIRST, m, k, sa, 0, sa};
-        DevView vb{(uint32_t *)rb + (size_t)i * k * n * sb, LBX_POLFIRST, k, n, sb, 0, sb};
-        DevView vc{(uint32_t *)rc + (size_t)i * m * n * sc, LBX_POLFIRST, m, n, sc, 0, sc};
-        if (mid)
-            LBX_TRY(fft_prime_product(ctx, plan->primes[i], lpts, va, vb, vc, m, k, n, sc, method, s, mid));
-        else if (sa + sb <= 2 && sc == 1)
-            LBX_TRY(constant_product(ctx, plan->primes[i], va, vb, vc, m, k, n, s));
-        else
-            LBX_TRY(fft_prime_product(ctx, plan->primes[i], lpts, va, vb, vc, m, k, n, sc, method, s));
-    }
+    const DevView va{(uint32_t *)ra, LBX_POLFIRST, m, k, sa, 0, sa}, vb{(uint32_t *)rb, LBX_POLFIRST, k, n, sb, 0, sb};
+    LBX_TRY(prime_products(ctx, plan->primes, va, m * k * sa, vb, k * n * sb, (uint32_t *)rc, m, k, n, sc, lpts, method,
+                           s, mid));
     const dim3 grid(grid_of(m * n * sc, 128));
     const int nlm = crt_width(r, nl).nlm;
     if (nlm == 2)
@@ -935,7 +956,6 @@ lbx_status zz_product(lbx_ctx *ctx, int nl, int cl, const DevView &a, const DevV
                       size_t k, size_t n, size_t sc, int method, hipStream_t s)
 {
     const size_t sa = a.size, sb = b.size;
-    const bool full = sc == sa + sb - 1;
     unsigned lpts = 0;
     size_t pts = 1;
     while (pts < sc) {  // mul_crtla :151-154
@@ -995,20 +1015,9 @@ lbx_status zz_product(lbx_ctx *ctx, int nl, int cl, const DevView &a, const DevV
     hipLaunchKernelGGL(residues, dim3(grid_of(k * n * sb, 256)), dim3(256), 0, s, b, nl, k * n, sb,
                        (const uint32_t *)dk, r, (uint32_t *)rb);
     LBX_TRY_HIP(hipGetLastError());
-    lbx_status bst = LBX_ERR_UNSUPPORTED;
-    if (full && r >= kBatchMinPrimes)
-        bst = primes_as_batch(ctx, primes, (const uint32_t *)ra, m * k * sa, (const uint32_t *)rb, k * n * sb,
-                              (uint32_t *)rc, m, k, n, sa, sb, lpts, method, s);
-    if (bst != LBX_ERR_UNSUPPORTED) LBX_TRY(bst);
-    for (int i = 0; i < r && bst == LBX_ERR_UNSUPPORTED; ++i) {
-        DevView va{(uint32_t *)ra + (size_t)i * m * k * sa, LBX_POLFIRST, m, k, sa, 0, sa};
-        DevView vb{(uint32_t *)rb + (size_t)i * k * n * sb, LBX_POLFIRST, k, n, sb, 0, sb};
-        DevView vc{(uint32_t *)rc + (size_t)i * m * n * sc, LBX_POLFIRST, m, n, sc, 0, sc};
-        if (sa + sb <= 2 && sc == 1)
-            LBX_TRY(constant_product(ctx, primes[i], va, vb, vc, m, k, n, s));
-        else
-            LBX_TRY(fft_prime_product(ctx, primes[i], lpts, va, vb, vc, m, k, n, sc, method, s));
-    }
+    const DevView va{(uint32_t *)ra, LBX_POLFIRST, m, k, sa, 0, sa}, vb{(uint32_t *)rb, LBX_POLFIRST, k, n, sb, 0, sb};
+    LBX_TRY(prime_products(ctx, primes, va, m * k * sa, vb, k * n * sb, (uint32_t *)rc, m, k, n, sc, lpts, method, s,
+                           nullptr));
     hipLaunchKernelGGL(zz_crt_kernel, dim3(grid_of(m * n * sc, 128)), dim3(128), 0, s, (const uint32_t *)rc, m * n,
                        sc, (const uint32_t *)dk, r, cl, c);
     LBX_TRY_HIP(hipGetLastError());

@@ -237,6 +237,28 @@ constexpr int dif_last_rp()
     return (SEND % Cfg<L>::RLOG) ? (SEND % Cfg<L>::RLOG) : Cfg<L>::RLOG;
 }
 
+// The words of a whole forward transform (all L stages) to its row o.
+template <int L>
+__device__ __forceinline__ void dif_store(const uint32_t (&x)[Cfg<L>::R], int tp, uint32_t *__restrict__ o)
+{
+    using C = Cfg<L>;
+    constexpr int RP = dif_last_rp<L, L>();
+#pragma unroll
+    for (int u = 0; u < (C::R >> RP); ++u) {
+        const int g = tp + u * C::TP;
+        if constexpr (RP >= 2) {
+#pragma unroll
+            for (int q = 0; q < (1 << RP); q += 4)
+                *reinterpret_cast<uint4 *>(o + (g << RP) + q) =
+                    make_uint4(x[u * (1 << RP) + q], x[u * (1 << RP) + q + 1], x[u * (1 << RP) + q + 2],
+                               x[u * (1 << RP) + q + 3]);
+        } else {
+#pragma unroll
+            for (int q = 0; q < (1 << RP); ++q) o[(g << RP) + q] = x[u * (1 << RP) + q];
+        }
+    }
+}
+
 // DIF stages [0, SEND) of one polynomial per TP threads.  With SEND == L the
 // result is the full transform (R consecutive words per thread are stored as
 // 16-byte vectors); with SEND < L the data is left in natural storage order
@@ -279,22 +301,8 @@ __device__ __forceinline__ void dif_body(const DevView &in, size_t entries, cons
     constexpr int RP = dif_last_rp<L, SEND>();
     constexpr int NG = C::R >> RP;
     if (!active) return;
-    uint32_t *o = out + e * C::N;
     if constexpr (SEND == L) {
-#pragma unroll
-        for (int u = 0; u < NG; ++u) {
-            const int g = tp + u * C::TP;
-            if constexpr (RP >= 2) {
-#pragma unroll
-                for (int q = 0; q < (1 << RP); q += 4)
-                    *reinterpret_cast<uint4 *>(o + (g << RP) + q) =
-                        make_uint4(x[u * (1 << RP) + q], x[u * (1 << RP) + q + 1], x[u * (1 << RP) + q + 2],
-                                   x[u * (1 << RP) + q + 3]);
-            } else {
-#pragma unroll
-                for (int q = 0; q < (1 << RP); ++q) o[(g << RP) + q] = x[u * (1 << RP) + q];
-            }
-        }
+        dif_store<L>(x, tp, out + e * C::N);
     } else {  // block-major: [block][entry][2^(L-SEND) words]
 #pragma unroll
         for (int u = 0; u < NG; ++u)

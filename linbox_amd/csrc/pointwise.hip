@@ -30,7 +30,9 @@ namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-template <int TI, int TJ>
+// DEEP > 0 issues the loads of that many inner steps together (small tiles with
+// few waves per CU wait for every load otherwise).
+template <int TI, int TJ, int DEEP = 0>
 __device__ __forceinline__ void pw_plain_body(const uint32_t *__restrict__ A, const uint32_t *__restrict__ B,
                                               uint32_t *__restrict__ C, int m, int k, int n, size_t npts,
                                               uint32_t p, const PlainConst &pc, size_t t, int i0, int j0)
@@ -44,7 +46,7 @@ __device__ __forceinline__ void pw_plain_body(const uint32_t *__restrict__ A, co
         for (int jj = 0; jj < TJ; ++jj) acc[ii][jj] = 0;
     for (int q0 = 0; q0 < k; q0 += (int)pc.fold) {
         const int q1 = min(k, q0 + (int)pc.fold);
-        for (int q = q0; q < q1; ++q) {
+        const auto step = [&](int q) {
             uint32_t a[TI], b[TJ];
 #pragma unroll
             for (int ii = 0; ii < TI; ++ii)
@@ -56,6 +58,12 @@ __device__ __forceinline__ void pw_plain_body(const uint32_t *__restrict__ A, co
             for (int ii = 0; ii < TI; ++ii)
 #pragma unroll
                 for (int jj = 0; jj < TJ; ++jj) acc[ii][jj] += (uint64_t)a[ii] * b[jj];
+        };
+        if constexpr (DEEP > 0) {
+#pragma unroll DEEP
+            for (int q = q0; q < q1; ++q) step(q);
+        } else {
+            for (int q = q0; q < q1; ++q) step(q);
         }
 #pragma unroll
         for (int ii = 0; ii < TI; ++ii)
@@ -72,15 +80,27 @@ __device__ __forceinline__ void pw_plain_body(const uint32_t *__restrict__ A, co
         }
 }
 
-template <int TI, int TJ>
+// Primes of one launch, in the kernel arguments.
+struct PlainPrimes {
+    uint32_t p[kMultiPrimes];
+    PlainConst pc[kMultiPrimes];
+};
+
+// One output tile at one point per lane; item = tile * npts + t, so a wave's
+// lanes take consecutive points and transforms shorter than a wave share it.
+template <int T>
 __global__ void __launch_bounds__(256) pw_plain_kernel(const uint32_t *__restrict__ A, const uint32_t *__restrict__ B,
                                                        uint32_t *__restrict__ C, int m, int k, int n, size_t npts,
-                                                       uint32_t p, PlainConst pc)
+                                                       unsigned log_npts, size_t items, PlainPrimes primes)
 {
-    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (t >= npts) return;
-    const int tiles_j = (n + TJ - 1) / TJ;
-    pw_plain_body<TI, TJ>(A, B, C, m, k, n, npts, p, pc, t, (blockIdx.y / tiles_j) * TI, (blockIdx.y % tiles_j) * TJ);
+    const size_t item = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (item >= items) return;
+    const unsigned i = blockIdx.y;  // prime
+    const int tiles_j = (n + T - 1) / T;
+    const size_t t = item & (npts - 1);
+    const int tile = (int)(item >> log_npts);
+    pw_plain_body<T, T, T == 2 ? 8 : (T == 4 ? 2 : 0)>(A + (size_t)i * m * k * npts, B + (size_t)i * k * n * npts, C + (size_t)i * m * n * npts, m, k,
+                        n, npts, primes.p[i], primes.pc[i], t, (tile / tiles_j) * T, (tile % tiles_j) * T);
 }
 
 // Persistent work-queue form over the items of a batch: each workgroup takes
@@ -679,16 +699,38 @@ hipError_t launch_zero_counters(uint32_t *counters, int n, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_pointwise_plain(const uint32_t *A, const uint32_t *B, uint32_t *C, size_t m, size_t k, size_t n,
-                                  size_t npts, uint32_t p, uint32_t scale, hipStream_t s)
+template <int T>
+static hipError_t plain_launch(const uint32_t *A, const uint32_t *B, uint32_t *C, size_t m, size_t k, size_t n,
+                               size_t npts, unsigned r, const PlainPrimes &primes, hipStream_t s)
 {
-    constexpr int TI = 8, TJ = 8;
-    const PlainConst pc = plain_const(p, scale);
-    const size_t tiles = ((m + TI - 1) / TI) * ((n + TJ - 1) / TJ);
-    if (tiles > 65535) return hipErrorInvalidValue;
-    dim3 grid((unsigned)((npts + 255) / 256), (unsigned)tiles);
-    hipLaunchKernelGGL((pw_plain_kernel<TI, TJ>), grid, dim3(256), 0, s, A, B, C, (int)m, (int)k, (int)n, npts, p, pc);
+    const size_t tiles = ((m + T - 1) / T) * ((n + T - 1) / T), items = tiles * npts;
+    // groups of one wave spread a few waves over more CUs
+    const unsigned block = items * r < (size_t)device_cus() * 512 ? 64 : 256;
+    const size_t blocks = (items + block - 1) / block;
+    if (tiles > 0x7fffffff || blocks > 0x7fffffff) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(pw_plain_kernel<T>, dim3((unsigned)blocks, r), dim3(block), 0, s, A, B, C, (int)m, (int)k, (int)n,
+                       npts, (unsigned)__builtin_ctzll(npts), items, primes);
     return hipGetLastError();
+}
+
+hipError_t launch_pointwise_plain(const uint32_t *A, const uint32_t *B, uint32_t *C, size_t m, size_t k, size_t n,
+                                  size_t npts, unsigned r, const uint32_t *p, const PlainConst *pc, hipStream_t s)
+{
+    if (r == 0 || r > (unsigned)kMultiPrimes || (npts & (npts - 1))) return hipErrorInvalidValue;
+    PlainPrimes primes;
+    for (unsigned i = 0; i < (unsigned)kMultiPrimes; ++i) {
+        primes.p[i] = i < r ? p[i] : 0;
+        primes.pc[i] = i < r ? pc[i] : PlainConst{};
+    }
+    // the widest tile that still gives every CU eight waves: a wide tile re-reads
+    // less, a narrow one fills the chip.  Whole products, us, with the 8x8 / 4x4 /
+    // 2x2 tile: 10x20x30 at 2^12 points 53 / 43 / 46; 32^3 at 2^11 66 / 51 / 57, at
+    // 2^13 117 / 121 / 174; 48^3 at 2^10 77 / 61 / 73; 16^3 at 2^8 32 / 22 / 22.
+    const size_t full = 8 * (size_t)device_cus();
+    const auto waves = [&](size_t T) { return ((m + T - 1) / T) * ((n + T - 1) / T) * npts / 64 * r; };
+    if (waves(8) >= full) return plain_launch<8>(A, B, C, m, k, n, npts, r, primes, s);
+    if (waves(4) >= full) return plain_launch<4>(A, B, C, m, k, n, npts, r, primes, s);
+    return plain_launch<2>(A, B, C, m, k, n, npts, r, primes, s);
 }
 
 size_t limb_block_bytes(size_t rows, size_t kdim) { return rpad_of(rows) * kpad_of(kdim) * 4; }

@@ -226,3 +226,22 @@ def test_midproduct_pm_basis_level(ctx):
     st, row = orc.mul_fft_prime(p, 1, m, n, a0, ord1 + 1, ser, ord1 + ord2)
     assert st == 0
     assert np.array_equal(got[:n], row.reshape(n, -1)[:, ord1:ord1 + ord2])
+
+
+@pytest.mark.parametrize("small_left", [True, False])
+@pytest.mark.parametrize("layouts", [("polfirst",) * 3, ("matfirst", "matrowfirst", "matfirst")])
+@pytest.mark.parametrize("p", [998244353, 1000000007])
+def test_midproduct_reversed_load(ctx, p, layouts, small_left):
+    """The plain form reads the small operand reversed in its transform: small
+    operands of exactly hdeg coefficients, fewer, and one; hdeg over and under
+    half the transform; one prime and several."""
+    m, k, n = 3, 5, 4
+    for (ss, sl, sc, n0) in [(9, 17, 9, 0), (4, 17, 9, 0), (1, 6, 6, 3), (16, 31, 16, 0), (33, 70, 40, 40)]:
+        rng = np.random.default_rng(ss + sl)
+        sa, sb = (ss, sl) if small_left else (sl, ss)
+        a, b = rand(rng, p, m * k * sa), rand(rng, p, k * n * sb)
+        n1 = 2 * n0 - 1 if n0 else 0
+        say("midproduct reversed load", p, layouts, small_left, ss, sl, sc, n0)
+        ref = correlation(p, m, k, n, a, sa, b, sb, sc, small_left, n0, n1)
+        got = gpu_mid(ctx, p, m, k, n, a, sa, b, sb, sc, small_left, n0, n1, lbx.METHOD_PLAIN_U64, layouts)
+        assert np.array_equal(np.asarray(ref, dtype=np.uint64).reshape(-1), got)

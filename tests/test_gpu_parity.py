@@ -599,3 +599,20 @@ def test_mul_layouts_large(ctx, monkeypatch, p, m, k, n, sa, sb, layouts):
         got = C.to_polfirst()
         assert np.array_equal(got[:, 3:3 + sa + sb - 1], ref)
         assert not got[:, :3].any() and not got[:, 3 + sa + sb - 1:].any()  # the rest of the storage is kept
+
+
+@pytest.mark.parametrize("m,k,n,sa,sb", [
+    (1, 1, 1, 1, 2), (2, 3, 1, 2, 1), (9, 1, 17, 3, 2), (17, 70, 3, 5, 9),  # transforms shorter than a wave
+    (8, 8, 8, 16, 17), (33, 9, 40, 31, 33), (5, 130, 6, 64, 65),  # tile remainders, one operand over half the length
+    (24, 16, 24, 1025, 1000), (65, 15, 66, 300, 213), (100, 20, 90, 2000, 2097)])  # 2x2, 4x4 and 8x8 tiles
+@pytest.mark.parametrize("p", [2013265921, 268435399])
+def test_plain_whole_transforms(ctx, p, m, k, n, sa, sb):
+    """The three-launch plain product, of one prime and of three."""
+    rng = np.random.default_rng(m * k * n + sa)
+    a, b = rand(rng, p, m * k * sa).reshape(m * k, sa), rand(rng, p, k * n * sb).reshape(k * n, sb)
+    A, B = PolynomialMatrix.from_polfirst(a, m, k), PolynomialMatrix.from_polfirst(b, k, n)
+    C = PolynomialMatrix(m, n, sa + sb - 1)
+    say("plain whole transforms", p, m, k, n, sa, sb)
+    PolynomialMatrixMulDomain(p, ctx, method=lbx.METHOD_PLAIN_U64).mul(C, A, B)
+    xs = [int(x) for x in rng.integers(0, p, 2)]
+    assert check_by_evaluation(a, b, C.to_polfirst(), p, m, k, n, sa, sb, sa + sb - 1, xs)
