@@ -744,6 +744,7 @@ lbx_status lbx_destroy(lbx_ctx *ctx)
             if (ctx->last_done) (void)hipEventDestroy(ctx->last_done);
             if (ctx->aux) (void)hipStreamDestroy(ctx->aux);
             mp_release(ctx);
+            if (ctx->zz_bits) (void)hipHostFree(ctx->zz_bits);
             batch_release(ctx);
             stager_release(ctx);
         }

@@ -46,6 +46,7 @@ struct lbx_ctx {
     // an event recorded at its end (see StreamOrder)
     hipStream_t last_stream = nullptr;
     hipEvent_t last_done = nullptr;
+    unsigned *zz_bits = nullptr;  // pinned: partial maxima of an integer product's bit sizes (mp.hip)
     lbx::HostStager *stager = nullptr;  // created by the first large host copy
     int profiling = 0;  // 0 off, 1 stages, 2 stages and kernels
     bool check = false;           // check every whole product at a random point (lbx_set_check)

@@ -12,17 +12,19 @@
 // p_i < 2^31 with 2^(lpts+1) | p_i - 1, chosen in the deterministic order of
 // RandomFFTPrime::generatePrimes (random-fftprime.h:107-133) until their
 // product exceeds the bound, then recombined on the device:
-//   1. residue kernel: every nlimbs-word coefficient -> its residue mod each p_i
-//      (Horner over the 32-bit limbs with Shoup products);
-//   2. one single-prime NTT product per p_i (the same kernels as lbx_polymat_mul_u32);
-//   3. CRT kernel: Garner's mixed-radix digits v_i of each coefficient, then
-//      X mod P = sum_i v_i (prod_{j<i} p_j mod P) in 32-bit limbs, reduced by
-//      shift-and-subtract, written as nlimbs words.
+//   1. residue kernel: every nlimbs-word coefficient of both operands -> its
+//      residue mod each p_i (signed digits times the powers of 2^32);
+//   2. the products mod every p_i: three launches for all primes where the
+//      plain pointwise form serves (multi.hip), one product a prime otherwise;
+//   3. CRT kernel: X mod P = sum_i y_i (M/p_i mod P) - q (M mod P) with the
+//      quotient q from a fixed-point sum, reduced by two quotient digits, or
+//      from Garner's mixed-radix digits beyond 32 primes or 16 words.
 // The reference picks ~23-bit primes for fgemm on doubles (:162-164); the
 // primes here are 31-bit because every step is 32-bit integer arithmetic.
 // Products are unique, so the output is identical.
 #include <algorithm>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -39,7 +41,9 @@ struct MpPlan {
     unsigned lpts = 0;
     int nlimbs = 0;
     bool reduce = false;          // few-primes plans: some prime is below the modulus
-    uint32_t *d_const = nullptr;  // device constant block, layout described at MpLayout / FpLayout
+    uint32_t *d_const = nullptr;  // device constant block, layout described at MpLayout / FpLayout / ZzLayout
+    size_t res_off = 0;           // word offset of the residue constants (ResidueBlock)
+    size_t crt_off = 0;           // word offset of the direct recombination constants (CrtBlock), 0: none
 };
 
 namespace {
@@ -192,12 +196,11 @@ bool generate_primes(uint64_t pbound, const Limbs &prodbound, unsigned kmin, std
 //   [2r..3r)       2^32 mod p_i
 //   [3r..4r)       Shoup constant of 2^32 mod p_i
 //   [4r..4r+2r^2)  Garner inverses (p_j mod p_i)^-1 and their Shoup constants, i*r+j
-//   then r*nlimbs  prod_{j<i} p_j mod P, then nlimbs words of P;
-//   for the register kernels (nq = their word count NLM, else 0): off and s,
-//   Q = P 2^(32 off + s) in nq words, and r*nq words of
-//   (prod_{j<i} p_j mod P) 2^(32 off + s) (mp_div.h).
+//   then r*nlimbs  prod_{j<i} p_j mod P, then nlimbs words of P
+// (the mixed-radix kernel's), followed by the residue constants
+// (ResidueBlock) and, for the direct kernels, a CrtBlock.
 struct MpLayout {
-    int r, nl, nq = 0;
+    int r, nl;
     __host__ __device__ int primes() const { return 0; }
     __host__ __device__ int onep() const { return r; }
     __host__ __device__ int r32() const { return 2 * r; }
@@ -205,28 +208,8 @@ struct MpLayout {
     __host__ __device__ int inv() const { return 4 * r; }
     __host__ __device__ int mi() const { return 4 * r + 2 * r * r; }
     __host__ __device__ int P() const { return mi() + r * nl; }
-    __host__ __device__ int sh() const { return P() + nl; }
-    __host__ __device__ int Q() const { return sh() + 2; }
-    __host__ __device__ int mq() const { return Q() + nq; }
-    __host__ __device__ int words() const { return mq() + r * nq; }
+    __host__ __device__ int words() const { return P() + nl; }
 };
-
-// Register widths (RM primes, NLM words) of the CRT kernel mp_product
-// launches for r primes and an nl-word modulus, {0, 0} for the general
-// kernel; a plan's constants are laid out for that width (nq = NLM).  Narrow
-// moduli get narrow kernels: a word-size P (3 primes) takes 2-word
-// arithmetic and remainders instead of 8-word ones.
-struct CrtWidth {
-    int rm, nlm;
-};
-inline CrtWidth crt_width(int r, int nl)
-{
-    if (r <= 4 && nl <= 2) return {4, 2};
-    if (r <= 8 && nl <= 4) return {8, 4};
-    if (r <= 16 && nl <= 8) return {16, 8};
-    if (r <= 32 && nl <= 16) return {32, 16};
-    return {0, 0};
-}
 
 // Word index of element idx (entry idx / size, coefficient idx % size) of a
 // view.  A polfirst view without window (stride = size, no shift) maps idx to
@@ -238,32 +221,141 @@ __device__ __forceinline__ size_t elem_index(const DevView &v, size_t idx, size_
     return view_index(v, e, t);
 }
 
-// Residues of nlimbs-word coefficients modulo every prime:
-// out[i][e*size + t] for e < entries, t < size.
-// The limb count is bounded at compile time (NLM >= nl), so the limbs stay in
-// registers and the Horner steps unroll.
-template <int NLM>
-__global__ void __launch_bounds__(256) mp_residue_kernel(DevView in, int nl, size_t entries, size_t size,
-                                                         const uint32_t *__restrict__ K, int r,
-                                                         uint32_t *__restrict__ out)
+// ---- residues --------------------------------------------------------------
+// Residues of nl-word coefficients x (unsigned, or two's complement) modulo
+// every prime, out[i][e*size + t].  x = sum_l d_l 2^(32 l), l <= nl, with signed
+// digits |d_l| <= 2^31 (a carry chain once per coefficient); with the constants
+// 2^(32 l) mod p centred to |c| < p/2 < 2^30 each digit is one v_mad_i64_i32 of
+// magnitude at most 2^61, folded every third digit (plain_s_fold: after a fold
+// |acc| < 2^60 + 2^34, and three more products stay below 2^63) and reduced
+// once.  Constants of prime i, kTail + nl + 1 words: the PlainSConst of scale 1
+// (c0p, c1, c1p, f60, off), p, then c_0 .. c_nl.
+//
+// Bound by the multiply-adds (nl + 1 and some ten more products a prime for
+// each coefficient), with r words written for nl read.  The words of a group's
+// coefficients are staged through LDS where they are contiguous, so the loads
+// are whole lines whatever nl is.  Both operands in one launch: 2^20
+// coefficients of 6 words each, 14 primes: 91 us in two launches of a Horner
+// scheme with two Shoup products a word, 38 us here.
+struct ResidueBlock {
+    static constexpr int kTail = 7;
+    int nl;
+    __host__ __device__ int stride() const { return kTail + nl + 1; }
+};
+
+void residue_constants(std::vector<uint32_t> &K, const std::vector<uint32_t> &primes, int nl)
 {
-    const size_t total = entries * size;
-    const MpLayout lay{r, nl};
-    for (size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (size_t)gridDim.x * 256) {
-        const uint32_t *src = in.base + elem_index(in, idx, size) * nl;
-        uint32_t limb[NLM];
-#pragma unroll
-        for (int l = 0; l < NLM; ++l) limb[l] = l < nl ? src[l] : 0u;
-        for (int i = 0; i < r; ++i) {
-            const uint32_t p = K[lay.primes() + i], onep = K[lay.onep() + i];
-            const uint32_t c = K[lay.r32() + i], cp = K[lay.r32p() + i];
-            uint32_t v = 0;
-#pragma unroll
-            for (int l = NLM - 1; l >= 0; --l)
-                if (l < nl) v = add_mod(shoup_mul(v, c, cp, p), shoup_mul(limb[l], 1u, onep, p), p);
-            out[(size_t)i * total + idx] = v;
+    for (const uint32_t p : primes) {
+        const PlainSConst pc = plain_s_const(p, 1);
+        const uint32_t head[ResidueBlock::kTail] = {pc.c0p, pc.c1, pc.c1p, pc.f60, (uint32_t)pc.off,
+                                                    (uint32_t)(pc.off >> 32), p};
+        K.insert(K.end(), head, head + ResidueBlock::kTail);
+        const uint32_t r32 = (uint32_t)(((uint64_t)1 << 32) % p);
+        uint32_t w = 1 % p;
+        for (int l = 0; l <= nl; ++l) {
+            K.push_back((uint32_t)centre(w, p));
+            w = (uint32_t)((uint64_t)w * r32 % p);
         }
     }
+}
+
+struct ResidueArgs {
+    DevView in[2];
+    size_t total[2], size[2];
+    uint32_t *out[2];
+    unsigned blocks0;  // groups of the first operand
+};
+
+constexpr int kResidueStage = 8;  // widest coefficient staged through LDS
+
+// NL > 0: nl = NL words; NL = 0: any nl <= kMaxLimbs.
+template <int NL, bool SIGNED>
+__global__ void __launch_bounds__(256) residue_kernel(ResidueArgs A, int any_nl, int r, const uint32_t *__restrict__ K)
+{
+    constexpr int NW = NL ? NL : kMaxLimbs;
+    __shared__ uint32_t stage[NL ? 256 * NL : 1];
+    const int nl = NL ? NL : any_nl;
+    const int op = blockIdx.x < A.blocks0 ? 0 : 1;
+    const DevView &in = A.in[op];
+    const size_t total = A.total[op], size = A.size[op];
+    const size_t idx0 = (size_t)(blockIdx.x - (op ? A.blocks0 : 0)) * 256, idx = idx0 + threadIdx.x;
+    const bool contiguous = in.layout == 0 && in.stor == size && in.shift == 0;
+    uint32_t w[NW];
+    if (NL && contiguous) {
+        const uint32_t *src = in.base + idx0 * NL;
+        const unsigned words = (unsigned)(total - idx0 < 256 ? total - idx0 : 256) * NL;
+        uint32_t v[NL ? NL : 1];
+#pragma unroll
+        for (int j = 0; j < (NL ? NL : 1); ++j) v[j] = src[min(j * 256 + threadIdx.x, words - 1)];  // issued together
+#pragma unroll
+        for (int j = 0; j < (NL ? NL : 1); ++j) stage[j * 256 + threadIdx.x] = v[j];
+        __syncthreads();
+        if (idx >= total) return;
+#pragma unroll
+        for (int l = 0; l < NW; ++l) w[l] = stage[threadIdx.x * NW + l];
+    } else {
+        if (idx >= total) return;
+        const uint32_t *src = in.base + elem_index(in, idx, size) * nl;
+#pragma unroll
+        for (int l = 0; l < NW; ++l) w[l] = (NL || l < nl) ? src[l] : 0u;
+    }
+    // signed digits: w_l + carry as a signed word, carry 1 when that subtracts 2^32
+    uint32_t carry = 0, top = 0;
+#pragma unroll
+    for (int l = 0; l < NW; ++l) {
+        if (NL || l < nl) {
+            if (SIGNED) top = w[l];
+            w[l] += carry;
+            carry = (w[l] >> 31) | (w[l] < carry ? 1u : 0u);
+        }
+    }
+    const int32_t last = (int32_t)carry - (SIGNED ? (int32_t)(top >> 31) : 0);  // digit nl, in {-1, 0, 1}
+    uint32_t *__restrict__ out = A.out[op] + idx;
+    for (int i = 0; i < r; ++i, K += ResidueBlock{nl}.stride()) {
+        PlainSConst pc;
+        pc.c0 = 1;
+        pc.c0p = K[0], pc.c1 = K[1], pc.c1p = K[2], pc.f60 = K[3];
+        pc.off = ((uint64_t)K[5] << 32) | K[4];
+        const uint32_t *c = K + ResidueBlock::kTail;
+        int64_t acc = (int64_t)last * (int32_t)c[nl];
+#pragma unroll
+        for (int l = 0; l < NW; ++l) {
+            if (NL || l < nl) {
+                if (l % 3 == 2) acc = plain_s_fold(acc, pc);
+                acc += (int64_t)(int32_t)w[l] * (int32_t)c[l];
+            }
+        }
+        out[(size_t)i * total] = plain_s_finish(acc, K[6], pc);
+    }
+}
+
+// Residues of a (ea x a.size coefficients) into ra and of b into rb.
+template <bool SIGNED>
+hipError_t launch_residues(const DevView &a, size_t ea, uint32_t *ra, const DevView &b, size_t eb, uint32_t *rb, int nl,
+                           int r, const uint32_t *K, hipStream_t s)
+{
+    ResidueArgs A;
+    A.in[0] = a, A.in[1] = b;
+    A.size[0] = a.size, A.size[1] = b.size;
+    A.total[0] = ea * a.size, A.total[1] = eb * b.size;
+    A.out[0] = ra, A.out[1] = rb;
+    const size_t b0 = (A.total[0] + 255) / 256, b1 = (A.total[1] + 255) / 256;
+    if (b0 + b1 > 0x7fffffff) return hipErrorInvalidValue;
+    A.blocks0 = (unsigned)b0;
+    auto k = residue_kernel<0, SIGNED>;
+    switch (nl) {
+    case 1: k = residue_kernel<1, SIGNED>; break;
+    case 2: k = residue_kernel<2, SIGNED>; break;
+    case 3: k = residue_kernel<3, SIGNED>; break;
+    case 4: k = residue_kernel<4, SIGNED>; break;
+    case 5: k = residue_kernel<5, SIGNED>; break;
+    case 6: k = residue_kernel<6, SIGNED>; break;
+    case 7: k = residue_kernel<7, SIGNED>; break;
+    case 8: k = residue_kernel<8, SIGNED>; break;
+    }
+    static_assert(kResidueStage == 8, "one kernel per staged width");
+    hipLaunchKernelGGL(k, dim3((unsigned)(b0 + b1)), dim3(256), 0, s, A, nl, r, K);
+    return hipGetLastError();
 }
 
 // Garner recombination of r residues and reduction mod P.
@@ -332,66 +424,166 @@ __global__ void __launch_bounds__(128) mp_crt_kernel(const uint32_t *__restrict_
     }
 }
 
-// The same recombination with the prime count and the limb count bounded at
-// compile time (RM, NLM): every array index is then a constant, so v and the
-// accumulator stay in registers (the general kernel above indexes them at run
-// time and keeps them in scratch memory).  The accumulator is formed against
-// P moved to the top of NLM words (Q = P 2^(32 off + s), normalized), reduced
-// by two quotient digits of Knuth's division (mp_div.h) instead of 41 steps of
-// shift-and-subtract, and shifted back into nl words.
-template <int RM, int NLM>
-__global__ void __launch_bounds__(128) mp_crt_small_kernel(const uint32_t *__restrict__ res, size_t entries,
-                                                           size_t size, const uint32_t *__restrict__ K, int r, int nl,
-                                                           DevView out)
+// ---- direct recombination ---------------------------------------------------
+// X = sum_i y_i (M/p_i) - q M with y_i = r_i (M/p_i)^-1 mod p_i and q =
+// floor(sum_i y_i / p_i) (or the nearest integer, for the symmetric range), M
+// the product of the primes: r products a coefficient where the mixed-radix
+// digits above take r (r-1) / 2 modular ones.  q comes from the fixed-point sum
+// S = sum_i y_i floor(2^56 / p_i), at most r 2^31 <= 2^36 below 2^56 sum_i y_i/p_i
+// for r <= 32 primes above 2^24 (so that the reciprocals are words).
+//  * Modulus P: M > 2 P^2 k min(sa,sb) > 2 X, so sum_i y_i/p_i = q + X/M has its
+//    fraction in [0, 1/2): adding 2^37 to S before the shift gives q exactly.
+//  * Integers: |X| < bound/2, and the direct form is taken when M > bound (1 +
+//    2^-16), so |X/M| < 1/2 - 2^-18: adding 2^55 rounds to the nearest q exactly.
+// Other plans (more primes, smaller ones, the rare tight M) keep the kernels
+// on mixed-radix digits.  Every word of the sum has a compile-time index: NW
+// words, the constants padded to them.  With MOD the sum is taken against
+// Q = P 2^(32 off + s), P moved to the top of NW words (sum_i y_i (M_i mod P) + q
+// ((-M) mod P) < (32 (2^31 - 1) + 31) P < 2^36 P), reduced by two quotient
+// digits of Knuth's division (mp_div.h) and shifted back; without, modulo
+// 2^(32 NW).  The group's words leave through LDS where they are contiguous.
+//
+// Constants: per prime p, (M/p)^-1 mod p with its Shoup constant, floor(2^56 /
+// p), NW words of M/p; then NW words of -M; then (MOD) off, s and NW words of Q.
+// Bound by the multiply-adds: 2047 x 1024 coefficients, 14 primes, 6 words: 140 us
+// on mixed-radix digits, 57 us here.
+struct CrtBlock {
+    static constexpr int kHead = 4;
+    int r, nw;
+    __host__ __device__ int prime(int i) const { return i * (kHead + nw); }
+    __host__ __device__ int neg() const { return r * (kHead + nw); }
+    __host__ __device__ int sh() const { return neg() + nw; }
+    __host__ __device__ int Q() const { return sh() + 2; }
+};
+constexpr int kCrtMaxPrimes = 32;
+constexpr uint32_t kCrtMinPrime = 1u << 24;
+
+template <int NW, bool MOD>
+__global__ void __launch_bounds__(128) crt_direct_kernel(const uint32_t *__restrict__ res, size_t entries, size_t size,
+                                                         const uint32_t *__restrict__ K, int r, int ow, DevView out)
 {
+    constexpr int NA = MOD ? NW + 2 : NW;
+    __shared__ uint32_t stage[128 * NW];
     const size_t total = entries * size;
-    const MpLayout lay{r, nl, NLM};
-    const int off = (int)K[lay.sh()], s = (int)K[lay.sh() + 1];
-    uint32_t q[NLM];
+    const CrtBlock lay{r, NW};
+    const size_t idx0 = (size_t)blockIdx.x * 128, idx = idx0 + threadIdx.x;
+    const bool live = idx < total;
+    const size_t at = live ? idx : total - 1;
+    uint32_t acc[NA];
 #pragma unroll
-    for (int l = 0; l < NLM; ++l) q[l] = K[lay.Q() + l];
-    const uint32_t qinv = div21_inverse(q[NLM - 1]);  // Q is normalized: its top word has its top bit set
-    for (size_t idx = (size_t)blockIdx.x * 128 + threadIdx.x; idx < total; idx += (size_t)gridDim.x * 128) {
-        uint32_t v[RM], rv[RM];
-        uint32_t acc[NLM + 2];
+    for (int l = 0; l < NA; ++l) acc[l] = 0;
+    uint64_t S = MOD ? (uint64_t)1 << 37 : (uint64_t)1 << 55;
+    // acc += t * (NW words at w)
+    const auto add = [&](uint32_t t, const uint32_t *w) {
+        uint64_t carry = 0;
 #pragma unroll
-        for (int l = 0; l < NLM + 2; ++l) acc[l] = 0;
+        for (int l = 0; l < NW; ++l) {
+            const uint64_t sum = (uint64_t)w[l] * t + acc[l] + carry;
+            acc[l] = (uint32_t)sum;
+            carry = sum >> 32;
+        }
+        if (MOD) {
+            const uint64_t hi = (uint64_t)acc[NA - 2] + carry;
+            acc[NA - 2] = (uint32_t)hi;
+            acc[NA - 1] += (uint32_t)(hi >> 32);
+        }
+    };
+    constexpr int kAhead = 8;  // residues loaded together
+    for (int i0 = 0; i0 < r; i0 += kAhead) {
+        uint32_t rv[kAhead];
 #pragma unroll
-        for (int i = 0; i < RM; ++i) rv[i] = i < r ? res[(size_t)i * total + idx] : 0u;  // loads issued together
+        for (int j = 0; j < kAhead; ++j) rv[j] = i0 + j < r ? res[(size_t)(i0 + j) * total + at] : 0u;
 #pragma unroll
-        for (int i = 0; i < RM; ++i) {
-            if (i < r) {
-                const uint32_t p = K[lay.primes() + i], onep = K[lay.onep() + i];
-                uint32_t t = rv[i];
-#pragma unroll
-                for (int j = 0; j < i; ++j) {
-                    const uint32_t vj = shoup_mul(v[j], 1u, onep, p);
-                    t = shoup_mul(sub_mod(t, vj, p), K[lay.inv() + 2 * (i * r + j)], K[lay.inv() + 2 * (i * r + j) + 1],
-                                  p);
-                }
-                v[i] = t;
-                // acc += v_i * (prod_{j<i} p_j mod P) 2^(32 off + s)
-                const uint32_t *mi = K + lay.mq() + i * NLM;
-                uint64_t carry = 0;
-#pragma unroll
-                for (int l = 0; l < NLM; ++l) {
-                    const uint64_t sum = (uint64_t)mi[l] * t + acc[l] + carry;
-                    acc[l] = (uint32_t)sum;
-                    carry = sum >> 32;
-                }
-                const uint64_t top = (uint64_t)acc[NLM] + carry;
-                acc[NLM] = (uint32_t)top;
-                acc[NLM + 1] += (uint32_t)(top >> 32);
+        for (int j = 0; j < kAhead; ++j) {
+            if (i0 + j < r) {
+                const uint32_t *c = K + lay.prime(i0 + j);
+                const uint32_t y = shoup_mul(rv[j], c[1], c[2], c[0]);
+                S += (uint64_t)y * c[3];
+                add(y, c + CrtBlock::kHead);
             }
         }
-        // acc < r 2^31 Q <= 2^36 Q: acc mod Q = (X mod P) 2^(32 off + s) in acc[0..NLM)
-        knuth_rem2<NLM>(acc, q, qinv);
-        uint32_t *dst = out.base + elem_index(out, idx, size) * nl;
-#pragma unroll
-        for (int l = 0; l < NLM; ++l)
-            if (l >= off) dst[l - off] = s ? (acc[l] >> s) | (acc[l + 1] << (32 - s)) : acc[l];
-        for (int l = NLM - off; l < nl; ++l) dst[l] = 0;  // words of P's leading zero limbs
     }
+    add((uint32_t)(S >> 56), K + lay.neg());
+    if constexpr (MOD) {
+        const int off = (int)K[lay.sh()], sh = (int)K[lay.sh() + 1];
+        uint32_t q[NW];
+#pragma unroll
+        for (int l = 0; l < NW; ++l) q[l] = K[lay.Q() + l];
+        knuth_rem2<NW>(acc, q, div21_inverse(q[NW - 1]));  // Q is normalized: its top word has its top bit set
+        // words off.. of acc >> sh; the words of P's leading zero limbs are zero
+#pragma unroll
+        for (int l = 0; l < NW; ++l)
+            if (l >= off && l - off < ow)
+                stage[threadIdx.x * ow + l - off] = sh ? (acc[l] >> sh) | (acc[l + 1] << (32 - sh)) : acc[l];
+        for (int l = NW - off; l < ow; ++l) stage[threadIdx.x * ow + l] = 0;
+    } else {
+#pragma unroll
+        for (int l = 0; l < NW; ++l)
+            if (l < ow) stage[threadIdx.x * ow + l] = acc[l];
+    }
+    if (out.layout == 0 && out.stor == size && out.shift == 0) {
+        __syncthreads();
+        uint32_t *dst = out.base + idx0 * ow;
+        const int words = (int)(total - idx0 < 128 ? total - idx0 : 128) * ow;
+        for (int w = threadIdx.x; w < words; w += 128) dst[w] = stage[w];
+    } else if (live) {
+        uint32_t *dst = out.base + elem_index(out, idx, size) * ow;
+        for (int l = 0; l < ow; ++l) dst[l] = stage[threadIdx.x * ow + l];
+    }
+}
+
+// Words of the direct kernel that serves r primes and ow-word results, 0 for none.
+int crt_words(const std::vector<uint32_t> &primes, int ow)
+{
+    if (primes.size() > (size_t)kCrtMaxPrimes || ow > 16) return 0;
+    for (const uint32_t p : primes)
+        if (p < kCrtMinPrime) return 0;
+    return ow <= 2 ? 2 : (ow <= 4 ? 4 : (ow <= 8 ? 8 : 16));
+}
+
+template <bool MOD>
+hipError_t launch_crt_direct(int nw, const uint32_t *res, size_t entries, size_t size, const uint32_t *K, int r, int ow,
+                             const DevView &out, hipStream_t s)
+{
+    const size_t grid = (entries * size + 127) / 128;
+    if (grid > 0x7fffffff) return hipErrorInvalidValue;
+    auto k = nw == 2 ? crt_direct_kernel<2, MOD>
+                     : (nw == 4 ? crt_direct_kernel<4, MOD>
+                                : (nw == 8 ? crt_direct_kernel<8, MOD> : crt_direct_kernel<16, MOD>));
+    hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(128), 0, s, res, entries, size, K, r, ow, out);
+    return hipGetLastError();
+}
+
+// Product of the primes, and of all but prime i (i >= 0).
+Limbs prime_product(const std::vector<uint32_t> &primes, int skip = -1)
+{
+    Limbs M{1};
+    for (size_t i = 0; i < primes.size(); ++i)
+        if ((int)i != skip) limbs_mul_small(M, primes[i]);
+    return M;
+}
+
+// Appends a CrtBlock: word(x, dst) writes the NW words of the value x (a
+// multiword integer) as the kernel's sum takes it.
+template <class F, class G>
+void crt_constants(std::vector<uint32_t> &K, const std::vector<uint32_t> &primes, int nw, F &&words, G &&neg_words)
+{
+    const CrtBlock lay{(int)primes.size(), nw};
+    const size_t base = K.size();
+    K.resize(base + lay.Q() + nw, 0);
+    for (size_t i = 0; i < primes.size(); ++i) {
+        const uint32_t p = primes[i];
+        uint32_t w = 1 % p;
+        for (size_t j = 0; j < primes.size(); ++j)
+            if (j != i) w = (uint32_t)((uint64_t)w * (primes[j] % p) % p);
+        uint32_t *c = &K[base + lay.prime((int)i)];
+        c[0] = p;
+        c[1] = invmod_h(w, p);
+        c[2] = shoup_pre(c[1], p);
+        c[3] = (uint32_t)(((uint64_t)1 << 56) / p);
+        words(prime_product(primes, (int)i), c + CrtBlock::kHead);
+    }
+    neg_words(prime_product(primes), &K[base + lay.neg()]);
 }
 
 // ---- few-primes route (three-primes.inl:67-191) ----------------------------
@@ -555,25 +747,8 @@ lbx_status get_plan(lbx_ctx *ctx, const uint32_t *Pw, int nl, size_t k, size_t m
     std::vector<uint32_t> primes;
     if (!generate_primes((uint64_t)1 << 31, bound, lpts, primes)) return LBX_ERR_NOT_ENOUGH_PRIMES;
     const int r = (int)primes.size();
-    // word count of the register kernel mp_product launches for (r, nl), 0 for the general one
-    const int nq = crt_width(r, nl).nlm;
-    const MpLayout lay{r, nl, nq};
+    const MpLayout lay{r, nl};
     std::vector<uint32_t> K((size_t)lay.words(), 0);
-    // P moved to the top of nq words with its top bit set: 2^(32 off + s)
-    const int np = (int)P.size(), off = nq - np, sbits = __builtin_clz(P.back());
-    auto place = [&](const Limbs &x, uint32_t *dst) {  // x < P: x 2^(32 off + s) in nq words
-        uint32_t prev = 0;
-        for (int l = 0; l < np; ++l) {
-            const uint32_t w = l < (int)x.size() ? x[l] : 0u;
-            dst[off + l] = sbits ? (w << sbits) | prev : w;
-            prev = sbits ? w >> (32 - sbits) : 0u;
-        }
-    };
-    if (nq) {
-        K[lay.sh()] = (uint32_t)off;
-        K[lay.sh() + 1] = (uint32_t)sbits;
-        place(P, &K[lay.Q()]);
-    }
     Limbs M{1};
     for (int i = 0; i < r; ++i) {
         const uint32_t p = primes[i];
@@ -589,7 +764,6 @@ lbx_status get_plan(lbx_ctx *ctx, const uint32_t *Pw, int nl, size_t k, size_t m
         }
         const Limbs mi = limbs_mod(M, P);
         for (int l = 0; l < nl; ++l) K[lay.mi() + i * nl + l] = l < (int)mi.size() ? mi[l] : 0;
-        if (nq) place(mi, &K[lay.mq() + i * nq]);
         limbs_mul_small(M, p);
         M = limbs_mod(M, P);
     }
@@ -598,6 +772,37 @@ lbx_status get_plan(lbx_ctx *ctx, const uint32_t *Pw, int nl, size_t k, size_t m
     plan->primes = primes;
     plan->lpts = lpts;
     plan->nlimbs = nl;
+    plan->res_off = K.size();
+    residue_constants(K, primes, nl);
+    if (const int nw = crt_words(primes, nl)) {
+        // P at the top of nw words with its top bit set: Q = P 2^(32 off + sh)
+        const int np = (int)P.size(), off = nw - np, sh = __builtin_clz(P.back());
+        const auto place = [&](const Limbs &x, uint32_t *dst) {  // x < P: x 2^(32 off + sh) in nw words
+            uint32_t prev = 0;
+            for (int l = 0; l < np; ++l) {
+                const uint32_t w = l < (int)x.size() ? x[l] : 0u;
+                dst[off + l] = sh ? (w << sh) | prev : w;
+                prev = sh ? w >> (32 - sh) : 0u;
+            }
+        };
+        plan->crt_off = K.size();
+        const CrtBlock cb{r, nw};
+        crt_constants(K, primes, nw, [&](const Limbs &x, uint32_t *dst) { place(limbs_mod(x, P), dst); },
+                      [&](const Limbs &x, uint32_t *dst) {  // (-M) mod P
+                          const Limbs mm = limbs_mod(x, P);
+                          Limbs d(np, 0);
+                          uint64_t borrow = 0;
+                          for (int l = 0; l < np; ++l) {
+                              const uint64_t t = (uint64_t)P[l] - (l < (int)mm.size() ? mm[l] : 0) - borrow;
+                              d[l] = (uint32_t)t;
+                              borrow = (t >> 32) & 1;
+                          }
+                          place(limbs_mod(d, P), dst);
+                      });
+        K[plan->crt_off + cb.sh()] = (uint32_t)off;
+        K[plan->crt_off + cb.sh() + 1] = (uint32_t)sh;
+        place(P, &K[plan->crt_off + cb.Q()]);
+    }
     hipError_t e = hipMalloc(&plan->d_const, K.size() * 4);
     if (e == hipSuccess) e = hipMemcpy(plan->d_const, K.data(), K.size() * 4, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
@@ -762,33 +967,16 @@ lbx_status mp_product(lbx_ctx *ctx, const uint32_t *Pw, int nl, const DevView &a
     LBX_TRY(ensure(ctx, "mp_ra", (size_t)r * m * k * sa * 4, &ra));
     LBX_TRY(ensure(ctx, "mp_rb", (size_t)r * k * n * sb * 4, &rb));
     LBX_TRY(ensure(ctx, "mp_rc", (size_t)r * m * n * sc * 4, &rc));
-    auto residues = nl <= 8 ? mp_residue_kernel<8> : mp_residue_kernel<kMaxLimbs>;
-    hipLaunchKernelGGL(residues, dim3(grid_of(m * k * sa, 256)), dim3(256), 0, s, a, nl, m * k, sa, plan->d_const, r,
-                       (uint32_t *)ra);
-    LBX_TRY_HIP(hipGetLastError());
-    hipLaunchKernelGGL(residues, dim3(grid_of(k * n * sb, 256)), dim3(256), 0, s, b, nl, k * n, sb, plan->d_const, r,
-                       (uint32_t *)rb);
-    LBX_TRY_HIP(hipGetLastError());
+    LBX_TRY_HIP(launch_residues<false>(a, m * k, (uint32_t *)ra, b, k * n, (uint32_t *)rb, nl, r,
+                                       plan->d_const + plan->res_off, s));
     const DevView va{(uint32_t *)ra, LBX_POLFIRST, m, k, sa, 0, sa}, vb{(uint32_t *)rb, LBX_POLFIRST, k, n, sb, 0, sb};
     LBX_TRY(prime_products(ctx, plan->primes, va, m * k * sa, vb, k * n * sb, (uint32_t *)rc, m, k, n, sc, lpts, method,
                            s, mid));
-    const dim3 grid(grid_of(m * n * sc, 128));
-    const int nlm = crt_width(r, nl).nlm;
-    if (nlm == 2)
-        hipLaunchKernelGGL((mp_crt_small_kernel<4, 2>), grid, dim3(128), 0, s, (const uint32_t *)rc, m * n, sc,
-                           plan->d_const, r, nl, c);
-    else if (nlm == 4)
-        hipLaunchKernelGGL((mp_crt_small_kernel<8, 4>), grid, dim3(128), 0, s, (const uint32_t *)rc, m * n, sc,
-                           plan->d_const, r, nl, c);
-    else if (nlm == 8)
-        hipLaunchKernelGGL((mp_crt_small_kernel<16, 8>), grid, dim3(128), 0, s, (const uint32_t *)rc, m * n, sc,
-                           plan->d_const, r, nl, c);
-    else if (nlm == 16)
-        hipLaunchKernelGGL((mp_crt_small_kernel<32, 16>), grid, dim3(128), 0, s, (const uint32_t *)rc, m * n, sc,
-                           plan->d_const, r, nl, c);
-    else
-        hipLaunchKernelGGL(mp_crt_kernel, grid, dim3(128), 0, s, (const uint32_t *)rc, m * n, sc, plan->d_const, r,
-                           nl, c);
+    if (plan->crt_off)
+        return from_hip(launch_crt_direct<true>(crt_words(plan->primes, nl), (const uint32_t *)rc, m * n, sc,
+                                                plan->d_const + plan->crt_off, r, nl, c, s));
+    hipLaunchKernelGGL(mp_crt_kernel, dim3(grid_of(m * n * sc, 128)), dim3(128), 0, s, (const uint32_t *)rc, m * n, sc,
+                       plan->d_const, r, nl, c);
     LBX_TRY_HIP(hipGetLastError());
     return LBX_OK;
 }
@@ -809,31 +997,41 @@ constexpr int kZzMaxPrimes = 96;
 
 namespace {
 
-// Constant block: primes, Shoup constants of 1, 2^32 mod p_i and its Shoup
-// constant, 2^(32 nl) mod p_i, Garner inverses (p_j mod p_i)^-1 with their
-// Shoup constants at 2(i r + j), then W_i = prod_{j<i} p_j mod 2^(32 cl) in cl
-// words each, then M mod 2^(32 cl).
+// Constant block: primes, Shoup constants of 1, Garner inverses (p_j mod
+// p_i)^-1 with their Shoup constants at 2(i r + j), then W_i = prod_{j<i} p_j mod
+// 2^(32 cl) in cl words each, then M mod 2^(32 cl) (the mixed-radix kernel's),
+// followed by the residue constants and, for the direct kernels, a CrtBlock.
 struct ZzLayout {
     int r, cl;
     __host__ __device__ int primes() const { return 0; }
     __host__ __device__ int onep() const { return r; }
-    __host__ __device__ int r32() const { return 2 * r; }
-    __host__ __device__ int r32p() const { return 3 * r; }
-    __host__ __device__ int top() const { return 4 * r; }
-    __host__ __device__ int inv() const { return 5 * r; }
-    __host__ __device__ int W() const { return 5 * r + 2 * r * r; }
+    __host__ __device__ int inv() const { return 2 * r; }
+    __host__ __device__ int W() const { return 2 * r + 2 * r * r; }
     __host__ __device__ int M() const { return W() + r * cl; }
     __host__ __device__ int words() const { return M() + cl; }
 };
 
 // Largest bit size of the absolute values of nl-word two's complement
-// coefficients (Givaro's bitsize, 0 for 0), max-accumulated into *out.
-__global__ void __launch_bounds__(256) zz_logmax_kernel(DevView in, int nl, size_t entries, size_t size,
+// coefficients (Givaro's bitsize, 0 for 0) of both operands: group g writes the
+// maximum of its share to out[g], in pinned host memory that the host reduces
+// after its wait (groups [0, gridDim.x/2) the first operand, the rest the
+// second).  The share of a group is a run of coefficients, so a wave reads
+// 64 nl contiguous words.  One launch and one wait for both operands: 2 x 404K
+// coefficients of two words took 75 us each with an atomic maximum per wave,
+// 6 us for both here.
+constexpr unsigned kLogmaxGroups = 256;  // groups an operand
+
+__global__ void __launch_bounds__(256) zz_logmax_kernel(DevView a, size_t ea, DevView b, size_t eb, int nl,
                                                         unsigned *__restrict__ out)
 {
-    const size_t total = entries * size;
+    __shared__ unsigned wave_max[4];
+    const unsigned half = gridDim.x / 2;
+    const bool second = blockIdx.x >= half;
+    const DevView &in = second ? b : a;
+    const size_t size = in.size, total = (second ? eb : ea) * size;
     unsigned best = 0;
-    for (size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (size_t)gridDim.x * 256) {
+    for (size_t idx = (size_t)(blockIdx.x - (second ? half : 0)) * 256 + threadIdx.x; idx < total;
+         idx += (size_t)half * 256) {
         const uint32_t *src = in.base + elem_index(in, idx, size) * nl;
         const bool neg = src[nl - 1] >> 31;
         // |x|: the words themselves, or their two's complement negation
@@ -854,34 +1052,11 @@ __global__ void __launch_bounds__(256) zz_logmax_kernel(DevView in, int nl, size
         const unsigned o = __shfl_xor(best, off);
         best = o > best ? o : best;
     }
-    if ((threadIdx.x & 63) == 0 && best) atomicMax(out, best);
-}
-
-// Residues mod every prime of nl-word two's complement coefficients: Horner over
-// the words as unsigned, minus 2^(32 nl) when the sign bit is set.
-template <int NLM>
-__global__ void __launch_bounds__(256) zz_residue_kernel(DevView in, int nl, size_t entries, size_t size,
-                                                         const uint32_t *__restrict__ K, int r,
-                                                         uint32_t *__restrict__ out)
-{
-    const size_t total = entries * size;
-    const ZzLayout lay{r, 0};
-    for (size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (size_t)gridDim.x * 256) {
-        const uint32_t *src = in.base + elem_index(in, idx, size) * nl;
-        uint32_t limb[NLM];
-#pragma unroll
-        for (int l = 0; l < NLM; ++l) limb[l] = l < nl ? src[l] : 0u;
-        const bool neg = src[nl - 1] >> 31;
-        for (int i = 0; i < r; ++i) {
-            const uint32_t p = K[lay.primes() + i], onep = K[lay.onep() + i];
-            const uint32_t c = K[lay.r32() + i], cp = K[lay.r32p() + i];
-            uint32_t v = 0;
-#pragma unroll
-            for (int l = NLM - 1; l >= 0; --l)
-                if (l < nl) v = add_mod(shoup_mul(v, c, cp, p), shoup_mul(limb[l], 1u, onep, p), p);
-            if (neg) v = sub_mod(v, K[lay.top() + i], p);
-            out[(size_t)i * total + idx] = v;
-        }
+    if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = best;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; ++w) best = wave_max[w] > best ? wave_max[w] : best;
+        out[blockIdx.x] = best;
     }
 }
 
@@ -935,18 +1110,114 @@ __global__ void __launch_bounds__(128) zz_crt_kernel(const uint32_t *__restrict_
     }
 }
 
-// Largest coefficient bit size of a view (one pass, one read-back).
-lbx_status zz_logmax(lbx_ctx *ctx, const DevView &v, int nl, unsigned *bits, hipStream_t s)
+// Largest coefficient bit sizes of both operands.
+lbx_status zz_logmax(lbx_ctx *ctx, const DevView &a, const DevView &b, int nl, unsigned *la, unsigned *lb,
+                     hipStream_t s)
 {
-    void *w = nullptr;
-    LBX_TRY(ensure(ctx, "zz_logmax", 256, &w));
-    LBX_TRY_HIP(hipMemsetAsync(w, 0, 4, s));
-    const size_t entries = v.rows * v.cols;
-    hipLaunchKernelGGL(zz_logmax_kernel, dim3(grid_of(entries * v.size, 256)), dim3(256), 0, s, v, nl, entries, v.size,
-                       (unsigned *)w);
+    if (!ctx->zz_bits)
+        LBX_TRY_HIP(hipHostMalloc((void **)&ctx->zz_bits, 2 * kLogmaxGroups * sizeof(unsigned), hipHostMallocDefault));
+    const size_t ea = a.rows * a.cols, eb = b.rows * b.cols, most = std::max(ea * a.size, eb * b.size);
+    const unsigned half = (unsigned)std::min<size_t>(kLogmaxGroups, (most + 255) / 256);
+    hipLaunchKernelGGL(zz_logmax_kernel, dim3(2 * half), dim3(256), 0, s, a, ea, b, eb, nl, ctx->zz_bits);
     LBX_TRY_HIP(hipGetLastError());
-    LBX_TRY_HIP(hipMemcpyAsync(bits, w, 4, hipMemcpyDeviceToHost, s));
     LBX_TRY_HIP(hipStreamSynchronize(s));
+    const unsigned *v = ctx->zz_bits;
+    *la = *std::max_element(v, v + half);
+    *lb = *std::max_element(v + half, v + 2 * half);
+    return LBX_OK;
+}
+
+// Plan of an integer product: FFT primes whose product exceeds bound = 2 maxA
+// maxB k min(sa,sb), maxA maxB = 2^lab (:78-86), and the constants for nl-word
+// inputs and cl-word results.  Kept in the context by these numbers; at most
+// kZzPlans of them (other data of the same program has few bit sizes).
+constexpr size_t kZzPlans = 64;
+
+lbx_status get_zz_plan(lbx_ctx *ctx, unsigned lab, size_t k, size_t minsz, unsigned lpts, int nl, int cl, MpPlan **out)
+{
+    const std::string prefix = "zz|";
+    const std::string key = prefix + std::to_string(lab) + "|" + std::to_string(k) + "|" + std::to_string(minsz) + "|" +
+                            std::to_string(lpts) + "|" + std::to_string(nl) + "|" + std::to_string(cl);
+    const auto it = ctx->mp_plans.find(key);
+    if (it != ctx->mp_plans.end()) {
+        *out = it->second;
+        return LBX_OK;
+    }
+    Limbs bound{1};
+    for (unsigned i = 0; i < lab + 1; ++i) limbs_mul_small(bound, 2);
+    limbs_mul_small(bound, (uint32_t)k);
+    limbs_mul_small(bound, (uint32_t)minsz);
+    limbs_trim(bound);
+    const size_t bits = 32 * (bound.size() - 1) + 32 - __builtin_clz(bound.back());  // bound < 2^bits
+    if (bits > (size_t)32 * cl) return LBX_ERR_SIZE_MISMATCH;  // bound/2 < 2^(bits-1) needs bits-1 bits and a sign
+    std::vector<uint32_t> primes;
+    if (!generate_primes((uint64_t)1 << 31, bound, lpts, primes) || (int)primes.size() > kZzMaxPrimes)
+        return LBX_ERR_NOT_ENOUGH_PRIMES;
+    const int r = (int)primes.size();
+    const ZzLayout lay{r, cl};
+    std::vector<uint32_t> K((size_t)lay.words(), 0);
+    const auto low = [&](const Limbs &x, uint32_t *dst, int n) {  // x mod 2^(32 n)
+        for (int l = 0; l < n; ++l) dst[l] = l < (int)x.size() ? x[l] : 0;
+    };
+    Limbs W{1};  // prod_{j<i} p_j
+    for (int i = 0; i < r; ++i) {
+        const uint32_t p = primes[i];
+        K[lay.primes() + i] = p;
+        K[lay.onep() + i] = shoup_pre(1, p);
+        for (int j = 0; j < i; ++j) {
+            const uint32_t inv = invmod_h(primes[j] % p, p);
+            K[lay.inv() + 2 * (i * r + j)] = inv;
+            K[lay.inv() + 2 * (i * r + j) + 1] = shoup_pre(inv, p);
+        }
+        low(W, &K[lay.W() + i * cl], cl);
+        limbs_mul_small(W, p);
+    }
+    low(W, &K[lay.M()], cl);
+    std::unique_ptr<MpPlan> plan(new MpPlan());
+    plan->primes = primes;
+    plan->lpts = lpts;
+    plan->nlimbs = nl;
+    plan->res_off = K.size();
+    residue_constants(K, primes, nl);
+    // M > bound (1 + 2^-16): M 2^16 > bound (2^16 + 1)
+    Limbs lhs = W, rhs = bound;
+    limbs_mul_small(lhs, 1u << 16);
+    limbs_mul_small(rhs, (1u << 16) + 1);
+    const int nw = limbs_cmp(lhs, rhs) > 0 ? crt_words(primes, cl) : 0;
+    if (nw) {
+        plan->crt_off = K.size();
+        crt_constants(K, primes, nw, [&](const Limbs &x, uint32_t *dst) { low(x, dst, nw); },
+                      [&](const Limbs &x, uint32_t *dst) {  // -M mod 2^(32 nw)
+                          low(x, dst, nw);
+                          uint32_t carry = 1;
+                          for (int l = 0; l < nw; ++l) {
+                              dst[l] = ~dst[l] + carry;
+                              carry = carry && dst[l] == 0;
+                          }
+                      });
+    }
+    size_t held = 0;
+    for (const auto &kv : ctx->mp_plans) held += kv.first.compare(0, prefix.size(), prefix) == 0;
+    if (held >= kZzPlans) {  // their constants may be in use by work still queued
+        (void)hipDeviceSynchronize();
+        for (auto p = ctx->mp_plans.begin(); p != ctx->mp_plans.end();) {
+            if (p->first.compare(0, prefix.size(), prefix) != 0) {
+                ++p;
+                continue;
+            }
+            (void)hipFree(p->second->d_const);
+            delete p->second;
+            p = ctx->mp_plans.erase(p);
+        }
+    }
+    LBX_TRY_HIP(hipMalloc(&plan->d_const, K.size() * 4));
+    const hipError_t e = hipMemcpy(plan->d_const, K.data(), K.size() * 4, hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        (void)hipFree(plan->d_const);
+        return from_hip(e);
+    }
+    ctx->mp_plans[key] = plan.get();
+    *out = plan.release();
     return LBX_OK;
 }
 
@@ -963,63 +1234,24 @@ lbx_status zz_product(lbx_ctx *ctx, int nl, int cl, const DevView &a, const DevV
         ++lpts;
     }
     unsigned la = 0, lb = 0;
-    LBX_TRY(zz_logmax(ctx, a, nl, &la, s));
-    LBX_TRY(zz_logmax(ctx, b, nl, &lb, s));
-    // bound = 2 maxA maxB k min(sa,sb), maxA = 2^la, maxB = 2^lb (:78-86);
-    // |coefficient| < bound/2 must fit cl words with its sign
-    Limbs bound{1};
-    for (unsigned i = 0; i < la + lb + 1; ++i) limbs_mul_small(bound, 2);
-    limbs_mul_small(bound, (uint32_t)k);
-    limbs_mul_small(bound, (uint32_t)(sa < sb ? sa : sb));
-    limbs_trim(bound);
-    size_t bits = 32 * (bound.size() - 1) + 32 - __builtin_clz(bound.back());  // bound < 2^bits
-    if (bits > (size_t)32 * cl) return LBX_ERR_SIZE_MISMATCH;  // bound/2 < 2^(bits-1) needs bits-1 bits and a sign
-    std::vector<uint32_t> primes;
-    if (!generate_primes((uint64_t)1 << 31, bound, lpts, primes) || (int)primes.size() > kZzMaxPrimes)
-        return LBX_ERR_NOT_ENOUGH_PRIMES;
-    const int r = (int)primes.size();
-    const ZzLayout lay{r, cl};
-    std::vector<uint32_t> K((size_t)lay.words(), 0);
-    Limbs W{1};  // prod_{j<i} p_j, kept below 2^(32 cl)
-    for (int i = 0; i < r; ++i) {
-        const uint32_t p = primes[i];
-        K[lay.primes() + i] = p;
-        K[lay.onep() + i] = shoup_pre(1, p);
-        const uint32_t r32 = (uint32_t)(((uint64_t)1 << 32) % p);
-        K[lay.r32() + i] = r32;
-        K[lay.r32p() + i] = shoup_pre(r32, p);
-        uint64_t top = 1;
-        for (int l = 0; l < nl; ++l) top = top * r32 % p;
-        K[lay.top() + i] = (uint32_t)top;
-        for (int j = 0; j < i; ++j) {
-            const uint32_t inv = invmod_h(primes[j] % p, p);
-            K[lay.inv() + 2 * (i * r + j)] = inv;
-            K[lay.inv() + 2 * (i * r + j) + 1] = shoup_pre(inv, p);
-        }
-        for (int l = 0; l < cl; ++l) K[lay.W() + i * cl + l] = l < (int)W.size() ? W[l] : 0;
-        limbs_mul_small(W, p);
-        if ((int)W.size() > cl) W.resize(cl);
-    }
-    for (int l = 0; l < cl; ++l) K[lay.M() + l] = l < (int)W.size() ? W[l] : 0;
-    void *dk, *ra, *rb, *rc;
-    LBX_TRY(ensure(ctx, "zz_const", K.size() * 4, &dk));
-    // the stream is idle here (zz_logmax waited for it): a blocking copy from K
-    LBX_TRY_HIP(hipMemcpy(dk, K.data(), K.size() * 4, hipMemcpyHostToDevice));
+    LBX_TRY(zz_logmax(ctx, a, b, nl, &la, &lb, s));
+    MpPlan *plan;
+    LBX_TRY(get_zz_plan(ctx, la + lb, k, sa < sb ? sa : sb, lpts, nl, cl, &plan));
+    const int r = (int)plan->primes.size();
+    void *ra, *rb, *rc;
     LBX_TRY(ensure(ctx, "mp_ra", (size_t)r * m * k * sa * 4, &ra));
     LBX_TRY(ensure(ctx, "mp_rb", (size_t)r * k * n * sb * 4, &rb));
     LBX_TRY(ensure(ctx, "mp_rc", (size_t)r * m * n * sc * 4, &rc));
-    auto residues = nl <= 8 ? zz_residue_kernel<8> : zz_residue_kernel<kZzMaxIn>;
-    hipLaunchKernelGGL(residues, dim3(grid_of(m * k * sa, 256)), dim3(256), 0, s, a, nl, m * k, sa,
-                       (const uint32_t *)dk, r, (uint32_t *)ra);
-    LBX_TRY_HIP(hipGetLastError());
-    hipLaunchKernelGGL(residues, dim3(grid_of(k * n * sb, 256)), dim3(256), 0, s, b, nl, k * n, sb,
-                       (const uint32_t *)dk, r, (uint32_t *)rb);
-    LBX_TRY_HIP(hipGetLastError());
+    LBX_TRY_HIP(launch_residues<true>(a, m * k, (uint32_t *)ra, b, k * n, (uint32_t *)rb, nl, r,
+                                      plan->d_const + plan->res_off, s));
     const DevView va{(uint32_t *)ra, LBX_POLFIRST, m, k, sa, 0, sa}, vb{(uint32_t *)rb, LBX_POLFIRST, k, n, sb, 0, sb};
-    LBX_TRY(prime_products(ctx, primes, va, m * k * sa, vb, k * n * sb, (uint32_t *)rc, m, k, n, sc, lpts, method, s,
-                           nullptr));
+    LBX_TRY(prime_products(ctx, plan->primes, va, m * k * sa, vb, k * n * sb, (uint32_t *)rc, m, k, n, sc, lpts, method,
+                           s, nullptr));
+    if (plan->crt_off)
+        return from_hip(launch_crt_direct<false>(crt_words(plan->primes, cl), (const uint32_t *)rc, m * n, sc,
+                                                 plan->d_const + plan->crt_off, r, cl, c, s));
     hipLaunchKernelGGL(zz_crt_kernel, dim3(grid_of(m * n * sc, 128)), dim3(128), 0, s, (const uint32_t *)rc, m * n,
-                       sc, (const uint32_t *)dk, r, cl, c);
+                       sc, (const uint32_t *)plan->d_const, r, cl, c);
     LBX_TRY_HIP(hipGetLastError());
     return LBX_OK;
 }

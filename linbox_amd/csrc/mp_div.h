@@ -1,8 +1,8 @@
 // Remainder of a multiword accumulator by a normalized multiword modulus,
 // shared by the CRT kernels and a host build of the same code.
 //
-// The CRT recombination forms U = sum_i v_i (M_i mod P) 2^sh with v_i < 2^31
-// and r <= 32 terms, so U < 2^36 Q where Q = P 2^sh.  sh = 32 off + s places P
+// The CRT recombination forms U = (sum_i y_i (M/p_i mod P) + q (-M mod P)) 2^sh
+// with y_i < 2^31, r <= 32 terms and q < r, so U < 2^36 Q where Q = P 2^sh.  sh = 32 off + s places P
 // at the top of NL words with its top bit set (off = NL - limbs(P),
 // s = leading zeros of P's top word), which makes Q a normalized divisor of
 // exactly NL words.  U then has NL + 2 words, its quotient by Q is below 2^36,

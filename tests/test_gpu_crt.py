@@ -178,3 +178,34 @@ def test_batched_primes_with_plan_eviction(ctx, crt):
                                       m, k, n, a, sa, b, sb)
         assert st == 0 and len(primes) >= 6
         assert np.array_equal(dc.download(), ref), (m, k, n, sa, sb)
+
+
+@pytest.mark.parametrize("nl", [2, 3, 4, 5, 6, 7, 8, 9, 16])
+def test_crt_word_counts(ctx, nl):
+    """Every staged coefficient width and wider ones, with moduli that fill their
+    words, that leave the top bits free and that leave the top word zero, and
+    operands of P - 1, 0 and random values, against Python integers."""
+    rng = np.random.default_rng(nl)
+    for bits in (32 * nl, 32 * nl - 13, 32 * nl - 32 + 1, max(33, 32 * nl - 40)):
+        P = (1 << bits) - 1 - 2 * int(rng.integers(1, 1 << 20)) if bits > 33 else (1 << 33) - 9
+        m, k, n, sa, sb = 2, 2, 2, 45, 4
+
+        def draw(count):
+            v = [int.from_bytes(rng.bytes(4 * nl + 8), "little") % P for _ in range(count)]
+            for i in range(0, count, 3):
+                v[i] = (P - 1, 0, 1, 0xFFFFFFFF % P)[i // 3 % 4]
+            return v
+
+        def words(v):
+            return np.array([[(x >> (32 * l)) & 0xFFFFFFFF for l in range(nl)] for x in v], np.uint32).reshape(-1)
+        A, B = draw(m * k * sa), draw(k * n * sb)
+        say("crt word counts", nl, bits)
+        got = gpu_mp(ctx, P, nl, m, k, n, words(A), sa, words(B), sb, lbx.METHOD_AUTO)
+        ref = [0] * (m * n * (sa + sb - 1))
+        for i in range(m):
+            for j in range(n):
+                for q in range(k):
+                    for u in range(sa):
+                        for v in range(sb):
+                            ref[(i * n + j) * (sa + sb - 1) + u + v] += A[(i * k + q) * sa + u] * B[(q * n + j) * sb + v]
+        assert np.array_equal(got, words([x % P for x in ref])), (nl, bits)

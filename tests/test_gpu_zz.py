@@ -177,3 +177,36 @@ def test_zz_errors(ctx):
         with pytest.raises(LinboxError) as e:
             mul_zz(c, a, b, ctx=ctx)
         assert e.value.status == 11  # LBX_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("wi", [1, 2, 3, 4, 5, 6, 7, 8, 9])
+def test_zz_word_counts(ctx, wi):
+    """Every staged coefficient width and the next one, more coefficients than a
+    group, extreme values and windows of larger storage; 3 to 20 primes, so both
+    recombinations."""
+    lo, hi = -(1 << (32 * wi - 1)), (1 << (32 * wi - 1)) - 1
+    rnd = random.Random(100 + wi)
+    m, k, n, sa, sb = 2, 3, 2, 47, 5
+    pool = [lo, hi, -1, 0, 1, lo + 1, hi - 1, -(1 << 31), (1 << 31) - 1]
+    A = [rnd.choice(pool) if rnd.random() < 0.5 else rnd.randrange(lo, hi + 1) for _ in range(m * k * sa)]
+    B = [rnd.choice(pool) if rnd.random() < 0.5 else rnd.randrange(lo, hi + 1) for _ in range(k * n * sb)]
+    ref = naive(A, B, m, k, n, sa, sb)
+    wo = out_words(A, B, k, sa, sb)
+    say("zz word counts", wi, wo)
+    assert gpu_zz(ctx, A, B, m, k, n, sa, sb, wi, wo) == ref
+    # the same operands in matfirst storage, and as windows of longer rows
+    def window(v, rows, cols, size, layout, words):
+        M = PolynomialMatrix(rows, cols, size + 3, layout, nlimbs=words)
+        w = to_limbs(v, words).reshape(rows * cols, size, words)
+        d = np.zeros((rows * cols, size + 3, words), np.uint32)
+        d[:, 2:2 + size] = w
+        M.data[:] = (d if layout == "polfirst" else d.transpose(1, 0, 2)).reshape(-1)
+        return M, M.at(2, size + 1)
+
+    for layout in ("polfirst", "matfirst"):
+        C, Cv = window([0] * (m * n * (sa + sb - 1)), m, n, sa + sb - 1, layout, wo)
+        mul_zz(Cv, window(A, m, k, sa, layout, wi)[1], window(B, k, n, sb, layout, wi)[1], ctx=ctx)
+        got = np.asarray(C.data).reshape((m * n, -1, wo) if layout == "polfirst" else (-1, m * n, wo))
+        got = got if layout == "polfirst" else got.transpose(1, 0, 2)
+        assert from_limbs(np.ascontiguousarray(got[:, 2:-1]).reshape(-1), wo) == ref
+        assert not got[:, :2].any() and not got[:, -1:].any()
