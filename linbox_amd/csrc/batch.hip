@@ -456,7 +456,7 @@ lbx_status build_plan(lbx_ctx *ctx, const std::vector<lbx_job> &jobs, const std:
         if ((st = twiddles(ctx, x.p, L, root, kTwMont, &J.twf)) != LBX_OK) return fail(st);
         if ((st = twiddles(ctx, x.p, L, invroot(x.p, L, root), kTwShoup, &J.twi)) != LBX_OK) return fail(st);
         const uint32_t inv_n = invmod_h((uint32_t)(((uint64_t)1 << L) % x.p), x.p);
-        J.pc = plain_const(x.p, inv_n);
+        J.pc = plain_s_const(x.p, inv_n);
         J.form = 0;
         if (icls[j] >= 0) {
             uint8_t *base = (uint8_t *)plan->ws + ioff[j];
@@ -502,7 +502,8 @@ lbx_status build_plan(lbx_ctx *ctx, const std::vector<lbx_job> &jobs, const std:
     std::vector<MfmaItem> mi;
     std::vector<TrItem> tr;
     for (uint32_t j : order) {
-        const BatchJob &J = plan->jobs[j];
+        BatchJob &J = plan->jobs[j];
+        J.h = J.form == 1 ? ~0u : J.p >> 1;
         if (J.form == 1) {
             limb_items_for(J, j, li);
             mfma_items_for(J, j, (uint32_t)std::max(1, ctx->ppi_tuned[icls[j]]), mi);

@@ -214,37 +214,41 @@ private:
 };
 
 // AUTO picks the INT8 form where it measured faster on gfx950 (both forms are
-// bit-exact): for large products.  Below, the split transforms and the seven
-// launches it needs cost more than the VALU pointwise they replace (plain /
-// INT8, us: 32^3 at 2^8 points 27 / 36, at 2^13 116 / 177; 48^3 at 2^13 311 /
-// 304; 64^2x32 at 2^11 91 / 97, at 2^13 347 / 291; 64^3 at 2^6 33 / 43, at 2^8
-// 45 / 44, at 2^10 91 / 81, at 2^13 616 / 427; 96^3 at 2^8 99 / 65).  MFMA tiles
-// are 32x32 with a 64-deep inner step, so every dimension must be at least 16,
-// and an inner dimension below 32 is mostly padding (100x17x100 at 2^13: 557 / 719).
+// bit-exact): for large products on long transforms, and sooner where its
+// padding (rows to 32, the inner dimension to 64) adds nothing.  Elsewhere the
+// split transforms and the seven launches it needs cost more than the VALU
+// pointwise they replace.  Whole products, plain / INT8, us:
+//             2^8 points  2^10       2^11       2^12        2^13
+//   32^3        22 / 36   32 / 52    48 / 70    65 / 109   108 / 178
+//   64^2x32     31 / 40   53 / 61    81 / 97   147 / 158   312 / 290
+//   64^3        39 / 44   69 / 81   117 / 123  231 / 220   490 / 420
+//   80^3        58 / 59  106 / 135  198 / 249  398 / 446   799 / 852
+//   96^3        67 / 65  151 / 152  287 / 301  588 / 530  1208 / 1034
+//   100^3       67 / 73  186 / 187  342 / 357  688 / 641  1422 / 1271
+//   128x64x64   52 / 56  104 / 103  196 / 193  411 / 352   861 / 687
+//   128^3       90 / 82  273 / 238  558 / 467 1157 / 841  2403 / 1637
 int choose_method(int method, size_t m, size_t k, size_t n, unsigned L)
 {
     if (method == LBX_METHOD_PLAIN_U64 || method == LBX_METHOD_INT8_MFMA) return method;
     if (m < 16 || n < 16 || k < 16) return LBX_METHOD_PLAIN_U64;
-    const double mkn = (double)m * k * n, two17 = (double)(1u << 17);
-    const bool big = mkn >= 4 * two17 || (mkn >= 2 * two17 && L >= 8) || (mkn >= two17 && k >= 32 && L >= 13);
+    const auto up = [](size_t x, size_t to) { return (double)((x + to - 1) / to * to); };
+    const double mkn = (double)m * k * n, used = mkn / (up(m, 32) * up(k, 64) * up(n, 32));
+    const double two18 = (double)(1u << 18);
+    const bool big = (L >= 12 && mkn >= two18 && used >= 0.45) ||
+                     (mkn >= 2 * two18 && used >= 0.95 && mkn * (double)((uint64_t)1 << L) >= 2048 * two18);
     return big ? LBX_METHOD_INT8_MFMA : LBX_METHOD_PLAIN_U64;
 }
 
-// The plain form's operand layout: point-major blocks from the split
-// transforms (each operand word read once per output tile) for large matrices,
-// polfirst transform output (one point per lane, operands re-read once per
-// 8-wide register tile) otherwise.  Measured on gfx950 (2013265921, whole
-// products): 128^3 at 2^14 points 5.58 ms point-major against 7.23 ms; 128^3 at
-// 2^11 0.865 against 0.863 ms; 64^3 at 2^13 0.749 against 0.679 ms; 32^3 at 2^13
-// 0.289 against 0.192 ms -- the split transforms cost more than the re-reads
-// below ~100 rows.  LBX_PLAIN_LAYOUT = "point" or "entry" overrides the choice
+// The plain form's operand layout: polfirst transform output (one point per
+// lane), which the tiled pointwise kernel reads at a cost that no longer pays
+// for split transforms at any size (entry-major / point-major, us: 96^3 at 2^13
+// points 1208 / 2175, 128^3 at 2^8 90 / 125, at 2^13 2403 / 2579, 160^3 at 2^13
+// 4544 / 9193).  LBX_PLAIN_LAYOUT = "point" takes the point-major form
 // (measurement and tests).
-bool plain_point_major(size_t m, size_t k, size_t n)
+bool plain_point_major()
 {
     const char *e = std::getenv("LBX_PLAIN_LAYOUT");
-    if (e && !std::strcmp(e, "point")) return true;
-    if (e && !std::strcmp(e, "entry")) return false;
-    return m >= 96 && n >= 96 && k >= 64;
+    return e && !std::strcmp(e, "point");
 }
 
 // Bytes of head -> tail intermediate per chunk.  The default, 2 GiB, gives one
@@ -374,7 +378,7 @@ lbx_status multi_prime(MultiProduct &mp, unsigned i, uint32_t p, const MidSpec *
     mp.p[i] = p;
     mp.twa[i] = mid && !mid->small_left ? twi : twf;
     mp.twb[i] = mid && mid->small_left ? twi : twf;
-    mp.pc[i] = plain_const(p, invmod_h((uint32_t)(((size_t)1 << mp.L) % p), p));
+    mp.scale[i] = invmod_h((uint32_t)(((size_t)1 << mp.L) % p), p);
     return LBX_OK;
 }
 
@@ -391,7 +395,7 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
     if (L > (unsigned)kMaxLog) return LBX_ERR_UNSUPPORTED;
     method = choose_method(method, m, k, n, L);
     const bool int8 = method == LBX_METHOD_INT8_MFMA;
-    const bool split = L >= 8 && L <= (unsigned)kMaxLdsLog && (int8 || plain_point_major(m, k, n));
+    const bool split = L >= 8 && L <= (unsigned)kMaxLdsLog && (int8 || plain_point_major());
     // whole transforms of both operands in one launch (a middle product's
     // reversal included)
     const bool fused = !split && !int8 && L >= 1 && L <= (unsigned)kMaxLdsLog;
@@ -572,7 +576,7 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
         mp.ahat = (uint32_t *)ahat, mp.bhat = (uint32_t *)bhat, mp.chat = (uint32_t *)chat;
         mp.count = count;
         mp.p[0] = p, mp.twa[0] = twa, mp.twb[0] = twb, mp.twc[0] = twc;
-        mp.pc[0] = plain_const(p, inv_n);
+        mp.scale[0] = inv_n;
         {
             KernelTimer kt(ctx, s, "kernel dif", timing);
             LBX_TRY_HIP(launch_multi_forward(mp, s));
@@ -612,9 +616,8 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
     } else {
         {
             KernelTimer kt(ctx, s, "kernel pw_plain", timing);
-            const PlainConst pc = plain_const(p, inv_n);
             LBX_TRY_HIP(launch_pointwise_plain((const uint32_t *)ahat, (const uint32_t *)bhat, (uint32_t *)chat, m, k,
-                                               n, N, 1, &p, &pc, s));
+                                               n, N, 1, &p, &inv_n, s));
         }
         st.mark("Pointwise mult");
     }
@@ -639,9 +642,9 @@ lbx_status constant_product(lbx_ctx *ctx, uint32_t p, const DevView &a, const De
     LBX_TRY(ws.get("chat", m * n * 4, &chat));
     LBX_TRY_HIP(launch_gather(a, m * k, 1, (uint32_t *)ahat, 1, s));
     LBX_TRY_HIP(launch_gather(b, k * n, 1, (uint32_t *)bhat, 1, s));
-    const PlainConst pc = plain_const(p, 1);
+    const uint32_t one = 1 % p;
     LBX_TRY_HIP(launch_pointwise_plain((const uint32_t *)ahat, (const uint32_t *)bhat, (uint32_t *)chat, m, k, n, 1, 1,
-                                       &p, &pc, s));
+                                       &p, &one, s));
     LBX_TRY_HIP(launch_scatter((const uint32_t *)chat, 1, m * n, 1, c, s));
     return LBX_OK;
 }

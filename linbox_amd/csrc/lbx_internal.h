@@ -142,7 +142,7 @@ struct MultiProduct {
     size_t cstride, count;
     uint32_t p[kMultiPrimes];
     const uint2 *twa[kMultiPrimes], *twb[kMultiPrimes], *twc[kMultiPrimes];  // Montgomery, Montgomery, Shoup tables
-    PlainConst pc[kMultiPrimes];                                           // with the scale 2^-L
+    uint32_t scale[kMultiPrimes];                                          // 2^-L mod p
 };
 hipError_t launch_multi_forward(const MultiProduct &mp, hipStream_t s);
 hipError_t launch_multi_pointwise(const MultiProduct &mp, hipStream_t s);
@@ -151,9 +151,15 @@ hipError_t launch_multi_inverse(const MultiProduct &mp, hipStream_t s);
 // ---- pointwise stage (pointwise.hip) ----
 // C[e'][t] = scale * sum_q A[i*k+q][t] B[q*n+j][t] mod p at every point t < npts,
 // all operands polfirst with row stride npts (e' = i*n+j); r such products, of
-// primes p[i] with constants pc[i], one after the other in each buffer.
+// primes p[i] with scale[i] < p[i], one after the other in each buffer.
+// launch_pointwise_plain takes words in [0, p) and any npts (a power of two);
+// launch_pointwise_tiled centred int32 words where pointwise_tiled says so.
 hipError_t launch_pointwise_plain(const uint32_t *A, const uint32_t *B, uint32_t *C, size_t m, size_t k,
-                                  size_t n, size_t npts, unsigned r, const uint32_t *p, const PlainConst *pc,
+                                  size_t n, size_t npts, unsigned r, const uint32_t *p, const uint32_t *scale,
+                                  hipStream_t s);
+bool pointwise_tiled(size_t npts);
+hipError_t launch_pointwise_tiled(const uint32_t *A, const uint32_t *B, uint32_t *C, size_t m, size_t k,
+                                  size_t n, size_t npts, unsigned r, const uint32_t *p, const uint32_t *scale,
                                   hipStream_t s);
 
 // Bytes of one point's limb block for an operand with `rows` rows and inner
@@ -186,7 +192,8 @@ struct BatchJob {
     uint32_t *c;
     uint32_t *ahat, *bhat, *chat;  // m*k, k*n, m*n rows of 2^L words
     const uint2 *twf, *twi;        // root: forward (Montgomery) table; its inverse: inverse (Shoup) table
-    PlainConst pc;                 // plain epilogue constants with scale 2^-L
+    PlainSConst pc;                // plain epilogue constants with scale 2^-L
+    uint32_t h;                    // forward outputs above h less p: p/2 (plain, centred) or 2^32 - 1 (INT8)
     uint8_t *alimb, *blimb;        // INT8: per-point limb blocks of A and B^T (limb_block_bytes each)
     uint32_t *cmat;                // INT8: point-major product [t][i*n+j]
     MfmaConst mc;                  // INT8 epilogue constants with scale 2^-L

@@ -22,6 +22,7 @@ struct FwdArgs {
     size_t astride, bstride, rev_a, rev_b;
     uint32_t *ahat, *bhat;
     size_t ea, eb, ga;
+    bool centre;  // outputs centred to int32
     uint32_t p[kMultiPrimes];
     const uint2 *twa[kMultiPrimes], *twb[kMultiPrimes];
 };
@@ -39,8 +40,8 @@ struct InvArgs {
 // most rev coefficients then), zero where that is outside the view.
 template <int L, bool HALFZERO>
 __device__ __forceinline__ void forward_entry(const DevView &in, size_t rev, size_t e, bool active,
-                                              const uint2 *__restrict__ tw, uint32_t p, uint32_t *__restrict__ out,
-                                              int tp, uint32_t *lds)
+                                              const uint2 *__restrict__ tw, uint32_t p, uint32_t h,
+                                              uint32_t *__restrict__ out, int tp, uint32_t *lds)
 {
     using C = Cfg<L>;
     constexpr int RP0 = C::RLOG;
@@ -69,7 +70,7 @@ __device__ __forceinline__ void forward_entry(const DevView &in, size_t rev, siz
             }
     }
     dif_passes<L, 0, L, HALFZERO>(x, lds, tp, tw, p);
-    if (active) dif_store<L>(x, tp, out + e * C::N);
+    if (active) dif_store<L, true>(x, tp, out + e * C::N, p, h);
 }
 
 template <int L>
@@ -87,10 +88,11 @@ __global__ void __launch_bounds__(Cfg<L>::BLOCK) multi_dif_kernel(FwdArgs A)
     const int pib = threadIdx.x / C::TP, tp = threadIdx.x % C::TP;
     const size_t e = (size_t)(isa ? blockIdx.x : blockIdx.x - A.ga) * C::G + pib;
     uint32_t *lds = lds_all + pib * C::STRIDE;
+    const uint32_t h = A.centre ? A.p[i] >> 1 : ~0u;
     if ((rev ? rev : in.size) * 2 <= (size_t)C::N)
-        forward_entry<L, true>(in, rev, e, e < entries, global_ptr(tw), A.p[i], out, tp, lds);
+        forward_entry<L, true>(in, rev, e, e < entries, global_ptr(tw), A.p[i], h, out, tp, lds);
     else
-        forward_entry<L, false>(in, rev, e, e < entries, global_ptr(tw), A.p[i], out, tp, lds);
+        forward_entry<L, false>(in, rev, e, e < entries, global_ptr(tw), A.p[i], h, out, tp, lds);
 }
 
 template <int L>
@@ -158,6 +160,7 @@ hipError_t launch_multi_forward(const MultiProduct &mp, hipStream_t s)
     A.bhat = mp.bhat;
     A.ea = mp.m * mp.k;
     A.eb = mp.k * mp.n;
+    A.centre = pointwise_tiled((size_t)1 << mp.L);
     for (int i = 0; i < kMultiPrimes; ++i) {
         const bool on = i < (int)mp.r;
         A.p[i] = on ? mp.p[i] : 0;
@@ -176,8 +179,10 @@ hipError_t launch_multi_forward(const MultiProduct &mp, hipStream_t s)
 hipError_t launch_multi_pointwise(const MultiProduct &mp, hipStream_t s)
 {
     if (!in_range(mp)) return hipErrorInvalidValue;
-    return launch_pointwise_plain(mp.ahat, mp.bhat, mp.chat, mp.m, mp.k, mp.n, (size_t)1 << mp.L, mp.r, mp.p, mp.pc,
-                                  s);
+    const size_t npts = (size_t)1 << mp.L;
+    if (pointwise_tiled(npts))
+        return launch_pointwise_tiled(mp.ahat, mp.bhat, mp.chat, mp.m, mp.k, mp.n, npts, mp.r, mp.p, mp.scale, s);
+    return launch_pointwise_plain(mp.ahat, mp.bhat, mp.chat, mp.m, mp.k, mp.n, npts, mp.r, mp.p, mp.scale, s);
 }
 
 hipError_t launch_multi_inverse(const MultiProduct &mp, hipStream_t s)

@@ -428,9 +428,9 @@ __global__ void __launch_bounds__(kBatchNttThreads, (batch_waves<L, INVERSE>()))
             uint32_t *out = global_ptr(isa ? J.ahat : J.bhat);
             const uint2 *tw = global_ptr(J.twf);
             if (in.size * 2 <= (size_t)C::N)
-                dif_body<L, L, true>(in, e_end, id, tw, J.p, out, e_base, tid, lds);
+                dif_body<L, L, true, true>(in, e_end, id, tw, J.p, out, e_base, tid, lds, J.h);
             else
-                dif_body<L, L, false>(in, e_end, id, tw, J.p, out, e_base, tid, lds);
+                dif_body<L, L, false, true>(in, e_end, id, tw, J.p, out, e_base, tid, lds, J.h);
         } else {
             DevView out;
             out.base = global_ptr(J.c);

@@ -237,12 +237,18 @@ constexpr int dif_last_rp()
     return (SEND % Cfg<L>::RLOG) ? (SEND % Cfg<L>::RLOG) : Cfg<L>::RLOG;
 }
 
-// The words of a whole forward transform (all L stages) to its row o.
-template <int L>
-__device__ __forceinline__ void dif_store(const uint32_t (&x)[Cfg<L>::R], int tp, uint32_t *__restrict__ o)
+// The words of a whole forward transform (all L stages) to its row o; with
+// CENTRE those above h less p (h = p/2: centred to int32; h = 2^32 - 1: as they are).
+template <int L, bool CENTRE>
+__device__ __forceinline__ void dif_store(uint32_t (&x)[Cfg<L>::R], int tp, uint32_t *__restrict__ o, uint32_t p,
+                                          uint32_t h)
 {
     using C = Cfg<L>;
     constexpr int RP = dif_last_rp<L, L>();
+    if constexpr (CENTRE) {
+#pragma unroll
+        for (int q = 0; q < C::R; ++q) x[q] -= x[q] > h ? p : 0u;
+    }
 #pragma unroll
     for (int u = 0; u < (C::R >> RP); ++u) {
         const int g = tp + u * C::TP;
@@ -263,10 +269,10 @@ __device__ __forceinline__ void dif_store(const uint32_t (&x)[Cfg<L>::R], int tp
 // result is the full transform (R consecutive words per thread are stored as
 // 16-byte vectors); with SEND < L the data is left in natural storage order
 // as 2^(L-SEND) independent blocks for the remaining stages.
-template <int L, int SEND, bool HALFZERO>
+template <int L, int SEND, bool HALFZERO, bool CENTRE = false>
 __device__ __forceinline__ void dif_body(const DevView &in, size_t entries, const EntryMap &map,
                                          const uint2 *__restrict__ tw, uint32_t p, uint32_t *__restrict__ out,
-                                         size_t e_base, int tid, uint32_t *lds_all)
+                                         size_t e_base, int tid, uint32_t *lds_all, uint32_t h = ~0u)
 {
     using C = Cfg<L>;
     const int pib = tid / C::TP;
@@ -302,7 +308,7 @@ __device__ __forceinline__ void dif_body(const DevView &in, size_t entries, cons
     constexpr int NG = C::R >> RP;
     if (!active) return;
     if constexpr (SEND == L) {
-        dif_store<L>(x, tp, out + e * C::N);
+        dif_store<L, CENTRE>(x, tp, out + e * C::N, p, h);
     } else {  // block-major: [block][entry][2^(L-SEND) words]
 #pragma unroll
         for (int u = 0; u < NG; ++u)

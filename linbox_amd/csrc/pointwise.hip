@@ -5,12 +5,12 @@
 // The reference runs one fflas fgemm per point.  Here all points are one
 // launch, in one of two forms:
 //
-//  * plain: vector ALUs, one point per lane, a TIxTJ register tile of 64-bit
-//    accumulators per lane.  Each product a*b < p^2 < 2^62 is added with
-//    carry into (acc:u64, hi:u32), i.e. reduction is delayed to the end of the
-//    k loop, where (hi,acc) is reduced with three Shoup products.  Operands
-//    are read straight from the polfirst NTT output: consecutive lanes read
-//    consecutive points, so every load is coalesced.
+//  * plain: vector ALUs, one point per lane, a T x T register tile of 64-bit
+//    accumulators per lane.  The reduction is delayed to the end of the k loop:
+//    products of centred words (below 2^60) are folded every six or more steps,
+//    and the sum is reduced once with two Shoup products.  Operands are read
+//    straight from the polfirst NTT output: consecutive lanes read consecutive
+//    points, so every load is coalesced.
 //
 //  * INT8 MFMA: every residue is centred (|c| < p/2 < 2^30) and split into
 //    four balanced signed 8-bit digits, c = sum_s d_s 2^(8s).  Then
@@ -81,9 +81,10 @@ __device__ __forceinline__ void pw_plain_body(const uint32_t *__restrict__ A, co
 }
 
 // Primes of one launch, in the kernel arguments.
+template <class Const>
 struct PlainPrimes {
     uint32_t p[kMultiPrimes];
-    PlainConst pc[kMultiPrimes];
+    Const pc[kMultiPrimes];
 };
 
 // One output tile at one point per lane; item = tile * npts + t, so a wave's
@@ -91,7 +92,8 @@ struct PlainPrimes {
 template <int T>
 __global__ void __launch_bounds__(256) pw_plain_kernel(const uint32_t *__restrict__ A, const uint32_t *__restrict__ B,
                                                        uint32_t *__restrict__ C, int m, int k, int n, size_t npts,
-                                                       unsigned log_npts, size_t items, PlainPrimes primes)
+                                                       unsigned log_npts, size_t items,
+                                                       PlainPrimes<PlainConst> primes)
 {
     const size_t item = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (item >= items) return;
@@ -99,15 +101,120 @@ __global__ void __launch_bounds__(256) pw_plain_kernel(const uint32_t *__restric
     const int tiles_j = (n + T - 1) / T;
     const size_t t = item & (npts - 1);
     const int tile = (int)(item >> log_npts);
-    pw_plain_body<T, T, T == 2 ? 8 : (T == 4 ? 2 : 0)>(A + (size_t)i * m * k * npts, B + (size_t)i * k * n * npts, C + (size_t)i * m * n * npts, m, k,
+    pw_plain_body<T, T, T == 2 ? 8 : 2>(A + (size_t)i * m * k * npts, B + (size_t)i * k * n * npts, C + (size_t)i * m * n * npts, m, k,
                         n, npts, primes.p[i], primes.pc[i], t, (tile / tiles_j) * T, (tile % tiles_j) * T);
+}
+
+// One T x T output tile at 64 points by one wave, on centred int32 words: per
+// inner step a lane loads its point's T words of A and of B (256 contiguous
+// bytes per wave and word) and adds T^2 products (v_mad_i64_i32), folding every
+// pc.every-th step.
+//
+// Bound by the loads' latency unless enough of them are in flight: a wave of
+// 8x8 tiles has 2 waves a SIMD beside it at most.  The words of the next D
+// steps are therefore loaded ahead into registers, and the addresses cost no
+// vector instruction or register: tile and inner index are uniform across the
+// wave, so every load takes a scalar base and the lane's one 32-bit offset.  Rows
+// past the edge read the last row again (their products are not stored), and
+// steps past the end the last step.  Measured against unsigned words folded
+// every two or three steps near 2^31 and no loads ahead: 14 primes of 32^3 at
+// 2^11 points 180 -> 120 us, 5 of 24^3 at 2^11 38 -> 24 us; with the loads ahead it
+// is bound by its vector instructions, 64 multiply-adds a step of some 84.
+template <int T, int D>
+__device__ __forceinline__ void pw_tile(const uint32_t *__restrict__ A, const uint32_t *__restrict__ B,
+                                        uint32_t *__restrict__ C, int m, int k, int n, size_t npts, uint32_t p,
+                                        const PlainSConst &pc, uint32_t t, int i0, int j0)
+{
+    // uniform row and column bases of the next step to load
+    const char *pa[T], *pb[T];
+#pragma unroll
+    for (int ii = 0; ii < T; ++ii) pa[ii] = (const char *)(A + (size_t)min(i0 + ii, m - 1) * k * npts);
+#pragma unroll
+    for (int jj = 0; jj < T; ++jj) pb[jj] = (const char *)(B + (size_t)min(j0 + jj, n - 1) * npts);
+    const uint32_t off = t * 4;
+    const size_t step_a = npts * 4, step_b = (size_t)n * npts * 4;
+    int32_t a[D][T], b[D][T];
+    int q_load = 0;
+    const auto load = [&](int d) {
+#pragma unroll
+        for (int ii = 0; ii < T; ++ii) a[d][ii] = *(const int32_t *)(pa[ii] + off);
+#pragma unroll
+        for (int jj = 0; jj < T; ++jj) b[d][jj] = *(const int32_t *)(pb[jj] + off);
+        ++q_load;
+        const size_t sa = q_load < k ? step_a : 0, sb = q_load < k ? step_b : 0;
+#pragma unroll
+        for (int ii = 0; ii < T; ++ii) pa[ii] += sa;
+#pragma unroll
+        for (int jj = 0; jj < T; ++jj) pb[jj] += sb;
+    };
+    int64_t acc[T][T];
+#pragma unroll
+    for (int ii = 0; ii < T; ++ii)
+#pragma unroll
+        for (int jj = 0; jj < T; ++jj) acc[ii][jj] = 0;
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(d);
+    int since = 0;  // products since the last fold
+    for (int q0 = 0; q0 < k; q0 += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            if (q0 + d < k) {
+#pragma unroll
+                for (int ii = 0; ii < T; ++ii)
+#pragma unroll
+                    for (int jj = 0; jj < T; ++jj) acc[ii][jj] += (int64_t)a[d][ii] * b[d][jj];
+                if (++since == (int)pc.every) {
+                    since = 0;
+#pragma unroll
+                    for (int ii = 0; ii < T; ++ii)
+#pragma unroll
+                        for (int jj = 0; jj < T; ++jj) acc[ii][jj] = plain_s_fold(acc[ii][jj], pc);
+                }
+                load(d);
+            }
+        }
+    }
+#pragma unroll
+    for (int ii = 0; ii < T; ++ii)
+#pragma unroll
+        for (int jj = 0; jj < T; ++jj) {
+            if (i0 + ii >= m || j0 + jj >= n) continue;
+            C[((size_t)(i0 + ii) * n + j0 + jj) * npts + t] = plain_s_finish(acc[ii][jj], p, pc);
+        }
+}
+
+// Steps loaded ahead: some 32 words a lane whatever the tile.
+template <int T>
+constexpr int tile_ahead() { return T == 8 ? 2 : (T == 4 ? 3 : 6); }
+// Waves per SIMD: the 128 accumulator registers and 32 ahead of an 8x8 tile leave three.
+template <int T>
+constexpr int tile_waves() { return T == 8 ? 3 : (T == 4 ? 5 : 8); }
+
+// blockIdx.y is the prime.  The waves of a group take a wm x wn patch of tiles
+// at the same 64 points, so its A rows and B columns come from L1 after their
+// first use; groups on one XCD (blockIdx.x mod 8) share the points, so the
+// operands of 64 points are read into one L2 only.
+template <int T>
+__global__ void __launch_bounds__(256, tile_waves<T>()) pw_tiled_kernel(const uint32_t *__restrict__ A, const uint32_t *__restrict__ B,
+                                                       uint32_t *__restrict__ C, int m, int k, int n, size_t npts,
+                                                       int wn, int tiles_m, int tiles_n, unsigned patches,
+                                                       unsigned patches_n, PlainPrimes<PlainSConst> primes)
+{
+    const unsigned i = blockIdx.y, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned wm = (blockDim.x >> 6) / wn, runs = (unsigned)(npts >> 6), nb = runs < 8 ? runs : 8;
+    const unsigned low = blockIdx.x % nb, g = blockIdx.x / nb, patch = g % patches, run = g / patches * nb + low;
+    const int ti = (int)(patch / patches_n * wm + wave / wn), tj = (int)(patch % patches_n * wn + wave % wn);
+    if (ti >= tiles_m || tj >= tiles_n) return;
+    pw_tile<T, tile_ahead<T>()>(A + (size_t)i * m * k * npts, B + (size_t)i * k * n * npts,
+                                C + (size_t)i * m * n * npts, m, k, n, npts, primes.p[i], primes.pc[i],
+                                run * 64 + (threadIdx.x & 63), ti * T, tj * T);
 }
 
 // Persistent work-queue form over the items of a batch: each workgroup takes
 // 256 points of one output tile of one job at a time.
-__global__ void __launch_bounds__(256) batch_pointwise_kernel(const BatchJob *__restrict__ jobs,
-                                                              const PwItem *__restrict__ items, uint32_t nitems,
-                                                              uint32_t *counter)
+__global__ void __launch_bounds__(256, tile_waves<8>()) batch_pointwise_kernel(const BatchJob *__restrict__ jobs,
+                                                                               const PwItem *__restrict__ items,
+                                                                               uint32_t nitems, uint32_t *counter)
 {
     __shared__ uint32_t item_sh;
     for (;;) {
@@ -119,16 +226,16 @@ __global__ void __launch_bounds__(256) batch_pointwise_kernel(const BatchJob *__
         const PwItem w = items[it];
         const BatchJob &J = jobs[w.job];
         const size_t npts = (size_t)1 << J.L;
-        const size_t t = (size_t)w.pt0 + threadIdx.x;
+        const uint32_t t = w.pt0 + threadIdx.x;
         const uint32_t *A = global_ptr(J.ahat), *B = global_ptr(J.bhat);
         uint32_t *Cp = global_ptr(J.chat);
         if (t < npts) {
             if (J.tile == 0)
-                pw_plain_body<2, 2>(A, B, Cp, J.m, J.k, J.n, npts, J.p, J.pc, t, w.ti * 2, w.tj * 2);
+                pw_tile<2, tile_ahead<2>()>(A, B, Cp, J.m, J.k, J.n, npts, J.p, J.pc, t, w.ti * 2, w.tj * 2);
             else if (J.tile == 1)
-                pw_plain_body<4, 4>(A, B, Cp, J.m, J.k, J.n, npts, J.p, J.pc, t, w.ti * 4, w.tj * 4);
+                pw_tile<4, tile_ahead<4>()>(A, B, Cp, J.m, J.k, J.n, npts, J.p, J.pc, t, w.ti * 4, w.tj * 4);
             else
-                pw_plain_body<8, 8>(A, B, Cp, J.m, J.k, J.n, npts, J.p, J.pc, t, w.ti * 8, w.tj * 8);
+                pw_tile<8, tile_ahead<8>()>(A, B, Cp, J.m, J.k, J.n, npts, J.p, J.pc, t, w.ti * 8, w.tj * 8);
         }
     }
 }
@@ -699,38 +806,70 @@ hipError_t launch_zero_counters(uint32_t *counters, int n, hipStream_t s)
     return hipGetLastError();
 }
 
-template <int T>
-static hipError_t plain_launch(const uint32_t *A, const uint32_t *B, uint32_t *C, size_t m, size_t k, size_t n,
-                               size_t npts, unsigned r, const PlainPrimes &primes, hipStream_t s)
+template <class Const, class F>
+static PlainPrimes<Const> plain_primes(unsigned r, const uint32_t *p, const uint32_t *scale, F make)
 {
-    const size_t tiles = ((m + T - 1) / T) * ((n + T - 1) / T), items = tiles * npts;
-    // groups of one wave spread a few waves over more CUs
-    const unsigned block = items * r < (size_t)device_cus() * 512 ? 64 : 256;
-    const size_t blocks = (items + block - 1) / block;
-    if (tiles > 0x7fffffff || blocks > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(pw_plain_kernel<T>, dim3((unsigned)blocks, r), dim3(block), 0, s, A, B, C, (int)m, (int)k, (int)n,
-                       npts, (unsigned)__builtin_ctzll(npts), items, primes);
-    return hipGetLastError();
+    PlainPrimes<Const> primes{};
+    for (unsigned i = 0; i < r; ++i) {
+        primes.p[i] = p[i];
+        primes.pc[i] = make(p[i], scale[i]);
+    }
+    return primes;
 }
 
 hipError_t launch_pointwise_plain(const uint32_t *A, const uint32_t *B, uint32_t *C, size_t m, size_t k, size_t n,
-                                  size_t npts, unsigned r, const uint32_t *p, const PlainConst *pc, hipStream_t s)
+                                  size_t npts, unsigned r, const uint32_t *p, const uint32_t *scale, hipStream_t s)
 {
     if (r == 0 || r > (unsigned)kMultiPrimes || (npts & (npts - 1))) return hipErrorInvalidValue;
-    PlainPrimes primes;
-    for (unsigned i = 0; i < (unsigned)kMultiPrimes; ++i) {
-        primes.p[i] = i < r ? p[i] : 0;
-        primes.pc[i] = i < r ? pc[i] : PlainConst{};
-    }
+    const auto items = [&](size_t T) { return ((m + T - 1) / T) * ((n + T - 1) / T) * npts; };
+    // 2x2 tiles where 4x4 ones would leave CUs with fewer than eight waves
+    const bool wide = items(4) * r >= 512 * (size_t)device_cus();
+    const size_t blocks = (items(wide ? 4 : 2) + 255) / 256;
+    if (items(2) / npts > 0x7fffffff || blocks > 0x7fffffff) return hipErrorInvalidValue;
+    const unsigned lg = (unsigned)__builtin_ctzll(npts);
+    const PlainPrimes<PlainConst> primes = plain_primes<PlainConst>(r, p, scale, plain_const);
+    if (wide)
+        hipLaunchKernelGGL(pw_plain_kernel<4>, dim3((unsigned)blocks, r), dim3(256), 0, s, A, B, C, (int)m, (int)k,
+                           (int)n, npts, lg, items(4), primes);
+    else
+        hipLaunchKernelGGL(pw_plain_kernel<2>, dim3((unsigned)blocks, r), dim3(256), 0, s, A, B, C, (int)m, (int)k,
+                           (int)n, npts, lg, items(2), primes);
+    return hipGetLastError();
+}
+
+// Whole waves of points, and the lane's byte offset in 32 bits.
+bool pointwise_tiled(size_t npts) { return npts >= 64 && npts <= ((size_t)1 << 29); }
+
+template <int T>
+static hipError_t tiled_launch(const uint32_t *A, const uint32_t *B, uint32_t *C, size_t m, size_t k, size_t n,
+                               size_t npts, unsigned r, const uint32_t *p, const uint32_t *scale, hipStream_t s)
+{
+    const size_t tm = (m + T - 1) / T, tn = (n + T - 1) / T;
+    // groups of one wave where there are few, to spread them over the CUs
+    const bool few = tm * tn * (npts / 64) * r < 8 * (size_t)device_cus();
+    const size_t waves = few ? 1 : 4, wn = few ? 1 : (tm == 1 ? 4 : (tn == 1 ? 1 : 2)), wm = waves / wn;
+    const size_t pn = (tn + wn - 1) / wn, patches = (tm + wm - 1) / wm * pn, blocks = patches * (npts / 64);
+    if (blocks > 0x7fffffff) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(pw_tiled_kernel<T>, dim3((unsigned)blocks, r), dim3((unsigned)(64 * waves)), 0, s, A, B, C,
+                       (int)m, (int)k, (int)n, npts, (int)wn, (int)tm, (int)tn, (unsigned)patches, (unsigned)pn,
+                       plain_primes<PlainSConst>(r, p, scale, plain_s_const));
+    return hipGetLastError();
+}
+
+hipError_t launch_pointwise_tiled(const uint32_t *A, const uint32_t *B, uint32_t *C, size_t m, size_t k, size_t n,
+                                  size_t npts, unsigned r, const uint32_t *p, const uint32_t *scale, hipStream_t s)
+{
+    if (r == 0 || r > (unsigned)kMultiPrimes || (npts & (npts - 1)) || !pointwise_tiled(npts))
+        return hipErrorInvalidValue;
     // the widest tile that still gives every CU eight waves: a wide tile re-reads
     // less, a narrow one fills the chip.  Whole products, us, with the 8x8 / 4x4 /
-    // 2x2 tile: 10x20x30 at 2^12 points 53 / 43 / 46; 32^3 at 2^11 66 / 51 / 57, at
-    // 2^13 117 / 121 / 174; 48^3 at 2^10 77 / 61 / 73; 16^3 at 2^8 32 / 22 / 22.
+    // 2x2 tile: 24^3 at 2^12 points 53 / 51 / 54; 64^2x32 at 2^11 95 / 81 / 98, at 2^12
+    // 147 / 150 / 186; 64^3 at 2^10 80 / 68 / 86, at 2^12 230 / 240 / 322.
     const size_t full = 8 * (size_t)device_cus();
-    const auto waves = [&](size_t T) { return ((m + T - 1) / T) * ((n + T - 1) / T) * npts / 64 * r; };
-    if (waves(8) >= full) return plain_launch<8>(A, B, C, m, k, n, npts, r, primes, s);
-    if (waves(4) >= full) return plain_launch<4>(A, B, C, m, k, n, npts, r, primes, s);
-    return plain_launch<2>(A, B, C, m, k, n, npts, r, primes, s);
+    const auto waves = [&](size_t T) { return ((m + T - 1) / T) * ((n + T - 1) / T) * (npts / 64) * r; };
+    if (waves(8) >= full) return tiled_launch<8>(A, B, C, m, k, n, npts, r, p, scale, s);
+    if (waves(4) >= full) return tiled_launch<4>(A, B, C, m, k, n, npts, r, p, scale, s);
+    return tiled_launch<2>(A, B, C, m, k, n, npts, r, p, scale, s);
 }
 
 size_t limb_block_bytes(size_t rows, size_t kdim) { return rpad_of(rows) * kpad_of(kdim) * 4; }

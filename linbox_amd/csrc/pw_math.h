@@ -107,8 +107,10 @@ struct PlainSConst {
     uint32_t c0, c0p, c1, c1p;  // scale and 2^32 scale mod p, with Shoup constants
     uint32_t f60;               // 2^60 mod p
     uint64_t off;               // multiple of p, >= 2^63
+    uint32_t every;             // products between folds for this p: the largest n with
+                                // 2^60 + 2^34 + n floor(p/2)^2 < 2^63, at most 64
 };
-constexpr uint32_t kPlainSFold = 6;
+constexpr uint32_t kPlainSFold = 6;  // for every p < 2^31
 
 inline PlainSConst plain_s_const(uint32_t p, uint32_t scale)
 {
@@ -121,6 +123,9 @@ inline PlainSConst plain_s_const(uint32_t p, uint32_t scale)
     pc.f60 = (uint32_t)(((uint64_t)1 << 60) % p);
     const uint64_t two63 = (uint64_t)1 << 63;
     pc.off = ((two63 + p - 1) / p) * p;
+    const uint64_t half = p / 2, room = two63 - ((uint64_t)1 << 60) - ((uint64_t)1 << 34) - 1;
+    const uint64_t most = half ? room / (half * half) : 64;
+    pc.every = (uint32_t)(most > 64 ? 64 : most);
     return pc;
 }
 

@@ -71,6 +71,23 @@ uint32_t lbx_test_plain_s_dot(const uint32_t *a, const uint32_t *b, int n, uint3
     return plain_s_finish(acc, p, pc);
 }
 
+// The tiled plain form: the same with the fold period of this p.
+uint32_t lbx_test_plain_s_every(uint32_t p) { return plain_s_const(p, 1).every; }
+uint32_t lbx_test_plain_s_dot_every(const uint32_t *a, const uint32_t *b, int n, uint32_t p, uint32_t scale)
+{
+    const PlainSConst pc = plain_s_const(p, scale);
+    int64_t acc = 0;
+    uint32_t cnt = 0;
+    for (int q = 0; q < n; ++q) {
+        acc += (int64_t)centre(a[q], p) * centre(b[q], p);
+        if (++cnt == pc.every) {
+            cnt = 0;
+            acc = plain_s_fold(acc, pc);
+        }
+    }
+    return plain_s_finish(acc, p, pc);
+}
+
 int32_t lbx_test_centre(uint32_t x, uint32_t p) { return centre(x, p); }
 }
 

@@ -239,3 +239,23 @@ def test_planted_mistake_is_caught(lib):
     d = [t - 256 if t >= 128 else t for t in d]
     c = x - p
     assert sum(t << (8 * s) for s, t in enumerate(d)) != c
+
+
+@pytest.mark.parametrize("p", [3, 17, 97, 12289, 167772161, 998244353, 2013265921, 2113929217, 2147483647])
+def test_plain_signed_fold_period(lib, p):
+    """The tiled plain form folds every `every` products, the most that fit for
+    this p: the documented bound, and the largest products of either sign over
+    lengths around multiples of it."""
+    lib.lbx_test_plain_s_every.argtypes = [ctypes.c_uint32]
+    lib.lbx_test_plain_s_every.restype = ctypes.c_uint32
+    lib.lbx_test_plain_s_dot_every.argtypes = lib.lbx_test_plain_s_dot.argtypes
+    lib.lbx_test_plain_s_dot_every.restype = ctypes.c_uint32
+    every = lib.lbx_test_plain_s_every(p)
+    assert 6 <= every <= 64
+    used = lambda n: (1 << 60) + (1 << 34) + n * (p // 2) ** 2  # noqa: E731
+    assert used(every) < 1 << 63 and (every == 64 or used(every + 1) >= (1 << 63) - 1)
+    h, lo = p // 2, p // 2 + 1
+    for n in [1, every - 1, every, every + 1, 3 * every, 4096, 4097]:
+        for (x, y) in [(lo, lo), (h, lo), (h, h)]:
+            a, b = (ctypes.c_uint32 * n)(*([x] * n)), (ctypes.c_uint32 * n)(*([y] * n))
+            assert lib.lbx_test_plain_s_dot_every(a, b, n, p, 1) == n * x * y % p, (p, n, x, y)
