@@ -37,39 +37,52 @@ struct InvArgs {
 
 // One whole forward transform per TP threads.  Input coefficient t is
 // coefficient t of the view, or rev-1-t of it when rev != 0 (the view has at
-// most rev coefficients then), zero where that is outside the view.
-template <int L, bool HALFZERO>
-__device__ __forceinline__ void forward_entry(const DevView &in, size_t rev, size_t e, bool active,
+// most rev coefficients then), zero where that is outside the view.  One body
+// serves every layout (a stride) and both zero paddings (only the first stage
+// differs, behind a uniform branch): with a body for each the kernel is several
+// times as long, and a launch of few groups waits for its instructions (800
+// entries at 2^12 points: 21.0 us against 19.2 here; 57344 at 2^11: 164 against 149).
+template <int L>
+__device__ __forceinline__ void forward_entry(const DevView &in, size_t rev, size_t e, bool active, bool halfzero,
                                               const uint2 *__restrict__ tw, uint32_t p, uint32_t h,
                                               uint32_t *__restrict__ out, int tp, uint32_t *lds)
 {
     using C = Cfg<L>;
     constexpr int RP0 = C::RLOG;
     // input coefficients [lo, hi) are inside the view
-    const size_t lo = rev ? rev - in.size : 0, hi = rev ? rev : in.size;
-    const size_t ein = active ? e : 0;
-    uint32_t x[C::R];
-    if (in.layout == 0) {
-        const uint32_t *src = in.base + ein * in.stor + in.shift + (rev ? rev - 1 : 0);
-#pragma unroll
-        for (int u = 0; u < (C::R >> RP0); ++u)
-#pragma unroll
-            for (int q = 0; q < (1 << RP0); ++q) {
-                const int t = elem<L, L - RP0, RP0>(tp, u, q);
-                const bool in_range = active && (size_t)t >= lo && (size_t)t < hi;
-                x[u * (1 << RP0) + q] = in_range ? src[rev ? -t : t] : 0u;
-            }
-    } else {
-#pragma unroll
-        for (int u = 0; u < (C::R >> RP0); ++u)
-#pragma unroll
-            for (int q = 0; q < (1 << RP0); ++q) {
-                const size_t t = (size_t)elem<L, L - RP0, RP0>(tp, u, q);
-                const bool in_range = active && t >= lo && t < hi;
-                x[u * (1 << RP0) + q] = in_range ? in.base[view_index(in, ein, rev ? rev - 1 - t : t)] : 0u;
-            }
+    const int lo = (int)(rev ? rev - in.size : 0), hi = (int)min(rev ? rev : in.size, (size_t)C::N);
+    const size_t first = in.shift + (rev ? rev - 1 : 0);
+    size_t stride = 1, base = (active ? e : 0) * in.stor;
+    if (in.layout == 1) {
+        stride = in.rows * in.cols;
+        base = active ? e : 0;
+    } else if (in.layout == 2) {
+        const uint32_t cols = (uint32_t)in.cols, row = (uint32_t)(active ? e : 0) / cols;
+        stride = in.cols;
+        base = (size_t)row * in.cols * in.stor + ((uint32_t)(active ? e : 0) - row * cols);
     }
-    dif_passes<L, 0, L, HALFZERO>(x, lds, tp, tw, p);
+    const uint32_t *src = in.base + base + first * stride;
+    const ptrdiff_t step = rev ? -(ptrdiff_t)stride : (ptrdiff_t)stride;
+    uint32_t x[C::R];
+#pragma unroll
+    for (int u = 0; u < (C::R >> RP0); ++u)
+#pragma unroll
+        for (int q = 0; q < (1 << RP0); ++q) {
+            const int t = elem<L, L - RP0, RP0>(tp, u, q);
+            x[u * (1 << RP0) + q] = active && t >= lo && t < hi ? src[t * step] : 0u;
+        }
+    if (halfzero)
+        dif_pass<L, 0, RP0, true, 0, 1>(x, tp, tw, p);
+    else
+        dif_pass<L, 0, RP0, false, 0, 1>(x, tp, tw, p);
+    dif_pass<L, 0, RP0, false, 1, RP0>(x, tp, tw, p);
+    if constexpr (RP0 < L) {
+        constexpr int NRP = (L - RP0) < C::RLOG ? (L - RP0) : C::RLOG;
+        scatter<L, L - RP0, RP0>(x, lds, tp);
+        __syncthreads();
+        gather<L, L - RP0 - NRP, NRP>(x, lds, tp);
+        dif_passes<L, RP0, L, false>(x, lds, tp, tw, p);
+    }
     if (active) dif_store<L, true>(x, tp, out + e * C::N, p, h);
 }
 
@@ -89,10 +102,8 @@ __global__ void __launch_bounds__(Cfg<L>::BLOCK) multi_dif_kernel(FwdArgs A)
     const size_t e = (size_t)(isa ? blockIdx.x : blockIdx.x - A.ga) * C::G + pib;
     uint32_t *lds = lds_all + pib * C::STRIDE;
     const uint32_t h = A.centre ? A.p[i] >> 1 : ~0u;
-    if ((rev ? rev : in.size) * 2 <= (size_t)C::N)
-        forward_entry<L, true>(in, rev, e, e < entries, global_ptr(tw), A.p[i], h, out, tp, lds);
-    else
-        forward_entry<L, false>(in, rev, e, e < entries, global_ptr(tw), A.p[i], h, out, tp, lds);
+    forward_entry<L>(in, rev, e, e < entries, (rev ? rev : in.size) * 2 <= (size_t)C::N, global_ptr(tw), A.p[i], h, out,
+                     tp, lds);
 }
 
 template <int L>

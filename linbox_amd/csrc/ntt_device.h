@@ -116,7 +116,8 @@ __device__ __forceinline__ void gather(uint32_t (&x)[Cfg<L>::R], const uint32_t 
 // DIF stages S0..S0+RP-1 (span N>>(s+1) at stage s) on the registers.
 // tw_off: the twiddle table starts tw_off entries into the pow_w layout (an
 // LDS copy of the tail of the table).
-template <int L, int S0, int RP, bool HALFZERO>
+// Only the pass's stages [ST0, ST1) where given.
+template <int L, int S0, int RP, bool HALFZERO, int ST0 = 0, int ST1 = RP>
 __device__ __forceinline__ void dif_pass(uint32_t (&x)[Cfg<L>::R], int tp, const uint2 *__restrict__ tw, uint32_t p,
                                          int tw_off = 0)
 {
@@ -126,7 +127,7 @@ __device__ __forceinline__ void dif_pass(uint32_t (&x)[Cfg<L>::R], int tp, const
     for (int u = 0; u < NG; ++u) {
         const int off = (tp + u * TP) & ((1 << HL) - 1);
 #pragma unroll
-        for (int st = 0; st < RP; ++st) {
+        for (int st = ST0; st < ST1; ++st) {
             const int s = S0 + st;
             const int half = 1 << (RP - 1 - st);
             const uint2 *tws = tw + (N - (N >> s) - tw_off);
