@@ -239,18 +239,6 @@ int choose_method(int method, size_t m, size_t k, size_t n, unsigned L)
     return big ? LBX_METHOD_INT8_MFMA : LBX_METHOD_PLAIN_U64;
 }
 
-// The plain form's operand layout: polfirst transform output (one point per
-// lane), which the tiled pointwise kernel reads at a cost that no longer pays
-// for split transforms at any size (entry-major / point-major, us: 96^3 at 2^13
-// points 1208 / 2175, 128^3 at 2^8 90 / 125, at 2^13 2403 / 2579, 160^3 at 2^13
-// 4544 / 9193).  LBX_PLAIN_LAYOUT = "point" takes the point-major form
-// (measurement and tests).
-bool plain_point_major()
-{
-    const char *e = std::getenv("LBX_PLAIN_LAYOUT");
-    return e && !std::strcmp(e, "point");
-}
-
 // Bytes of head -> tail intermediate per chunk.  The default, 2 GiB, gives one
 // chunk per operand up to 128x128 entries of 2^14 points: smaller chunks
 // measured slower there (the hand-off through the last-level cache gains less
@@ -395,7 +383,7 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
     if (L > (unsigned)kMaxLog) return LBX_ERR_UNSUPPORTED;
     method = choose_method(method, m, k, n, L);
     const bool int8 = method == LBX_METHOD_INT8_MFMA;
-    const bool split = L >= 8 && L <= (unsigned)kMaxLdsLog && (int8 || plain_point_major());
+    const bool split = L >= 8 && L <= (unsigned)kMaxLdsLog && int8;
     // whole transforms of both operands in one launch (a middle product's
     // reversal included)
     const bool fused = !split && !int8 && L >= 1 && L <= (unsigned)kMaxLdsLog;
@@ -497,9 +485,8 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
     const bool timing = ws.timing();
     Stages st(ctx, s, timing);
     if (split) {
-        // split transforms: the last six forward stages write per-point blocks
-        // (digits for the INT8 form, words for the plain one) and the first
-        // six inverse stages read the point-major product
+        // split transforms: the last six forward stages write per-point digit
+        // blocks and the first six inverse stages read the point-major product
         const unsigned BL = kSplitBL;
         uint32_t *slot[2] = {(uint32_t *)scr, (uint32_t *)scr + (nslots - 1) * slot_words};
         Pipe fp{ctx, s, fwd_pipe};
@@ -521,25 +508,19 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
                 LBX_TRY(fp.handoff(chunk));
                 {
                     KernelTimer kt(ctx, fp.consumer(),
-                                   int8 ? (op == 0 ? "kernel dif_tail_limbs a" : "kernel dif_tail_limbs b")
-                                        : (op == 0 ? "kernel dif_tail_words a" : "kernel dif_tail_words b"),
-                                   timing);
+                                   op == 0 ? "kernel dif_tail_limbs a" : "kernel dif_tail_limbs b", timing);
                     LBX_TRY_HIP(launch_dif_tail_limbs(buf, (uint8_t *)(op == 0 ? al : bl), rows, r0, nr, valid, k,
-                                                      op == 0, L, BL, op == 0 ? twa : twb, p, fp.consumer(), int8));
+                                                      op == 0, L, BL, op == 0 ? twa : twb, p, fp.consumer()));
                 }
                 LBX_TRY(fp.done(chunk));
             }
         }
         LBX_TRY(fp.end(chunk));
         st.mark("direct FFT_DIF");
-        if (int8) {
+        {
             KernelTimer kt(ctx, s, "kernel pw_mfma", timing);
             LBX_TRY_HIP(launch_pointwise_mfma((const uint8_t *)al, (const uint8_t *)bl, (uint32_t *)cmat, m, k, n, N,
                                               p, inv_n, s));
-        } else {
-            KernelTimer kt(ctx, s, "kernel pw_plain_pm", timing);
-            LBX_TRY_HIP(launch_pointwise_plain_pm((const uint32_t *)al, (const uint32_t *)bl, (uint32_t *)cmat, m, k,
-                                                  n, N, p, inv_n, s));
         }
         st.mark("Pointwise mult");
         Pipe ip{ctx, s, inv_pipe};

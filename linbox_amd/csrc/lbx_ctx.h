@@ -272,8 +272,6 @@ lbx_status noalloc_attach(int device);
 void mp_release(lbx_ctx *ctx);
 // Frees the batch plans (graphs, descriptors) cached in a context.
 void batch_release(lbx_ctx *ctx);
-// Whether the plain form takes point-major operands (split transforms).
-bool plain_point_major();
 // Whether a view of `entries` x `count` coefficients that is not polfirst goes
 // through a polfirst copy in a product with 2^L points.
 bool copies_to_polfirst(const DevView &v, size_t entries, size_t count, unsigned L);

@@ -89,7 +89,7 @@ struct EntryMap {
     }
 };
 
-// Split transforms for the point-major pointwise form, with blocks of 2^BL
+// Split transforms for the INT8 pointwise form, with blocks of 2^BL
 // points (BL = kSplitBL, BL + 2 <= L <= 15):
 // forward head = DIF stages [0, L-BL) per entry, written block-major:
 //                word w of block j of output row l (input entry map(l)) at
@@ -110,11 +110,9 @@ constexpr unsigned kSplitBL = 6;
 int device_cus();
 hipError_t launch_ntt_forward_head(const DevView &in, size_t entries, const EntryMap &map, unsigned L, unsigned BL,
                                    const uint2 *tw, uint32_t p, uint32_t *out, hipStream_t s);
-// With limbs = false the tail writes the centred values (int32) instead of
-// their digits, in the same block geometry ([rpad][kpad] words per point).
 hipError_t launch_dif_tail_limbs(const uint32_t *X, uint8_t *Y, size_t rows_total, size_t row0, size_t rows_chunk,
                                  size_t rows_valid, size_t kdim, bool row_major, unsigned L, unsigned BL,
-                                 const uint2 *tw, uint32_t p, hipStream_t s, bool limbs = true);
+                                 const uint2 *tw, uint32_t p, hipStream_t s);
 hipError_t launch_dit_head(const uint32_t *Cm, size_t entries, size_t e_first, size_t e_count, unsigned L,
                            unsigned BL, const uint2 *tw, uint32_t p, uint32_t *Y, hipStream_t s);
 hipError_t launch_ntt_inverse_tail(const uint32_t *in, size_t entries, unsigned L, unsigned BL, const uint2 *tw,
@@ -172,11 +170,6 @@ hipError_t launch_to_limbs(const uint32_t *X, uint8_t *Y, size_t rows, size_t kd
 // INT8-MFMA pointwise: per point, C[t][i*n+j] (point-major) from limb blocks.
 hipError_t launch_pointwise_mfma(const uint8_t *Al, const uint8_t *Bl, uint32_t *Cmat, size_t m, size_t k,
                                  size_t n, size_t npts, uint32_t p, uint32_t scale, hipStream_t s);
-// Plain-form pointwise on point-major blocks of centred int32 values (the
-// geometry of limb_block_bytes: A as [rpad(m)][kpad(k)], B^T as [rpad(n)][kpad(k)]
-// words per point, padding zero): C[t][i*n+j] = scale * sum_q A[i][q] B^T[j][q] mod p.
-hipError_t launch_pointwise_plain_pm(const uint32_t *Aw, const uint32_t *Bw, uint32_t *Cmat, size_t m, size_t k,
-                                     size_t n, size_t npts, uint32_t p, uint32_t scale, hipStream_t s);
 // Point-major [t][e] -> polfirst [e][t] transpose of `entries` x npts words.
 hipError_t launch_point_to_entry(const uint32_t *X, uint32_t *Y, size_t entries, size_t npts, hipStream_t s);
 
