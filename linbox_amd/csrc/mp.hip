@@ -444,16 +444,17 @@ __global__ void __launch_bounds__(128) mp_crt_kernel(const uint32_t *__restrict_
 // 2^(32 NW).  The group's words leave through LDS where they are contiguous.
 //
 // Constants: per prime p, (M/p)^-1 mod p with its Shoup constant, floor(2^56 /
-// p), NW words of M/p; then NW words of -M; then (MOD) off, s and NW words of Q.
+// p), NW words of M/p; then NW words of -M; then (MOD) off, s, the reciprocal of
+// Q's top word (div21_inverse) and NW words of Q.
 // Bound by the multiply-adds: 2047 x 1024 coefficients, 14 primes, 6 words: 140 us
-// on mixed-radix digits, 50 us here (57 with the carries rebuilt from comparisons and eight words for six).
+// on mixed-radix digits, 47 us here (57 with the carries rebuilt from comparisons and eight words for six).
 struct CrtBlock {
     static constexpr int kHead = 4;
     int r, nw;
     __host__ __device__ int prime(int i) const { return i * (kHead + nw); }
     __host__ __device__ int neg() const { return r * (kHead + nw); }
     __host__ __device__ int sh() const { return neg() + nw; }
-    __host__ __device__ int Q() const { return sh() + 2; }
+    __host__ __device__ int Q() const { return sh() + 3; }
 };
 constexpr int kCrtMaxPrimes = 32;
 constexpr uint32_t kCrtMinPrime = 1u << 24;
@@ -522,7 +523,7 @@ __global__ void __launch_bounds__(128) crt_direct_kernel(const uint32_t *__restr
         uint32_t q[NW];
 #pragma unroll
         for (int l = 0; l < NW; ++l) q[l] = K[lay.Q() + l];
-        knuth_rem2<NW>(acc, q, div21_inverse(q[NW - 1]));  // Q is normalized: its top word has its top bit set
+        knuth_rem2<NW>(acc, q, K[lay.sh() + 2]);  // Q is normalized: its top word has its top bit set
         // words off.. of acc >> sh; the words of P's leading zero limbs are zero
 #pragma unroll
         for (int l = 0; l < NW; ++l)
@@ -822,6 +823,7 @@ lbx_status get_plan(lbx_ctx *ctx, const uint32_t *Pw, int nl, size_t k, size_t m
         K[plan->crt_off + cb.sh()] = (uint32_t)off;
         K[plan->crt_off + cb.sh() + 1] = (uint32_t)sh;
         place(P, &K[plan->crt_off + cb.Q()]);
+        K[plan->crt_off + cb.sh() + 2] = div21_inverse(K[plan->crt_off + cb.Q() + nw - 1]);
     }
     hipError_t e = hipMalloc(&plan->d_const, K.size() * 4);
     if (e == hipSuccess) e = hipMemcpy(plan->d_const, K.data(), K.size() * 4, hipMemcpyHostToDevice);
