@@ -379,8 +379,7 @@ def run_configs(reps=10):
     C = PolynomialMatrix(dim, dim, 2 * sa - 1, data=dc, nlimbs=nl)
     ms = timed(lambda: lbx.mul_mp(Pm, C, A, B, ctx=ctx, stream=stream.value))
     out["32x32_deg1023_P192"] = {"ms": round(ms, 4), "products_per_s": round(1e3 / ms, 1), "fft_primes": 14,
-                                 "pointwise": "auto: plain uint64 form, the 14 per-prime products as one call "
-                                              "of the batch kernels"}
+                                 "pointwise": "auto: plain form, the 14 per-prime products in shared launches"}
     ms = timed(lambda: lbx.mul_mp(Pm, C, A, B, ctx=ctx, method=lbx.METHOD_INT8_MFMA, stream=stream.value))
     out["32x32_deg1023_P192_int8"] = {"ms": round(ms, 4), "products_per_s": round(1e3 / ms, 1), "fft_primes": 14,
                                       "pointwise": "int8_mfma per prime (14 single-prime products)"}
