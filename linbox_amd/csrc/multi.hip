@@ -57,9 +57,9 @@ __device__ __forceinline__ void forward_entry(const DevView &in, size_t rev, siz
         stride = in.rows * in.cols;
         base = active ? e : 0;
     } else if (in.layout == 2) {
-        const uint32_t cols = (uint32_t)in.cols, row = (uint32_t)(active ? e : 0) / cols;
+        const size_t row = (active ? e : 0) / in.cols;
         stride = in.cols;
-        base = (size_t)row * in.cols * in.stor + ((uint32_t)(active ? e : 0) - row * cols);
+        base = row * in.cols * in.stor + ((active ? e : 0) - row * in.cols);
     }
     const uint32_t *src = in.base + base + first * stride;
     const ptrdiff_t step = rev ? -(ptrdiff_t)stride : (ptrdiff_t)stride;

@@ -121,33 +121,32 @@ __global__ void __launch_bounds__(256) pw_plain_kernel(const uint32_t *__restric
 // 2^11 points 180 -> 120 us, 5 of 24^3 at 2^11 38 -> 24 us; with the loads ahead it
 // is bound by its vector instructions, 64 multiply-adds a step of some 84.
 template <int T, int D>
-__device__ __forceinline__ void pw_tile(const uint32_t *__restrict__ A, const uint32_t *__restrict__ B,
-                                        uint32_t *__restrict__ C, int m, int k, int n, size_t npts, uint32_t p,
-                                        const PlainSConst &pc, uint32_t t, int i0, int j0)
+__device__ __forceinline__ void pw_accumulate(const uint32_t *__restrict__ A, const uint32_t *__restrict__ B, int m,
+                                              int k, int k0, int k1, int n, size_t npts, const PlainSConst &pc,
+                                              uint32_t t, int i0, int j0, int64_t (&acc)[T][T])
 {
     // uniform row and column bases of the next step to load
     const char *pa[T], *pb[T];
 #pragma unroll
-    for (int ii = 0; ii < T; ++ii) pa[ii] = (const char *)(A + (size_t)min(i0 + ii, m - 1) * k * npts);
+    for (int ii = 0; ii < T; ++ii) pa[ii] = (const char *)(A + ((size_t)min(i0 + ii, m - 1) * k + k0) * npts);
 #pragma unroll
-    for (int jj = 0; jj < T; ++jj) pb[jj] = (const char *)(B + (size_t)min(j0 + jj, n - 1) * npts);
+    for (int jj = 0; jj < T; ++jj) pb[jj] = (const char *)(B + ((size_t)k0 * n + min(j0 + jj, n - 1)) * npts);
     const uint32_t off = t * 4;
     const size_t step_a = npts * 4, step_b = (size_t)n * npts * 4;
     int32_t a[D][T], b[D][T];
-    int q_load = 0;
+    int q_load = k0;
     const auto load = [&](int d) {
 #pragma unroll
         for (int ii = 0; ii < T; ++ii) a[d][ii] = *(const int32_t *)(pa[ii] + off);
 #pragma unroll
         for (int jj = 0; jj < T; ++jj) b[d][jj] = *(const int32_t *)(pb[jj] + off);
         ++q_load;
-        const size_t sa = q_load < k ? step_a : 0, sb = q_load < k ? step_b : 0;
+        const size_t sa = q_load < k1 ? step_a : 0, sb = q_load < k1 ? step_b : 0;
 #pragma unroll
         for (int ii = 0; ii < T; ++ii) pa[ii] += sa;
 #pragma unroll
         for (int jj = 0; jj < T; ++jj) pb[jj] += sb;
     };
-    int64_t acc[T][T];
 #pragma unroll
     for (int ii = 0; ii < T; ++ii)
 #pragma unroll
@@ -155,10 +154,10 @@ __device__ __forceinline__ void pw_tile(const uint32_t *__restrict__ A, const ui
 #pragma unroll
     for (int d = 0; d < D; ++d) load(d);
     int since = 0;  // products since the last fold
-    for (int q0 = 0; q0 < k; q0 += D) {
+    for (int q0 = k0; q0 < k1; q0 += D) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-            if (q0 + d < k) {
+            if (q0 + d < k1) {
 #pragma unroll
                 for (int ii = 0; ii < T; ++ii)
 #pragma unroll
@@ -174,6 +173,15 @@ __device__ __forceinline__ void pw_tile(const uint32_t *__restrict__ A, const ui
             }
         }
     }
+}
+
+template <int T, int D>
+__device__ __forceinline__ void pw_tile(const uint32_t *__restrict__ A, const uint32_t *__restrict__ B,
+                                        uint32_t *__restrict__ C, int m, int k, int n, size_t npts, uint32_t p,
+                                        const PlainSConst &pc, uint32_t t, int i0, int j0)
+{
+    int64_t acc[T][T];
+    pw_accumulate<T, D>(A, B, m, k, 0, k, n, npts, pc, t, i0, j0, acc);
 #pragma unroll
     for (int ii = 0; ii < T; ++ii)
 #pragma unroll
@@ -208,6 +216,49 @@ __global__ void __launch_bounds__(256, tile_waves<T>()) pw_tiled_kernel(const ui
     pw_tile<T, tile_ahead<T>()>(A + (size_t)i * m * k * npts, B + (size_t)i * k * n * npts,
                                 C + (size_t)i * m * n * npts, m, k, n, npts, primes.p[i], primes.pc[i],
                                 run * 64 + (threadIdx.x & 63), ti * T, tj * T);
+}
+
+// The same tile with its inner dimension split over the kSplitK waves of a
+// group, for products too small to fill the chip with tiles: each wave sums its
+// part of the steps (a chain kSplitK times as short), the folded sums (below 2^60 +
+// 2^34 each, so four fit) meet in LDS and every wave finishes T^2 / kSplitK of the
+// outputs.
+constexpr int kSplitK = 4;
+template <int T>
+__global__ void __launch_bounds__(64 * kSplitK) pw_splitk_kernel(const uint32_t *__restrict__ A,
+                                                                 const uint32_t *__restrict__ B,
+                                                                 uint32_t *__restrict__ C, int m, int k, int n,
+                                                                 size_t npts, int tiles_n, unsigned tiles,
+                                                                 PlainPrimes<PlainSConst> primes)
+{
+    __shared__ int64_t part[kSplitK][T * T][64];
+    const unsigned i = blockIdx.y;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const unsigned runs = (unsigned)(npts >> 6), nb = runs < 8 ? runs : 8;
+    const unsigned low = blockIdx.x % nb, g = blockIdx.x / nb, tile = g % tiles, run = g / tiles * nb + low;
+    const int i0 = (int)(tile / tiles_n) * T, j0 = (int)(tile % tiles_n) * T;
+    const int per = (k + kSplitK - 1) / kSplitK, k0 = min(wave * per, k), k1 = min(k0 + per, k);
+    const uint32_t t = run * 64 + lane;
+    const PlainSConst &pc = primes.pc[i];
+    int64_t acc[T][T];
+    // a wave without steps loads the last one (in bounds) and sums nothing
+    pw_accumulate<T, tile_ahead<T>()>(A + (size_t)i * m * k * npts, B + (size_t)i * k * n * npts, m, k,
+                                      k0 < k1 ? k0 : k - 1, k0 < k1 ? k1 : k - 1, n, npts, pc, t, i0, j0, acc);
+#pragma unroll
+    for (int ii = 0; ii < T; ++ii)
+#pragma unroll
+        for (int jj = 0; jj < T; ++jj) part[wave][ii * T + jj][lane] = plain_s_fold(acc[ii][jj], pc);
+    __syncthreads();
+    uint32_t *Ci = C + (size_t)i * m * n * npts;
+#pragma unroll
+    for (int u = 0; u < T * T / kSplitK; ++u) {
+        const int e = wave * (T * T / kSplitK) + u, ii = e / T, jj = e % T;
+        int64_t sum = 0;
+#pragma unroll
+        for (int w = 0; w < kSplitK; ++w) sum += part[w][e][lane];
+        if (i0 + ii < m && j0 + jj < n)
+            Ci[((size_t)(i0 + ii) * n + j0 + jj) * npts + t] = plain_s_finish(sum, primes.p[i], pc);
+    }
 }
 
 // Persistent work-queue form over the items of a batch: each workgroup takes
@@ -751,6 +802,18 @@ hipError_t launch_pointwise_plain(const uint32_t *A, const uint32_t *B, uint32_t
 bool pointwise_tiled(size_t npts) { return npts >= 64 && npts <= ((size_t)1 << 29); }
 
 template <int T>
+static hipError_t splitk_launch(const uint32_t *A, const uint32_t *B, uint32_t *C, size_t m, size_t k, size_t n,
+                                size_t npts, unsigned r, const uint32_t *p, const uint32_t *scale, hipStream_t s)
+{
+    const size_t tn = (n + T - 1) / T, tiles = (m + T - 1) / T * tn, blocks = tiles * (npts / 64);
+    if (blocks > 0x7fffffff) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(pw_splitk_kernel<T>, dim3((unsigned)blocks, r), dim3(64 * kSplitK), 0, s, A, B, C, (int)m,
+                       (int)k, (int)n, npts, (int)tn, (unsigned)tiles,
+                       plain_primes<PlainSConst>(r, p, scale, plain_s_const));
+    return hipGetLastError();
+}
+
+template <int T>
 static hipError_t tiled_launch(const uint32_t *A, const uint32_t *B, uint32_t *C, size_t m, size_t k, size_t n,
                                size_t npts, unsigned r, const uint32_t *p, const uint32_t *scale, hipStream_t s)
 {
@@ -779,6 +842,14 @@ hipError_t launch_pointwise_tiled(const uint32_t *A, const uint32_t *B, uint32_t
     const auto waves = [&](size_t T) { return ((m + T - 1) / T) * ((n + T - 1) / T) * (npts / 64) * r; };
     if (waves(8) >= full) return tiled_launch<8>(A, B, C, m, k, n, npts, r, p, scale, s);
     if (waves(4) >= full) return tiled_launch<4>(A, B, C, m, k, n, npts, r, p, scale, s);
+    // too few tiles: from eight steps on the inner dimension is split, 4x4 tiles
+    // while that gives half the waves, 2x2 below.  Whole products, us, 2x2 unsplit /
+    // split rule: 64^3 at 2^6 points 25 / 22, at 2^8 38 / 33; 64^2x32 at 2^9 40 / 34;
+    // 16^3 at 2^9 21 / 20; 9x100x9 at 2^8 29 / 21; 3x300x5 at 2^10 60 / 32; 4x8x4 20 / 19.
+    if (k >= 8) {
+        if (2 * kSplitK * waves(4) >= full) return splitk_launch<4>(A, B, C, m, k, n, npts, r, p, scale, s);
+        return splitk_launch<2>(A, B, C, m, k, n, npts, r, p, scale, s);
+    }
     return tiled_launch<2>(A, B, C, m, k, n, npts, r, p, scale, s);
 }
 

@@ -616,3 +616,21 @@ def test_plain_whole_transforms(ctx, p, m, k, n, sa, sb):
     PolynomialMatrixMulDomain(p, ctx, method=lbx.METHOD_PLAIN_U64).mul(C, A, B)
     xs = [int(x) for x in rng.integers(0, p, 2)]
     assert check_by_evaluation(a, b, C.to_polfirst(), p, m, k, n, sa, sb, sa + sb - 1, xs)
+
+
+@pytest.mark.parametrize("m,k,n,sa,sb", [(2, 7, 3, 40, 30), (2, 8, 3, 40, 30), (5, 9, 6, 64, 65), (3, 300, 5, 33, 32),
+                                         (1, 13, 1, 200, 100), (20, 10, 17, 900, 140), (64, 64, 63, 130, 127)])
+@pytest.mark.parametrize("p", [2013265921, 998244353, 268435399])
+def test_plain_split_inner_dimension(ctx, p, m, k, n, sa, sb):
+    """Small plain products, whose inner dimension is split over the waves of a
+    group from eight steps on: parts of unequal length and empty ones, one prime
+    and three, operands of the largest centred size."""
+    rng = np.random.default_rng(m * k * n + sa)
+    a, b = rand(rng, p, m * k * sa).reshape(m * k, sa), rand(rng, p, k * n * sb).reshape(k * n, sb)
+    a[:, 0], b[:, 0] = p // 2, p // 2 + 1
+    C = PolynomialMatrix(m, n, sa + sb - 1)
+    say("plain split inner dimension", p, m, k, n, sa, sb)
+    PolynomialMatrixMulDomain(p, ctx, method=lbx.METHOD_PLAIN_U64).mul(
+        C, PolynomialMatrix.from_polfirst(a, m, k), PolynomialMatrix.from_polfirst(b, k, n))
+    xs = [int(x) for x in rng.integers(0, p, 2)]
+    assert check_by_evaluation(a, b, C.to_polfirst(), p, m, k, n, sa, sb, sa + sb - 1, xs)
