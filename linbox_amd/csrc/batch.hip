@@ -119,10 +119,14 @@ void tr_items_for(const BatchJob &J, uint32_t job, std::vector<TrItem> &out)
 void pw_items_for(const BatchJob &J, uint32_t job, std::vector<PwItem> &out)
 {
     const unsigned T = tile_dim(J.tile);
-    const uint32_t ti = (J.m + T - 1) / T, tj = (J.n + T - 1) / T, blocks = (((uint32_t)1 << J.L) + 255) / 256;
-    for (uint32_t b = 0; b < blocks; ++b)
-        for (uint32_t i = 0; i < ti; ++i)
-            for (uint32_t jj = 0; jj < tj; ++jj) out.push_back(PwItem{job, i, jj, b * 256});
+    const uint32_t tiles = ((J.m + T - 1) / T) * ((J.n + T - 1) / T), npts = (uint32_t)1 << J.L;
+    // four tiles at 64 points where there are four; the others at 256 points each,
+    // unless the transform has no more than 64
+    const uint32_t by_four = npts <= 64 ? tiles : tiles & ~3u;
+    for (uint32_t pt0 = 0; pt0 < npts; pt0 += 64)
+        for (uint32_t t0 = 0; t0 < by_four; t0 += 4) out.push_back(PwItem{job, t0, pt0, 0});
+    for (uint32_t pt0 = 0; pt0 < npts; pt0 += 256)
+        for (uint32_t t0 = by_four; t0 < tiles; ++t0) out.push_back(PwItem{job, t0, pt0, 1});
 }
 
 lbx_status upload(void **dst, const void *src, size_t bytes, hipStream_t s)

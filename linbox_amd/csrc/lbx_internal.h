@@ -209,9 +209,10 @@ struct MfmaItem {
 struct TrItem {
     uint32_t job, e0, t0, pad_;
 };
-// Pointwise work item: 256 points from pt0 of output tile (ti, tj).
+// Pointwise work item: 64 points from pt0 of output tiles tile0 .. tile0 + 3
+// (row-major), or 256 points of tile0 (one_tile).
 struct PwItem {
-    uint32_t job, ti, tj, pt0;
+    uint32_t job, tile0, pt0, one_tile;
 };
 constexpr int kBatchMinL = 4, kBatchMaxL = 13;
 constexpr int kBatchNttThreads = 512;
