@@ -30,6 +30,7 @@
 
 #include "lbx_ctx.h"
 #include "mp_div.h"
+#include "plan_key.h"
 
 namespace lbx {
 
@@ -751,8 +752,7 @@ lbx_status prime_products(lbx_ctx *ctx, const std::vector<uint32_t> &primes, con
 
 lbx_status get_plan(lbx_ctx *ctx, const uint32_t *Pw, int nl, size_t k, size_t minsz, unsigned lpts, MpPlan **out)
 {
-    std::string key((const char *)Pw, (size_t)nl * 4);
-    key += "|" + std::to_string(k) + "|" + std::to_string(minsz) + "|" + std::to_string(lpts);
+    const std::string key = mp_plan_key(Pw, nl, k, minsz, lpts);
     auto it = ctx->mp_plans.find(key);
     if (it != ctx->mp_plans.end()) {
         *out = it->second;
@@ -845,8 +845,7 @@ lbx_status get_plan(lbx_ctx *ctx, const uint32_t *Pw, int nl, size_t k, size_t m
 // p_i <= p, whose operands need the reduction of :143-146.
 lbx_status get_few_plan(lbx_ctx *ctx, uint32_t p, size_t k, size_t minsz, unsigned lpts, MpPlan **out)
 {
-    std::string key = "fp|" + std::to_string(p) + "|" + std::to_string(k) + "|" + std::to_string(minsz) + "|" +
-                      std::to_string(lpts);
+    const std::string key = few_plan_key(p, k, minsz, lpts);
     auto it = ctx->mp_plans.find(key);
     if (it != ctx->mp_plans.end()) {
         *out = it->second;
@@ -1157,9 +1156,7 @@ constexpr size_t kZzPlans = 64;
 
 lbx_status get_zz_plan(lbx_ctx *ctx, unsigned lab, size_t k, size_t minsz, unsigned lpts, int nl, int cl, MpPlan **out)
 {
-    const std::string prefix = "zz|";
-    const std::string key = prefix + std::to_string(lab) + "|" + std::to_string(k) + "|" + std::to_string(minsz) + "|" +
-                            std::to_string(lpts) + "|" + std::to_string(nl) + "|" + std::to_string(cl);
+    const std::string prefix = kZzPlanTag, key = zz_plan_key(lab, k, minsz, lpts, nl, cl);
     const auto it = ctx->mp_plans.find(key);
     if (it != ctx->mp_plans.end()) {
         *out = it->second;
