@@ -460,14 +460,58 @@ struct CrtBlock {
 constexpr int kCrtMaxPrimes = 32;
 constexpr uint32_t kCrtMinPrime = 1u << 24;
 
-// (over:sum) += t * w: one multiply-add with its carry out, which the compiler
-// would rebuild with a comparison.
-__device__ __forceinline__ void mad_carry(uint64_t &sum, uint32_t &over, uint32_t t, uint32_t w)
+// (over[i]:sum[i]) += t * w[i] for N columns: a multiply-add each with its carry
+// out, which the compiler would rebuild with comparisons.  A vector instruction may
+// read a carry two wait states after the one that wrote it at the earliest, and the
+// compiler does not look for that inside an asm block: the products of three or four
+// columns come first, then their carries,
+// with two or more instructions between;
+// two columns take one s_nop.
+template <int N>
+__device__ __forceinline__ void mad_carry(uint64_t *sum, uint32_t *over, uint32_t t, const uint32_t *w)
 {
-    asm("v_mad_u64_u32 %0, vcc, %2, %3, %0\n\tv_addc_co_u32_e32 %1, vcc, 0, %1, vcc"
-        : "+v"(sum), "+v"(over)
-        : "v"(t), "s"(w)
-        : "vcc");
+    static_assert(N >= 2 && N <= 4, "columns of one block");
+    uint64_t c0, c1, c2, c3;
+    if constexpr (N == 4) {
+        asm("v_mad_u64_u32 %0, %8, %12, %13, %0\n\t"
+            "v_mad_u64_u32 %1, %9, %12, %14, %1\n\t"
+            "v_mad_u64_u32 %2, %10, %12, %15, %2\n\t"
+            "v_mad_u64_u32 %3, %11, %12, %16, %3\n\t"
+            "v_addc_co_u32_e64 %4, %8, 0, %4, %8\n\t"
+            "v_addc_co_u32_e64 %5, %9, 0, %5, %9\n\t"
+            "v_addc_co_u32_e64 %6, %10, 0, %6, %10\n\t"
+            "v_addc_co_u32_e64 %7, %11, 0, %7, %11"
+            : "+&v"(sum[0]), "+&v"(sum[1]), "+&v"(sum[2]), "+&v"(sum[3]), "+&v"(over[0]), "+&v"(over[1]),
+              "+&v"(over[2]), "+&v"(over[3]), "=&s"(c0), "=&s"(c1), "=&s"(c2), "=&s"(c3)
+            : "v"(t), "s"(w[0]), "s"(w[1]), "s"(w[2]), "s"(w[3]));
+    } else if constexpr (N == 3) {
+        asm("v_mad_u64_u32 %0, %6, %9, %10, %0\n\t"
+            "v_mad_u64_u32 %1, %7, %9, %11, %1\n\t"
+            "v_mad_u64_u32 %2, %8, %9, %12, %2\n\t"
+            "v_addc_co_u32_e64 %3, %6, 0, %3, %6\n\t"
+            "v_addc_co_u32_e64 %4, %7, 0, %4, %7\n\t"
+            "v_addc_co_u32_e64 %5, %8, 0, %5, %8"
+            : "+&v"(sum[0]), "+&v"(sum[1]), "+&v"(sum[2]), "+&v"(over[0]), "+&v"(over[1]), "+&v"(over[2]),
+              "=&s"(c0), "=&s"(c1), "=&s"(c2)
+            : "v"(t), "s"(w[0]), "s"(w[1]), "s"(w[2]));
+    } else {
+        asm("v_mad_u64_u32 %0, %4, %6, %7, %0\n\t"
+            "v_mad_u64_u32 %1, %5, %6, %8, %1\n\t"
+            "s_nop 0\n\t"
+            "v_addc_co_u32_e64 %2, %4, 0, %2, %4\n\t"
+            "v_addc_co_u32_e64 %3, %5, 0, %3, %5"
+            : "+&v"(sum[0]), "+&v"(sum[1]), "+&v"(over[0]), "+&v"(over[1]), "=&s"(c0), "=&s"(c1)
+            : "v"(t), "s"(w[0]), "s"(w[1]));
+    }
+}
+
+// The same for NW >= 2 columns, in blocks of four and three (and two, of 2 and 5).
+template <int NW>
+__device__ __forceinline__ void mad_columns(uint64_t *sum, uint32_t *over, uint32_t t, const uint32_t *w)
+{
+    constexpr int N = NW % 4 == 0 || NW == 7 ? 4 : (NW >= 3 ? 3 : 2);
+    mad_carry<N>(sum, over, t, w);
+    if constexpr (NW > N) mad_columns<NW - N>(sum + N, over + N, t, w + N);
 }
 
 template <int NW, bool MOD>
@@ -488,10 +532,7 @@ __global__ void __launch_bounds__(128) crt_direct_kernel(const uint32_t *__restr
     for (int l = 0; l < NW; ++l) col[l] = 0, over[l] = 0;
     uint64_t S = MOD ? (uint64_t)1 << 37 : (uint64_t)1 << 55;
     // sum += t * (NW words at w)
-    const auto add = [&](uint32_t t, const uint32_t *w) {
-#pragma unroll
-        for (int l = 0; l < NW; ++l) mad_carry(col[l], over[l], t, w[l]);
-    };
+    const auto add = [&](uint32_t t, const uint32_t *w) { mad_columns<NW>(col, over, t, w); };
     constexpr int kAhead = 8;  // residues loaded together
     for (int i0 = 0; i0 < r; i0 += kAhead) {
         uint32_t rv[kAhead];
