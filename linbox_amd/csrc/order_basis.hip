@@ -691,6 +691,16 @@ __device__ __forceinline__ void grid_barrier(unsigned *bar, unsigned target)
     __syncthreads();
 }
 
+// Makes a count known to the group's other waves, behind the LDS words it covers: the
+// fence keeps the compiler from moving their stores past it (they are other arrays,
+// which it knows), and LDS does one wave's accesses in order.
+template <class T>
+__device__ __forceinline__ void publish(T *count, T value)
+{
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __hip_atomic_store(count, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 // i / d for 0 <= i < 2^20, d > 0, given r = 1 / (float)d: (i + 1/2) r is at least
 // 1/(2d) away from an integer, more than the products' rounding
 __device__ __forceinline__ int quot(int i, float r) { return (int)(((float)i + 0.5f) * r); }
@@ -1128,7 +1138,7 @@ __global__ void __launch_bounds__(kMbThreads) m_basis_cols_kernel(DevView serie,
                                 }
                                 if (wave == 0) book(applied, cc, dz == 0);
                             }
-                            if (wave == 0 && lane == 0) s_book = applied + 1;
+                            if (wave == 0 && lane == 0) publish(&s_book, applied + 1);
                             if (++applied < pub) fetch();
                         }
                         if (state >> 16) return true;
@@ -1238,9 +1248,7 @@ __global__ void __launch_bounds__(kMbThreads) m_basis_cols_kernel(DevView serie,
                                            : make_int4(pc[0], pc[1], pc[2], pc[3]);
                         pbits[P] = (int)rowbits;
                         pdet[P] = dcur;
-                        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-                        __hip_atomic_store(&s_pub, (unsigned)(P + 1) | rk << 8 | (rk == (unsigned)n ? 1u << 16 : 0u),
-                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        publish(&s_pub, (unsigned)(P + 1) | rk << 8 | (rk == (unsigned)n ? 1u << 16 : 0u));
                     }
                     __atomic_signal_fence(__ATOMIC_SEQ_CST);
                     __builtin_amdgcn_s_setprio(0);
