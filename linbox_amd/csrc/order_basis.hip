@@ -666,6 +666,19 @@ struct Centred {
     }
 };
 
+// A wait polls kMcSpinLimit times at most, and one that gives up sets the failure
+// flag: what follows works on unfinished data, and the flag alone keeps the host
+// from taking its result for one.  The flag only matters once a limit ran out, so
+// a wait reads it now and then.
+__device__ __forceinline__ bool wait_failed(unsigned *bar)
+{
+    return __hip_atomic_load(bar + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+}
+__device__ __forceinline__ void report_wait(unsigned *bar)
+{
+    __hip_atomic_store(bar + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // All groups of the grid meet here: bar[0] counts arrivals and is awaited to
 // reach `target`; bar[1] is set when a poll limit runs out (the host reports the
 // call as failed, and later barriers no longer wait).  What the groups exchange is
@@ -679,10 +692,9 @@ __device__ __forceinline__ void grid_barrier(unsigned *bar, unsigned target)
         __hip_atomic_fetch_add(bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         unsigned polls = 0;
         while ((int)(__hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - target) < 0) {
-            // the failure flag only matters once a limit ran out: read it now and then
-            if ((polls & 255) == 255 && __hip_atomic_load(bar + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
+            if ((polls & 255) == 255 && wait_failed(bar)) break;
             if (++polls == kMcSpinLimit) {
-                __hip_atomic_store(bar + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                report_wait(bar);
                 break;
             }
             __builtin_amdgcn_s_sleep(1);
@@ -1143,13 +1155,9 @@ __global__ void __launch_bounds__(kMbThreads) m_basis_cols_kernel(DevView serie,
                         }
                         if (state >> 16) return true;
                         if (pub >= want) return false;
-                        // the failure flag (global memory) only matters once a poll limit
-                        // ran out somewhere: read it now and then, not on every poll
-                        if ((polls & 255) == 255 &&
-                            __hip_atomic_load(bar + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                            return true;
+                        if ((polls & 255) == 255 && wait_failed(bar)) return true;
                         if (++polls == kMcSpinLimit) {
-                            __hip_atomic_store(bar + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            report_wait(bar);
                             return true;
                         }
                         // the wave whose turn is next polls without a pause
@@ -1262,12 +1270,14 @@ __global__ void __launch_bounds__(kMbThreads) m_basis_cols_kernel(DevView serie,
                 if (wave == 0 && lane == 0) s_e = e_run;
                 if (mine > found) {
                     // wait for the last panel's booking
-                    for (unsigned polls = 0; wave != 0 && polls < kMcSpinLimit; ++polls) {
-                        const int bk_n = __hip_atomic_load(&s_book, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                        if (__builtin_amdgcn_readfirstlane(bk_n) >= applied) break;
-                        if ((polls & 255) == 255 &&
-                            __hip_atomic_load(bar + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                    for (unsigned polls = 0; wave != 0;) {
+                        const int booked = __hip_atomic_load(&s_book, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        if (__builtin_amdgcn_readfirstlane(booked) >= applied) break;
+                        if ((polls & 255) == 255 && wait_failed(bar)) break;
+                        if (++polls == kMcSpinLimit) {
+                            report_wait(bar);
                             break;
+                        }
                     }
                     __atomic_signal_fence(__ATOMIC_SEQ_CST);
                     const int bc = col < n ? bidx[col] : -1;
