@@ -37,7 +37,8 @@ struct InvArgs {
 
 // One whole forward transform per TP threads.  Input coefficient t is
 // coefficient t of the view, or rev-1-t of it when rev != 0 (the view has at
-// most rev coefficients then), zero where that is outside the view.  One body
+// most rev coefficients then), zero where that is outside the view; out may be the
+// view's own storage.  One body
 // serves every layout (a stride) and both zero paddings (only the first stage
 // differs, behind a uniform branch): with a body for each the kernel is several
 // times as long, and a launch of few groups waits for its instructions (800
@@ -45,7 +46,7 @@ struct InvArgs {
 template <int L>
 __device__ __forceinline__ void forward_entry(const DevView &in, size_t rev, size_t e, bool active, bool halfzero,
                                               const uint2 *__restrict__ tw, uint32_t p, uint32_t h,
-                                              uint32_t *__restrict__ out, int tp, uint32_t *lds)
+                                              uint32_t *out, int tp, uint32_t *lds)
 {
     using C = Cfg<L>;
     constexpr int RP0 = C::RLOG;

@@ -13,7 +13,7 @@ using namespace ntt;
 template <int L, int SEND, bool HALFZERO>
 __global__ void __launch_bounds__(Cfg<L>::BLOCK) ntt_dif_kernel(DevView in, size_t entries, EntryMap map,
                                                                const uint2 *__restrict__ tw, uint32_t p,
-                                                               uint32_t *__restrict__ out)
+                                                               uint32_t *out)
 {
     extern __shared__ uint32_t lds_all[];
     dif_body<L, SEND, HALFZERO>(in, entries, map, tw, p, out, (size_t)blockIdx.x * Cfg<L>::G, threadIdx.x, lds_all);
@@ -39,7 +39,7 @@ __global__ void __launch_bounds__(Cfg<L>::BLOCK) dit_tail_persistent_kernel(cons
 }
 
 template <int L, int DSTART, bool SCALE>
-__global__ void __launch_bounds__(Cfg<L>::BLOCK) ntt_dit_kernel(const uint32_t *__restrict__ in, size_t entries,
+__global__ void __launch_bounds__(Cfg<L>::BLOCK) ntt_dit_kernel(const uint32_t *in, size_t entries,
                                                                const uint2 *__restrict__ tw, uint32_t p, DevView out,
                                                                size_t out_first, size_t count, uint32_t scale,
                                                                uint32_t scale_p)

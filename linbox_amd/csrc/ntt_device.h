@@ -241,7 +241,7 @@ constexpr int dif_last_rp()
 // The words of a whole forward transform (all L stages) to its row o; with
 // CENTRE those above h less p (h = p/2: centred to int32; h = 2^32 - 1: as they are).
 template <int L, bool CENTRE>
-__device__ __forceinline__ void dif_store(uint32_t (&x)[Cfg<L>::R], int tp, uint32_t *__restrict__ o, uint32_t p,
+__device__ __forceinline__ void dif_store(uint32_t (&x)[Cfg<L>::R], int tp, uint32_t *o, uint32_t p,
                                           uint32_t h)
 {
     using C = Cfg<L>;
@@ -269,10 +269,11 @@ __device__ __forceinline__ void dif_store(uint32_t (&x)[Cfg<L>::R], int tp, uint
 // DIF stages [0, SEND) of one polynomial per TP threads.  With SEND == L the
 // result is the full transform (R consecutive words per thread are stored as
 // 16-byte vectors); with SEND < L the data is left in natural storage order
-// as 2^(L-SEND) independent blocks for the remaining stages.
+// as 2^(L-SEND) independent blocks for the remaining stages.  out may be the
+// view's own storage (SEND == L): a group has read its polynomials before it stores.
 template <int L, int SEND, bool HALFZERO, bool CENTRE = false>
 __device__ __forceinline__ void dif_body(const DevView &in, size_t entries, const EntryMap &map,
-                                         const uint2 *__restrict__ tw, uint32_t p, uint32_t *__restrict__ out,
+                                         const uint2 *__restrict__ tw, uint32_t p, uint32_t *out,
                                          size_t e_base, int tid, uint32_t *lds_all, uint32_t h = ~0u)
 {
     using C = Cfg<L>;
@@ -324,9 +325,10 @@ __device__ __forceinline__ void dif_body(const DevView &in, size_t entries, cons
 
 // DIT stages [DSTART, L) of one polynomial per TP threads.  DSTART == 0 reads
 // bit-reversed input with 16-byte vector loads; DSTART > 0 continues a
-// transform whose first DSTART stages were applied blockwise.
+// transform whose first DSTART stages were applied blockwise.  The view may be
+// in's own storage, as for dif_body.
 template <int L, int DSTART, bool SCALE>
-__device__ __forceinline__ void dit_body(const uint32_t *__restrict__ in, size_t entries,
+__device__ __forceinline__ void dit_body(const uint32_t *in, size_t entries,
                                          const uint2 *__restrict__ tw, uint32_t p, const DevView &out,
                                          size_t out_first, size_t count, uint32_t scale, uint32_t scale_p,
                                          size_t e_base, int tid, uint32_t *lds_all)
