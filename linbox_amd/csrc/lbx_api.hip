@@ -227,6 +227,19 @@ private:
 //   100^3       67 / 73  186 / 187  342 / 357  688 / 641  1422 / 1271
 //   128x64x64   52 / 56  104 / 103  196 / 193  411 / 352   861 / 687
 //   128^3       90 / 82  273 / 238  558 / 467 1157 / 841  2403 / 1637
+// Above 2^kMaxLdsLog points the INT8 form has no split transforms and converts in
+// passes of its own, so it pays only where its tiles are well filled and the
+// products many (ms):
+//             2^16 points    2^17
+//   64^3        4.97 / 5.57   10.1 / 11.1
+//   80^3        8.20 / 10.1   17.0 / 20.2
+//   100^3       15.0 / 15.7   30.3 / 31.2
+//   128x64x128  15.1 / 15.2   30.8 / 31.2
+//   112^3       18.5 / 18.8   37.4 / 37.9
+//   96x128x96   15.9 / 15.7   33.0 / 31.7
+//   120^3       22.5 / 21.5   45.2 / 42.1
+//   128^3       24.5 / 22.2   50.3 / 46.4
+//   160^3       45.9 / 47.5
 int choose_method(int method, size_t m, size_t k, size_t n, unsigned L)
 {
     if (method == LBX_METHOD_PLAIN_U64 || method == LBX_METHOD_INT8_MFMA) return method;
@@ -234,6 +247,7 @@ int choose_method(int method, size_t m, size_t k, size_t n, unsigned L)
     const auto up = [](size_t x, size_t to) { return (double)((x + to - 1) / to * to); };
     const double mkn = (double)m * k * n, used = mkn / (up(m, 32) * up(k, 64) * up(n, 32));
     const double two18 = (double)(1u << 18);
+    if (L > (unsigned)kMaxLdsLog) return mkn > 4 * two18 && used >= 0.8 ? LBX_METHOD_INT8_MFMA : LBX_METHOD_PLAIN_U64;
     const bool big = (L >= 12 && mkn >= two18 && used >= 0.45) ||
                      (mkn >= 2 * two18 && used >= 0.95 && mkn * (double)((uint64_t)1 << L) >= 2048 * two18);
     return big ? LBX_METHOD_INT8_MFMA : LBX_METHOD_PLAIN_U64;
@@ -576,13 +590,16 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
         st.mark("inverse FFT_DIT");
         return LBX_OK;
     }
+    // transforms of several passes, and the short ones of the INT8 form.  The plain
+    // form's tiles take centred words: 32^3 at 2^16 points 1.16 ms, 48^3 2.69, 80^3 8.20,
+    // against 1.52, 4.08 and 14.7 on unsigned words in 4x4 tiles without loads ahead
     {
         KernelTimer kt(ctx, s, "kernel dif a", timing);
-        LBX_TRY_HIP(launch_ntt_forward(a, m * k, L, twa, p, (uint32_t *)ahat, s));
+        LBX_TRY_HIP(launch_ntt_forward(a, m * k, L, twa, p, (uint32_t *)ahat, s, !int8));
     }
     {
         KernelTimer kt(ctx, s, "kernel dif b", timing);
-        LBX_TRY_HIP(launch_ntt_forward(b, k * n, L, twb, p, (uint32_t *)bhat, s));
+        LBX_TRY_HIP(launch_ntt_forward(b, k * n, L, twb, p, (uint32_t *)bhat, s, !int8));
     }
     st.mark("direct FFT_DIF");
     if (method == LBX_METHOD_INT8_MFMA) {
@@ -597,7 +614,7 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
     } else {
         {
             KernelTimer kt(ctx, s, "kernel pw_plain", timing);
-            LBX_TRY_HIP(launch_pointwise_plain((const uint32_t *)ahat, (const uint32_t *)bhat, (uint32_t *)chat, m, k,
+            LBX_TRY_HIP(launch_pointwise_tiled((const uint32_t *)ahat, (const uint32_t *)bhat, (uint32_t *)chat, m, k,
                                                n, N, 1, &p, &inv_n, s));
         }
         st.mark("Pointwise mult");

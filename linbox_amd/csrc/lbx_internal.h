@@ -67,8 +67,9 @@ constexpr int kMaxLog = 27;     // longest transform: 2^27 points (the 2-adic va
 // contiguously to out[e*2^L ...].  Lengths 2^1..2^kMaxLdsLog stay in LDS
 // (one HBM read and write); longer ones, up to 2^kMaxLog, add HBM passes of
 // up to four stages each.  `in` and `out` may be the same polfirst storage.
+// centre (lengths above 2^kMaxLdsLog): outputs as int32 in (-p/2, p/2].
 hipError_t launch_ntt_forward(const DevView &in, size_t entries, unsigned L, const uint2 *tw, uint32_t p,
-                              uint32_t *out, hipStream_t s);
+                              uint32_t *out, hipStream_t s, bool centre = false);
 // Inverse DIT (bit-reversed in, natural out) of `entries` contiguous
 // polynomials in[e*2^L ...]; coefficients 0..count-1 of entry e are written
 // to the view `out` after multiplication by `scale` (scale==1: none).

@@ -10,13 +10,14 @@ namespace lbx {
 namespace {
 using namespace ntt;
 
-template <int L, int SEND, bool HALFZERO>
+template <int L, int SEND, bool HALFZERO, bool CENTRE>
 __global__ void __launch_bounds__(Cfg<L>::BLOCK) ntt_dif_kernel(DevView in, size_t entries, EntryMap map,
                                                                const uint2 *__restrict__ tw, uint32_t p,
                                                                uint32_t *out)
 {
     extern __shared__ uint32_t lds_all[];
-    dif_body<L, SEND, HALFZERO>(in, entries, map, tw, p, out, (size_t)blockIdx.x * Cfg<L>::G, threadIdx.x, lds_all);
+    dif_body<L, SEND, HALFZERO, CENTRE>(in, entries, map, tw, p, out, (size_t)blockIdx.x * Cfg<L>::G, threadIdx.x,
+                                        lds_all, CENTRE ? p >> 1 : ~0u);
 }
 
 template <int L, int SEND, bool HALFZERO>
@@ -56,13 +57,13 @@ hipError_t allow_lds(K k, size_t bytes)
     return hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
-template <int L, int SEND>
+template <int L, int SEND, bool CENTRE = false>
 hipError_t fwd_launch(const DevView &in, size_t entries, const EntryMap &map, const uint2 *tw, uint32_t p,
                       uint32_t *out, hipStream_t s)
 {
     using C = Cfg<L>;
     const unsigned grid = (unsigned)((entries + C::G - 1) / C::G);
-    auto k = (in.size * 2 <= (size_t)C::N) ? ntt_dif_kernel<L, SEND, true> : ntt_dif_kernel<L, SEND, false>;
+    auto k = (in.size * 2 <= (size_t)C::N) ? ntt_dif_kernel<L, SEND, true, CENTRE> : ntt_dif_kernel<L, SEND, false, CENTRE>;
     hipError_t e = allow_lds(k, C::LDS_BYTES);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k, dim3(grid), dim3(C::BLOCK), C::LDS_BYTES, s, in, entries, map, tw, p, out);
@@ -635,9 +636,9 @@ hipError_t dit_cols(unsigned rc, uint32_t *buf, size_t entries, unsigned L, unsi
 
 // Forward DIF of length 2^L > 2^15: column passes over stages [0, L-14)
 // from the view into out, then the LDS-resident DIF of the 2^(L-14) blocks of
-// every entry, in place.
+// every entry, in place; its outputs centred to int32 where asked.
 hipError_t ntt_forward_long(const DevView &in, size_t entries, unsigned L, const uint2 *tw, uint32_t p, uint32_t *out,
-                            hipStream_t s)
+                            bool centre, hipStream_t s)
 {
     const size_t N = (size_t)1 << L, M = (size_t)1 << kLongLds;
     unsigned s0 = 0;
@@ -650,7 +651,8 @@ hipError_t ntt_forward_long(const DevView &in, size_t entries, unsigned L, const
     const size_t blocks = entries << (L - kLongLds);
     const DevView bv{out, 0, blocks, 1, M, 0, M};
     const EntryMap id{0, blocks, 0};
-    return fwd_launch<kLongLds, kLongLds>(bv, blocks, id, tw + (N - M), p, out, s);
+    return centre ? fwd_launch<kLongLds, kLongLds, true>(bv, blocks, id, tw + (N - M), p, out, s)
+                  : fwd_launch<kLongLds, kLongLds>(bv, blocks, id, tw + (N - M), p, out, s);
 }
 
 // Inverse DIT of length 2^L > 2^15: the LDS-resident DIT of the 2^(L-14)
@@ -683,10 +685,12 @@ hipError_t ntt_inverse_long(uint32_t *in, size_t entries, unsigned L, const uint
 }  // namespace
 
 hipError_t launch_ntt_forward(const DevView &in, size_t entries, unsigned L, const uint2 *tw, uint32_t p,
-                              uint32_t *out, hipStream_t s)
+                              uint32_t *out, hipStream_t s, bool centre)
 {
     if (entries == 0) return hipSuccess;
-    if (L > (unsigned)kMaxLdsLog && L <= (unsigned)kMaxLog) return ntt_forward_long(in, entries, L, tw, p, out, s);
+    if (L > (unsigned)kMaxLdsLog && L <= (unsigned)kMaxLog)
+        return ntt_forward_long(in, entries, L, tw, p, out, centre, s);
+    if (centre) return hipErrorInvalidValue;
     const EntryMap id{0, entries, 0};
     switch (L) {
 #define LBX_CASE(l) \

@@ -88,7 +88,8 @@ struct PlainPrimes {
 };
 
 // One output tile at one point per lane; item = tile * npts + t, so a wave's
-// lanes take consecutive points and transforms shorter than a wave share it.
+// lanes take consecutive points and transforms shorter than a wave share it: the
+// form of products by constants and of transforms of fewer than 64 points.
 template <int T>
 __global__ void __launch_bounds__(256) pw_plain_kernel(const uint32_t *__restrict__ A, const uint32_t *__restrict__ B,
                                                        uint32_t *__restrict__ C, int m, int k, int n, size_t npts,
