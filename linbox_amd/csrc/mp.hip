@@ -191,23 +191,18 @@ bool generate_primes(uint64_t pbound, const Limbs &prodbound, unsigned kmin, std
     return false;
 }
 
-// Device constant block (32-bit words):
+// Constant block of the mixed-radix kernel (32-bit words), in plans whose
+// recombination is not the direct one:
 //   [0..r)         primes p_i
 //   [r..2r)        floor(2^32/p_i)            (Shoup constant of 1)
-//   [2r..3r)       2^32 mod p_i
-//   [3r..4r)       Shoup constant of 2^32 mod p_i
-//   [4r..4r+2r^2)  Garner inverses (p_j mod p_i)^-1 and their Shoup constants, i*r+j
+//   [2r..2r+2r^2)  Garner inverses (p_j mod p_i)^-1 and their Shoup constants, i*r+j
 //   then r*nlimbs  prod_{j<i} p_j mod P, then nlimbs words of P
-// (the mixed-radix kernel's), followed by the residue constants
-// (ResidueBlock) and, for the direct kernels, a CrtBlock.
 struct MpLayout {
     int r, nl;
     __host__ __device__ int primes() const { return 0; }
     __host__ __device__ int onep() const { return r; }
-    __host__ __device__ int r32() const { return 2 * r; }
-    __host__ __device__ int r32p() const { return 3 * r; }
-    __host__ __device__ int inv() const { return 4 * r; }
-    __host__ __device__ int mi() const { return 4 * r + 2 * r * r; }
+    __host__ __device__ int inv() const { return 2 * r; }
+    __host__ __device__ int mi() const { return 2 * r + 2 * r * r; }
     __host__ __device__ int P() const { return mi() + r * nl; }
     __host__ __device__ int words() const { return P() + nl; }
 };
@@ -791,6 +786,34 @@ lbx_status prime_products(lbx_ctx *ctx, const std::vector<uint32_t> &primes, con
     return LBX_OK;
 }
 
+// Primes, Shoup constants of 1 and Garner inverses (p_j mod p_i)^-1 with their Shoup
+// constants at 2(i r + j), j < i, of a mixed-radix recombination.
+void garner_constants(std::vector<uint32_t> &K, const std::vector<uint32_t> &primes, int at_primes, int at_one,
+                      int at_inv)
+{
+    const size_t r = primes.size();
+    for (size_t i = 0; i < r; ++i) {
+        const uint32_t p = primes[i];
+        K[at_primes + i] = p;
+        K[at_one + i] = shoup_pre(1, p);
+        for (size_t j = 0; j < i; ++j) {
+            const uint32_t inv = invmod_h(primes[j] % p, p);
+            K[at_inv + 2 * (i * r + j)] = inv;
+            K[at_inv + 2 * (i * r + j) + 1] = shoup_pre(inv, p);
+        }
+    }
+}
+
+lbx_status upload_plan(MpPlan *plan, const std::vector<uint32_t> &K)
+{
+    LBX_TRY_HIP(hipMalloc(&plan->d_const, K.size() * 4));
+    const hipError_t e = hipMemcpy(plan->d_const, K.data(), K.size() * 4, hipMemcpyHostToDevice);
+    if (e == hipSuccess) return LBX_OK;
+    (void)hipFree(plan->d_const);
+    plan->d_const = nullptr;
+    return from_hip(e);
+}
+
 lbx_status get_plan(lbx_ctx *ctx, const uint32_t *Pw, int nl, size_t k, size_t minsz, unsigned lpts, MpPlan **out)
 {
     const std::string key = mp_plan_key(Pw, nl, k, minsz, lpts);
@@ -808,35 +831,28 @@ lbx_status get_plan(lbx_ctx *ctx, const uint32_t *Pw, int nl, size_t k, size_t m
     limbs_mul_small(bound, (uint32_t)minsz);
     std::vector<uint32_t> primes;
     if (!generate_primes((uint64_t)1 << 31, bound, lpts, primes)) return LBX_ERR_NOT_ENOUGH_PRIMES;
-    const int r = (int)primes.size();
-    const MpLayout lay{r, nl};
-    std::vector<uint32_t> K((size_t)lay.words(), 0);
-    Limbs M{1};
-    for (int i = 0; i < r; ++i) {
-        const uint32_t p = primes[i];
-        K[lay.primes() + i] = p;
-        K[lay.onep() + i] = shoup_pre(1, p);
-        const uint32_t r32 = (uint32_t)(((uint64_t)1 << 32) % p);
-        K[lay.r32() + i] = r32;
-        K[lay.r32p() + i] = shoup_pre(r32, p);
-        for (int j = 0; j < i; ++j) {
-            const uint32_t inv = invmod_h(primes[j] % p, p);
-            K[lay.inv() + 2 * (i * r + j)] = inv;
-            K[lay.inv() + 2 * (i * r + j) + 1] = shoup_pre(inv, p);
-        }
-        const Limbs mi = limbs_mod(M, P);
-        for (int l = 0; l < nl; ++l) K[lay.mi() + i * nl + l] = l < (int)mi.size() ? mi[l] : 0;
-        limbs_mul_small(M, p);
-        M = limbs_mod(M, P);
-    }
-    for (int l = 0; l < nl; ++l) K[lay.P() + l] = Pw[l];
-    MpPlan *plan = new MpPlan();
+    const int r = (int)primes.size(), nw = crt_words(primes, nl);
+    std::vector<uint32_t> K;
+    std::unique_ptr<MpPlan> plan(new MpPlan());
     plan->primes = primes;
     plan->lpts = lpts;
     plan->nlimbs = nl;
+    if (!nw) {
+        const MpLayout lay{r, nl};
+        K.resize((size_t)lay.words(), 0);
+        garner_constants(K, primes, lay.primes(), lay.onep(), lay.inv());
+        Limbs M{1};
+        for (int i = 0; i < r; ++i) {
+            const Limbs mi = limbs_mod(M, P);
+            for (int l = 0; l < nl; ++l) K[lay.mi() + i * nl + l] = l < (int)mi.size() ? mi[l] : 0;
+            limbs_mul_small(M, primes[i]);
+            M = limbs_mod(M, P);
+        }
+        for (int l = 0; l < nl; ++l) K[lay.P() + l] = Pw[l];
+    }
     plan->res_off = K.size();
     residue_constants(K, primes, nl);
-    if (const int nw = crt_words(primes, nl)) {
+    if (nw) {
         // P at the top of nw words with its top bit set: Q = P 2^(32 off + sh)
         const int np = (int)P.size(), off = nw - np, sh = __builtin_clz(P.back());
         const auto place = [&](const Limbs &x, uint32_t *dst) {  // x < P: x 2^(32 off + sh) in nw words
@@ -866,15 +882,9 @@ lbx_status get_plan(lbx_ctx *ctx, const uint32_t *Pw, int nl, size_t k, size_t m
         place(P, &K[plan->crt_off + cb.Q()]);
         K[plan->crt_off + cb.sh() + 2] = div21_inverse(K[plan->crt_off + cb.Q() + nw - 1]);
     }
-    hipError_t e = hipMalloc(&plan->d_const, K.size() * 4);
-    if (e == hipSuccess) e = hipMemcpy(plan->d_const, K.data(), K.size() * 4, hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        if (plan->d_const) (void)hipFree(plan->d_const);
-        delete plan;
-        return from_hip(e);
-    }
-    ctx->mp_plans[key] = plan;
-    *out = plan;
+    LBX_TRY(upload_plan(plan.get(), K));
+    ctx->mp_plans[key] = plan.get();
+    *out = plan.release();
     return LBX_OK;
 }
 
@@ -898,7 +908,7 @@ lbx_status get_few_plan(lbx_ctx *ctx, uint32_t p, size_t k, size_t minsz, unsign
     limbs_mul_small(bound, (uint32_t)minsz);
     std::vector<uint32_t> primes;
     if (!generate_primes((uint64_t)1 << 31, bound, lpts, primes)) return LBX_ERR_NOT_ENOUGH_PRIMES;
-    MpPlan *plan = new MpPlan();
+    std::unique_ptr<MpPlan> plan(new MpPlan());
     plan->lpts = lpts;
     plan->nlimbs = 1;
     for (uint32_t q : primes) plan->reduce = plan->reduce || q <= p;
@@ -906,31 +916,19 @@ lbx_status get_few_plan(lbx_ctx *ctx, uint32_t p, size_t k, size_t minsz, unsign
         const int r = (int)primes.size();
         const FpLayout lay{r};
         std::vector<uint32_t> K((size_t)lay.words(), 0);
+        garner_constants(K, primes, lay.primes(), lay.onep(), lay.inv());
         uint32_t beta = 1 % p;
         for (int i = 0; i < r; ++i) {
             const uint32_t pi = primes[i];
-            K[lay.primes() + i] = pi;
-            K[lay.onep() + i] = shoup_pre(1, pi);
-            for (int j = 0; j < i; ++j) {
-                const uint32_t inv = invmod_h(primes[j] % pi, pi);
-                K[lay.inv() + 2 * (i * r + j)] = inv;
-                K[lay.inv() + 2 * (i * r + j) + 1] = shoup_pre(inv, pi);
-            }
             K[lay.beta() + 2 * i] = beta;
             K[lay.beta() + 2 * i + 1] = shoup_pre(beta, p);
             beta = (uint32_t)((uint64_t)beta * (pi % p) % p);  // beta *= p_i (:179-180)
         }
-        hipError_t e = hipMalloc(&plan->d_const, K.size() * 4);
-        if (e == hipSuccess) e = hipMemcpy(plan->d_const, K.data(), K.size() * 4, hipMemcpyHostToDevice);
-        if (e != hipSuccess) {
-            if (plan->d_const) (void)hipFree(plan->d_const);
-            delete plan;
-            return from_hip(e);
-        }
+        LBX_TRY(upload_plan(plan.get(), K));
         plan->primes = primes;
     }
-    ctx->mp_plans[key] = plan;
-    *out = plan;
+    ctx->mp_plans[key] = plan.get();
+    *out = plan.release();
     return LBX_OK;
 }
 
@@ -1059,10 +1057,10 @@ constexpr int kZzMaxPrimes = 96;
 
 namespace {
 
-// Constant block: primes, Shoup constants of 1, Garner inverses (p_j mod
-// p_i)^-1 with their Shoup constants at 2(i r + j), then W_i = prod_{j<i} p_j mod
-// 2^(32 cl) in cl words each, then M mod 2^(32 cl) (the mixed-radix kernel's),
-// followed by the residue constants and, for the direct kernels, a CrtBlock.
+// Constant block of the mixed-radix kernel, in plans whose recombination is not
+// the direct one: primes, Shoup constants of 1, Garner inverses (p_j mod p_i)^-1
+// with their Shoup constants at 2(i r + j), then W_i = prod_{j<i} p_j mod 2^(32 cl)
+// in cl words each, then M mod 2^(32 cl).
 struct ZzLayout {
     int r, cl;
     __host__ __device__ int primes() const { return 0; }
@@ -1214,36 +1212,32 @@ lbx_status get_zz_plan(lbx_ctx *ctx, unsigned lab, size_t k, size_t minsz, unsig
     if (!generate_primes((uint64_t)1 << 31, bound, lpts, primes) || (int)primes.size() > kZzMaxPrimes)
         return LBX_ERR_NOT_ENOUGH_PRIMES;
     const int r = (int)primes.size();
-    const ZzLayout lay{r, cl};
-    std::vector<uint32_t> K((size_t)lay.words(), 0);
     const auto low = [&](const Limbs &x, uint32_t *dst, int n) {  // x mod 2^(32 n)
         for (int l = 0; l < n; ++l) dst[l] = l < (int)x.size() ? x[l] : 0;
     };
-    Limbs W{1};  // prod_{j<i} p_j
-    for (int i = 0; i < r; ++i) {
-        const uint32_t p = primes[i];
-        K[lay.primes() + i] = p;
-        K[lay.onep() + i] = shoup_pre(1, p);
-        for (int j = 0; j < i; ++j) {
-            const uint32_t inv = invmod_h(primes[j] % p, p);
-            K[lay.inv() + 2 * (i * r + j)] = inv;
-            K[lay.inv() + 2 * (i * r + j) + 1] = shoup_pre(inv, p);
-        }
-        low(W, &K[lay.W() + i * cl], cl);
-        limbs_mul_small(W, p);
-    }
-    low(W, &K[lay.M()], cl);
+    // the direct form where M > bound (1 + 2^-16): M 2^16 > bound (2^16 + 1)
+    Limbs lhs = prime_product(primes), rhs = bound;
+    limbs_mul_small(lhs, 1u << 16);
+    limbs_mul_small(rhs, (1u << 16) + 1);
+    const int nw = limbs_cmp(lhs, rhs) > 0 ? crt_words(primes, cl) : 0;
+    std::vector<uint32_t> K;
     std::unique_ptr<MpPlan> plan(new MpPlan());
     plan->primes = primes;
     plan->lpts = lpts;
     plan->nlimbs = nl;
+    if (!nw) {
+        const ZzLayout lay{r, cl};
+        K.resize((size_t)lay.words(), 0);
+        garner_constants(K, primes, lay.primes(), lay.onep(), lay.inv());
+        Limbs W{1};  // prod_{j<i} p_j
+        for (int i = 0; i < r; ++i) {
+            low(W, &K[lay.W() + i * cl], cl);
+            limbs_mul_small(W, primes[i]);
+        }
+        low(W, &K[lay.M()], cl);
+    }
     plan->res_off = K.size();
     residue_constants(K, primes, nl);
-    // M > bound (1 + 2^-16): M 2^16 > bound (2^16 + 1)
-    Limbs lhs = W, rhs = bound;
-    limbs_mul_small(lhs, 1u << 16);
-    limbs_mul_small(rhs, (1u << 16) + 1);
-    const int nw = limbs_cmp(lhs, rhs) > 0 ? crt_words(primes, cl) : 0;
     if (nw) {
         plan->crt_off = K.size();
         crt_constants(K, primes, nw, [&](const Limbs &x, uint32_t *dst) { low(x, dst, nw); },
@@ -1270,12 +1264,7 @@ lbx_status get_zz_plan(lbx_ctx *ctx, unsigned lab, size_t k, size_t minsz, unsig
             p = ctx->mp_plans.erase(p);
         }
     }
-    LBX_TRY_HIP(hipMalloc(&plan->d_const, K.size() * 4));
-    const hipError_t e = hipMemcpy(plan->d_const, K.data(), K.size() * 4, hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        (void)hipFree(plan->d_const);
-        return from_hip(e);
-    }
+    LBX_TRY(upload_plan(plan.get(), K));
     ctx->mp_plans[key] = plan.get();
     *out = plan.release();
     return LBX_OK;

@@ -97,10 +97,10 @@ LBX_HD uint32_t plain_finish(uint64_t acc, uint32_t p, const PlainConst &pc)
 }
 
 // Plain form on centred operands: a, b in (-p/2, p/2] as int32, so |a b| < 2^60
-// and acc += a*b is one v_mad_i64_i32.  After at most kPlainSFold = 6 products
-// the bits above 2^60 are folded back (plain_s_fold: acc mod 2^60 +
-// floor(acc / 2^60) (2^60 mod p), one v_mad_i64_i32 more, which leaves
-// |acc| < 2^60 + 2^34, and 2^60 + 2^34 + 6 * 2^60 < 2^63); at the end
+// and acc += a*b is one v_mad_i64_i32.  Every `every` products the bits above
+// 2^60 are folded back (plain_s_fold: acc mod 2^60 + floor(acc / 2^60) (2^60 mod
+// p), one v_mad_i64_i32 more, which leaves |acc| < 2^60 + 2^34; six products more
+// fit whatever p is, 2^60 + 2^34 + 6 * 2^60 < 2^63, smaller p take more); at the end
 // acc + off (off a multiple of p >= 2^63, so the sum is in [0, 2^64)) is
 // reduced as in plain_finish.
 struct PlainSConst {
@@ -110,7 +110,7 @@ struct PlainSConst {
     uint32_t every;             // products between folds for this p: the largest n with
                                 // 2^60 + 2^34 + n floor(p/2)^2 < 2^63, at most 64
 };
-constexpr uint32_t kPlainSFold = 6;  // for every p < 2^31
+constexpr uint32_t kPlainSFold = 6;  // a period that serves every p < 2^31
 
 inline PlainSConst plain_s_const(uint32_t p, uint32_t scale)
 {
