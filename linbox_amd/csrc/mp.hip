@@ -193,16 +193,16 @@ bool generate_primes(uint64_t pbound, const Limbs &prodbound, unsigned kmin, std
 
 // Constant block of the mixed-radix kernel (32-bit words), in plans whose
 // recombination is not the direct one:
-//   [0..r)         primes p_i
-//   [r..2r)        floor(2^32/p_i)            (Shoup constant of 1)
-//   [2r..2r+2r^2)  Garner inverses (p_j mod p_i)^-1 and their Shoup constants, i*r+j
+//   [0..2r^2)      Garner inverses (p_j mod p_i)^-1 and their Shoup constants, i*r+j
+//   then r primes p_i and r words floor(2^32/p_i) (Shoup constant of 1)
 //   then r*nlimbs  prod_{j<i} p_j mod P, then nlimbs words of P
+// (the inverses first: with the primes first the kernel takes 2% more, 40 primes)
 struct MpLayout {
     int r, nl;
-    __host__ __device__ int primes() const { return 0; }
-    __host__ __device__ int onep() const { return r; }
-    __host__ __device__ int inv() const { return 2 * r; }
-    __host__ __device__ int mi() const { return 2 * r + 2 * r * r; }
+    __host__ __device__ int inv() const { return 0; }
+    __host__ __device__ int primes() const { return 2 * r * r; }
+    __host__ __device__ int onep() const { return 2 * r * r + r; }
+    __host__ __device__ int mi() const { return 2 * r * r + 2 * r; }
     __host__ __device__ int P() const { return mi() + r * nl; }
     __host__ __device__ int words() const { return P() + nl; }
 };
