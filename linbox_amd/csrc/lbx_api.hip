@@ -352,20 +352,41 @@ struct Pipe {
 };
 
 // Whether a matfirst or matrowfirst operand is moved into polfirst scratch
-// before its transforms (and such a result written through it).  The transform
-// kernels take an entry's coefficients one stride apart, a 64-byte sector for
-// every word, unless a group holds 16 or more neighbouring entries (2^13 words
-// a group: up to 2^9 points); the tiled copy reads and writes whole lines, at
-// the price of one more pass and one more launch.  Measured (copied against
-// direct, us): 64^3 at 2^11 points, 2^22 words an operand: 151 / 226 matfirst,
-// 163 / 205 matrowfirst; 96x48x80 at 2^12: the inverse's tail alone 231 direct;
-// 32^3 at 2^11, 2^20 words: 83 / 83 and 100 / 79; 128^3 at 2^9, 2^22 words:
-// 154 / 162 and 167 / 157; smaller operands lose the launches (16^3 at 2^11:
-// 56 / 49 and 70 / 47).
-bool copies_to_polfirst(const DevView &v, size_t entries, size_t count, unsigned L)
+// before its transforms, or such a result written through it.  The transform
+// kernels take an entry's coefficients one stride apart (the entries, or the
+// columns of a row), a 64-byte sector for every word; a short stride leaves the
+// rest of the sector to the entries beside it, and so does a group that holds 16
+// or more neighbouring entries (2^13 words a group: up to 2^9 points).  The tiled
+// copy reads and writes whole lines, at the price of a launch and one more pass.
+// Time of the direct product over that with the one view copied:
+//   operand, matrowfirst: stride 1 to 8, 0.79-0.98; 16 at 2^22 words 0.82-1.00, at 2^24
+//     0.92-1.06, but 1.06-1.11 at 2^14 and 2^15 points; 32 and more at 2^21 words
+//     0.80-0.98, 2^22 0.94-1.02, above 1.02-1.24
+//   operand, matfirst: 2^21 words 0.91 (2^10 points) to 1.01 (2^13), above 1.05-1.35
+//   result: stride 4, 0.78-0.97; 8, 0.83-1.03 but 1.06-1.49 at 2^12 to 2^15 points; 16
+//     and more 0.95-1.14 at 3 2^20 words, above 1.0-2.7
+//   operand read by three primes' products: stride 4, 0.90-0.99; 8, 0.93-1.07; 16,
+//     0.95-1.11; above 1.05-1.39, from 3 2^20 words on
+//   their recombined result: stride 8, 0.93-1.02; 16 and more at 6 2^20 words 0.97-1.02
+//     (1.11 at 2^16 points), at 2^24 1.07-1.57
+bool copies_to_polfirst(const DevView &v, size_t entries, size_t count, unsigned L, CopyUse use)
 {
-    return v.layout != LBX_POLFIRST && entries < ((size_t)1 << 32) && L >= 10 &&
-           count >= ((size_t)1 << 21) / entries + 1;
+    if (v.layout == LBX_POLFIRST || entries >= ((size_t)1 << 32) || L < 10) return false;
+    const size_t stride = v.layout == LBX_MATFIRST ? entries : v.cols;
+    size_t least = 16, words = (size_t)1 << 21;  // copied from this stride on, above this many words
+    switch (use) {
+    case CopyUse::kOperand:
+        least = v.layout == LBX_MATROWFIRST && (L == 14 || L == 15) ? 16 : 32;
+        if (v.layout == LBX_MATFIRST)
+            words = L >= 13 ? words : (size_t)9 << 18;
+        else
+            words = v.cols >= 32 ? ((size_t)1 << 22) - 1 : (size_t)3 << 21;
+        break;
+    case CopyUse::kResult: least = L >= 12 && L <= (unsigned)kMaxLdsLog ? 8 : 16; break;
+    case CopyUse::kSharedOperand: break;
+    case CopyUse::kRecombined: words = (size_t)3 << 21; break;
+    }
+    return stride >= least && count >= words / entries + 1;
 }
 
 lbx_status multi_prime(MultiProduct &mp, unsigned i, uint32_t p, const MidSpec *mid, Workspace &ws, hipStream_t s)
@@ -470,7 +491,8 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
     // before the tail writes them); rows are 16-byte multiples for the copy
     const auto load_polfirst = [&](DevView &v, size_t entries, bool one_chunk, void *blocks, void *hat) -> lbx_status {
         const size_t stor = split ? (v.size + 3) & ~(size_t)3 : N;
-        if (!copies_to_polfirst(v, entries, v.size, L) || v.size > N || stor > N || !one_chunk) return LBX_OK;
+        if (!one_chunk || v.size > N || stor > N || !copies_to_polfirst(v, entries, v.size, L, CopyUse::kOperand))
+            return LBX_OK;
         const DevView pf{(uint32_t *)(split ? blocks : hat), LBX_POLFIRST, v.rows, v.cols, stor, 0, v.size};
         LBX_TRY_HIP(launch_copy(v, pf, entries, v.size, 0, 0, s));
         v = pf;
@@ -481,7 +503,7 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
     // the result likewise leaves through the product's own buffer, free once
     // the inverse transform has read it
     DevView out = c;
-    if (copies_to_polfirst(c, m * n, count, L) && count <= N && (!split || cchunk >= m * n)) {
+    if (copies_to_polfirst(c, m * n, count, L, CopyUse::kResult) && count <= N && (!split || cchunk >= m * n)) {
         const size_t stor = split ? std::min((count + 3) & ~(size_t)3, N) : N;
         out = DevView{(uint32_t *)(split ? cmat : chat), LBX_POLFIRST, m, n, stor, 0, count};
     }

@@ -273,8 +273,10 @@ void mp_release(lbx_ctx *ctx);
 // Frees the batch plans (graphs, descriptors) cached in a context.
 void batch_release(lbx_ctx *ctx);
 // Whether a view of `entries` x `count` coefficients that is not polfirst goes
-// through a polfirst copy in a product with 2^L points.
-bool copies_to_polfirst(const DevView &v, size_t entries, size_t count, unsigned L);
+// through a polfirst copy in a product with 2^L points: one product's operand or
+// result, an operand that every prime's product reads, or a recombined result.
+enum class CopyUse { kOperand, kResult, kSharedOperand, kRecombined };
+bool copies_to_polfirst(const DevView &v, size_t entries, size_t count, unsigned L, CopyUse use);
 // The pointwise form LBX_METHOD_AUTO resolves to for m x k x n at 2^L points.
 int choose_method(int method, size_t m, size_t k, size_t n, unsigned L);
 

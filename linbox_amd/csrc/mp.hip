@@ -988,7 +988,7 @@ lbx_status mp_product(lbx_ctx *ctx, const uint32_t *Pw, int nl, const DevView &a
             const auto as_polfirst = [&](const DevView &v, size_t entries, const char *slot) -> DevView {
                 const size_t stor = (v.size + 3) & ~(size_t)3;
                 void *buf;
-                if (fp->reduce || !copies_to_polfirst(v, entries, v.size, lpts)) return v;
+                if (fp->reduce || !copies_to_polfirst(v, entries, v.size, lpts, CopyUse::kSharedOperand)) return v;
                 if (ensure(ctx, slot, entries * stor * 4, &buf) != LBX_OK) {
                     (void)hipGetLastError();
                     return v;
@@ -1007,7 +1007,8 @@ lbx_status mp_product(lbx_ctx *ctx, const uint32_t *Pw, int nl, const DevView &a
             // a result stored by coefficient is recombined polfirst, in the place
             // of the first prime's residues, and copied out in one pass
             DevView cv = c;
-            if (copies_to_polfirst(c, m * n, sc, lpts)) cv = DevView{(uint32_t *)rc, LBX_POLFIRST, m, n, sc, 0, sc};
+            if (copies_to_polfirst(c, m * n, sc, lpts, CopyUse::kRecombined))
+                cv = DevView{(uint32_t *)rc, LBX_POLFIRST, m, n, sc, 0, sc};
             const dim3 grid(grid_of(m * n * sc, 256));
             if (Pw[0] >= (1u << 31))
                 hipLaunchKernelGGL((few_primes_crt_kernel<kFewMaxPrimes, true>), grid, dim3(256), 0, s,

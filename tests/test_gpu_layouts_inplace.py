@@ -1,11 +1,11 @@
-"""Operands and results stored by coefficient that are over 2^21 words go through
-polfirst copies kept in the buffers of their own transforms: an operand's copy is
-read by the transform that writes over it, a result's is written by the inverse
-transform that reads it.  Here that meets every kind of transform: whole ones of
-2^14 and 2^15 points, split ones, those of several passes (2^16 and 2^17 points),
-a single prime and three; and middle products, whose small operand is reversed on
-the way.  Products are checked by evaluation at a random point and the stored forms
-against polfirst ones; middle products against the middle of the product."""
+"""Large operands and results stored by coefficient go through polfirst copies
+kept in the buffers of their own transforms: an operand's copy is read by the
+transform that writes over it, a result's is written by the inverse transform that
+reads it.  Here that meets every kind of transform: whole ones of 2^14 and 2^15
+points, split ones, those of several passes (2^16 and 2^17 points), a single prime
+and three; and middle products, whose small operand is reversed on the way.
+Products are checked by evaluation at a random point and the stored forms against
+polfirst ones; middle products against the middle of the product."""
 import numpy as np
 import pytest
 
@@ -20,12 +20,13 @@ BY_COEFFICIENT = [("matfirst", "matfirst", "matfirst"), ("matrowfirst", "matfirs
 
 
 @pytest.mark.parametrize("p,m,k,n,sa,sb", [
-    (998244353, 20, 17, 18, 8000, 8100),    # 2^14 points
-    (998244353, 13, 11, 12, 15000, 16200),  # 2^15
-    (2013265921, 8, 9, 8, 30000, 33001),    # 2^16: column passes and blocks
-    (469762049, 6, 6, 6, 60001, 70000),     # 2^17
-    (998244353, 17, 32, 18, 24000, 3700),   # one operand below 2^21 words, the other over half the transform
-    (268435399, 13, 11, 12, 15000, 16200),  # three FFT primes
+    (998244353, 40, 36, 33, 8000, 8100),    # 2^14 points
+    (998244353, 18, 33, 17, 15000, 16200),  # 2^15
+    (2013265921, 4, 33, 33, 35000, 5000),   # 2^16: column passes and blocks
+    (469762049, 3, 33, 33, 60001, 7000),    # 2^17
+    (998244353, 17, 32, 18, 24000, 3700),   # an operand below the line, the other over half the transform
+    (998244353, 192, 4, 4, 8000, 8000),     # short strides: matfirst copied, matrowfirst operands not
+    (268435399, 40, 36, 33, 4000, 4100),    # three FFT primes
 ])
 def test_products(ctx, p, m, k, n, sa, sb):
     rng = np.random.default_rng(m * k * n + sa)
@@ -47,10 +48,10 @@ def test_products(ctx, p, m, k, n, sa, sb):
 
 @pytest.mark.parametrize("small_left", [True, False])
 @pytest.mark.parametrize("p,m,k,n,hdeg", [
-    (998244353, 64, 40, 36, 1000),   # 2^11 points: whole (plain) or split (INT8) transforms
-    (998244353, 18, 16, 17, 8000),   # 2^14
-    (2013265921, 9, 8, 9, 32001),    # 2^16: column passes and blocks
-    (268435399, 40, 36, 40, 1500),   # three FFT primes
+    (998244353, 64, 40, 36, 2000),   # 2^12 points: whole (plain) or split (INT8) transforms
+    (998244353, 36, 33, 34, 8000),   # 2^14
+    (2013265921, 8, 33, 33, 16400),  # 2^16: column passes and blocks
+    (268435399, 64, 40, 36, 2000),   # three FFT primes
 ])
 def test_middle_products(ctx, p, m, k, n, hdeg, small_left):
     rng = np.random.default_rng(m * k * n + hdeg)
