@@ -215,18 +215,46 @@ private:
 
 // AUTO picks the INT8 form where it measured faster on gfx950 (both forms are
 // bit-exact): for large products on long transforms, and sooner where its
-// padding (rows to 32, the inner dimension to 64) adds nothing.  Elsewhere the
+// padding (rows to 32, the inner dimension to 64) adds little.  Elsewhere the
 // split transforms and the seven launches it needs cost more than the VALU
 // pointwise they replace.  Whole products, plain / INT8, us:
-//             2^8 points  2^10       2^11       2^12        2^13
-//   32^3        22 / 36   32 / 52    48 / 70    65 / 109   108 / 178
-//   64^2x32     31 / 40   53 / 61    81 / 97   147 / 158   312 / 290
-//   64^3        39 / 44   69 / 81   117 / 123  231 / 220   490 / 420
-//   80^3        58 / 59  106 / 135  198 / 249  398 / 446   799 / 852
-//   96^3        67 / 65  151 / 152  287 / 301  588 / 530  1208 / 1034
-//   100^3       67 / 73  186 / 187  342 / 357  688 / 641  1422 / 1271
-//   128x64x64   52 / 56  104 / 103  196 / 193  411 / 352   861 / 687
-//   128^3       90 / 82  273 / 238  558 / 467 1157 / 841  2403 / 1637
+//             2^8 points  2^9        2^10       2^11       2^12        2^13
+//   32^3        22 / 36              32 / 52    48 / 70    65 / 109   108 / 178
+//   64^2x32     31 / 40              53 / 61    81 / 97   147 / 158   312 / 290
+//   64^3        39 / 44              69 / 81   117 / 123  231 / 220   490 / 420
+//   64x128x64   46 / 53    69 / 68  105 / 105  178 / 200
+//   64x192x64   53 / 60    93 / 84  140 / 142  270 / 287
+//   80^3        58 / 59             106 / 135  198 / 249  398 / 446   799 / 852
+//   96^3        64 / 64    86 / 95  146 / 151  267 / 301  588 / 530  1208 / 1034
+//   100x64x100  55 / 62    75 / 84  131 / 126  232 / 244
+//   100^3       67 / 73             186 / 187  342 / 357  688 / 641  1422 / 1271
+//   120x64x120  60 / 64    91 / 88  150 / 145  293 / 297
+//   90x128x90   71 / 69   101 / 97  174 / 160  330 / 323
+//   100x128x100 75 / 76   112 / 109 216 / 198  404 / 378
+//   112^3       78 / 79   121 / 111 214 / 205  405 / 393
+//   80x128x128  79 / 71                        394 / 356
+//   128x100x128 77 / 81   117 / 113 216 / 226  443 / 441
+//   128x64x64   52 / 56             104 / 103  196 / 193  411 / 352   861 / 687
+//   128^3       90 / 82   135 / 122 273 / 238  558 / 467 1157 / 841  2403 / 1637
+//   160^3      153 / 156  258 / 291 479 / 552
+//   256^3 at 2^6 points 138 / 229, 2^7 200 / 261, 2^8 384 / 396
+// (primes near 2^31 take up to 8% more in the plain form)
+// Several primes share three launches in the plain form and take seven each in the
+// INT8 one (three primes: 64x128x64 at 2^9 155 / 210, 128^3 at 2^8 205 / 260, 128x64x128
+// at 2^9 255 / 298).
+static bool int8_below_2_12(size_t m, size_t k, size_t n, unsigned L, double mkn, double used, size_t r)
+{
+    const double work = mkn * (double)((uint64_t)1 << L) / (double)(1u << 29);
+    if (mkn < (double)(1u << 19)) return false;
+    if (r > 1) return L >= 10 && used >= 0.95 && work >= 1;
+    if (L < 8) return L == 7 && m <= 128 && n <= 128 && used >= 0.95 && work >= 2;  // 128x512x128 175 / 160
+    if (used >= 0.95 && work >= 0.75) return true;
+    if (m > 128 || k > 128 || n > 128) return false;  // its operands no longer fit registers and LDS
+    if (k <= 64) return used >= 0.85 ? L >= 9 && work >= 0.85 : L == 10 && used >= 0.6 && work >= 1.2;
+    if (used >= 0.8) return work >= 0.48;
+    return L >= 9 && (used >= 0.78 || (used >= 0.6 && k >= 108)) && work >= 0.8;
+}
+
 // Above 2^kMaxLdsLog points the INT8 form has no split transforms and converts in
 // passes of its own, so it pays only where its tiles are well filled and the
 // products many (ms):
@@ -240,17 +268,50 @@ private:
 //   120^3       22.5 / 21.5   45.2 / 42.1
 //   128^3       24.5 / 22.2   50.3 / 46.4
 //   160^3       45.9 / 47.5
-int choose_method(int method, size_t m, size_t k, size_t n, unsigned L)
+// Below 64 points the plain form has no tiles: each thread runs through the whole
+// inner dimension, whose loads it issues at most eight at a time and no further
+// than the next fold, so a long one costs whole latencies.  The INT8 form costs each
+// prime its seven launches, and more from an output of 64x64 on.  A line from the
+// times of both (fitted to 9 outputs x 9 inner dimensions x 3 lengths x 3 primes, whose
+// crossings it meets within some 10%), of which, as whole products,
+// inner dimension 64 / 128 / 256 / 1024, us, plain then INT8:
+//   32^2, p < 2^30    28 42 73 255     33 34 34 52
+//   32^2, p < 2^28    23 32 51 170     32 33 34 52
+//   100^2, p < 2^30   28 42 74 259     38 40 72 180
+//   200^2, p < 2^30   27 42 72 253     61 102 152 458
+//   32^2, three primes near 2^31
+//                     40 65 116 416    101 103 108 164
+static bool int8_below_2_6(size_t m, size_t k, size_t n, unsigned L, uint32_t p, size_t r)
+{
+    const double kk = (double)k, mn = (double)m * n, tiles = mn * (double)((uint64_t)1 << L);
+    // the plain form, us a step: its chain, or its products where they fill the chip
+    // (4x4 tiles then, which the kernel takes from 2^21 outputs on, at half the cost)
+    const double chain = p < (1u << 29) ? 0.147 : (p < (1u << 30) ? 0.23 : 0.37);
+    const double product = (p < (1u << 30) ? 4.2e-7 : 6.5e-7) * (tiles * (double)r >= (double)(1u << 21) ? 0.52 : 1.0);
+    const double plain = 16 + std::max(chain, tiles * product * (0.45 + 0.55 * (double)r)) * kk;
+    double int8 = 31 + (mn <= 1024 ? 0.02 : 0.04) * kk;
+    if (mn > 4096) int8 = m <= 128 && k <= 128 && n <= 128 ? 44 : 45 + 0.137 * kk;
+    if (mn > 16384) int8 = 55 + 0.45 * kk * (mn / 40000);
+    return (double)r * int8 < plain;
+}
+
+int choose_method(int method, size_t m, size_t k, size_t n, unsigned L, uint32_t p, size_t r)
 {
     if (method == LBX_METHOD_PLAIN_U64 || method == LBX_METHOD_INT8_MFMA) return method;
     if (m < 16 || n < 16 || k < 16) return LBX_METHOD_PLAIN_U64;
     const auto up = [](size_t x, size_t to) { return (double)((x + to - 1) / to * to); };
     const double mkn = (double)m * k * n, used = mkn / (up(m, 32) * up(k, 64) * up(n, 32));
     const double two18 = (double)(1u << 18);
-    if (L > (unsigned)kMaxLdsLog) return mkn > 4 * two18 && used >= 0.8 ? LBX_METHOD_INT8_MFMA : LBX_METHOD_PLAIN_U64;
-    const bool big = (L >= 12 && mkn >= two18 && used >= 0.45) ||
-                     (mkn >= 2 * two18 && used >= 0.95 && mkn * (double)((uint64_t)1 << L) >= 2048 * two18);
-    return big ? LBX_METHOD_INT8_MFMA : LBX_METHOD_PLAIN_U64;
+    bool int8;
+    if (!pointwise_tiled((size_t)1 << L))
+        int8 = int8_below_2_6(m, k, n, L, p, r);
+    else if (L < 12)
+        int8 = int8_below_2_12(m, k, n, L, mkn, used, r);
+    else if (L <= (unsigned)kMaxLdsLog)
+        int8 = mkn >= two18 && used >= 0.45;
+    else
+        int8 = mkn > 4 * two18 && used >= 0.8;
+    return int8 ? LBX_METHOD_INT8_MFMA : LBX_METHOD_PLAIN_U64;
 }
 
 // Bytes of head -> tail intermediate per chunk.  The default, 2 GiB, gives one
@@ -416,7 +477,7 @@ lbx_status fft_prime_product(lbx_ctx *ctx, uint32_t p, unsigned L, const DevView
     Workspace &ws = ws_in ? *ws_in : ctx_ws;
     const size_t N = (size_t)1 << L;
     if (L > (unsigned)kMaxLog) return LBX_ERR_UNSUPPORTED;
-    method = choose_method(method, m, k, n, L);
+    method = choose_method(method, m, k, n, L, p, 1);
     const bool int8 = method == LBX_METHOD_INT8_MFMA;
     const bool split = L >= 8 && L <= (unsigned)kMaxLdsLog && int8;
     // whole transforms of both operands in one launch (a middle product's

@@ -277,8 +277,9 @@ void batch_release(lbx_ctx *ctx);
 // result, an operand that every prime's product reads, or a recombined result.
 enum class CopyUse { kOperand, kResult, kSharedOperand, kRecombined };
 bool copies_to_polfirst(const DevView &v, size_t entries, size_t count, unsigned L, CopyUse use);
-// The pointwise form LBX_METHOD_AUTO resolves to for m x k x n at 2^L points.
-int choose_method(int method, size_t m, size_t k, size_t n, unsigned L);
+// The pointwise form LBX_METHOD_AUTO resolves to for m x k x n at 2^L points, modulo
+// r primes of about p's size.
+int choose_method(int method, size_t m, size_t k, size_t n, unsigned L, uint32_t p, size_t r);
 
 
 }  // namespace lbx

@@ -743,7 +743,7 @@ lbx_status prime_products(lbx_ctx *ctx, const std::vector<uint32_t> &primes, con
                           unsigned L, int method, hipStream_t s, const MidSpec *mid)
 {
     const size_t r = primes.size();
-    if (choose_method(method, m, k, n, L) != LBX_METHOD_PLAIN_U64 || L < 1 || L > (unsigned)kMaxLdsLog) {
+    if (choose_method(method, m, k, n, L, primes[0], r) != LBX_METHOD_PLAIN_U64 || L < 1 || L > (unsigned)kMaxLdsLog) {
         for (size_t i = 0; i < r; ++i) {
             DevView va = a, vb = b;
             va.base += i * astride;
