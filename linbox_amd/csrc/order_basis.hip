@@ -1307,12 +1307,15 @@ __global__ void __launch_bounds__(kMbThreads) m_basis_cols_kernel(DevView serie,
             int32_t sum[kMcMaxTasks][4];
             if (wave == 0) {
                 // s^(p-2), s the product of the D's: both products of a bit in every step, so that
-                // their chains overlap
+                // their chains overlap.  Only sums take it, and a step whose rows are all pivot
+                // rows (every step of a square serie of full rank) has none.
                 uint32_t v = K.one, sq = s_e;
-                for (uint32_t e = p - 2; e; e >>= 1) {
-                    const uint32_t f = e & 1 ? sq : K.one;
-                    v = mont_pos(v, f, K);
-                    sq = mont_pos(sq, sq, K);
+                if (nn) {
+                    for (uint32_t e = p - 2; e; e >>= 1) {
+                        const uint32_t f = e & 1 ? sq : K.one;
+                        v = mont_pos(v, f, K);
+                        sq = mont_pos(sq, sq, K);
+                    }
                 }
                 if (fresh_tid() == 0) {
                     s_inv[kb] = K.from(v);
