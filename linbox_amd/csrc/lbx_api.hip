@@ -284,6 +284,7 @@ static bool int8_below_2_12(size_t m, size_t k, size_t n, unsigned L, double mkn
 static bool int8_below_2_6(size_t m, size_t k, size_t n, unsigned L, uint32_t p, size_t r)
 {
     const double kk = (double)k, mn = (double)m * n, tiles = mn * (double)((uint64_t)1 << L);
+    if (tiles > (double)(1u << 26)) return false;  // of the largest, the form that needs less memory
     // the plain form, us a step: its chain, or its products where they fill the chip
     // (4x4 tiles then, which the kernel takes from 2^21 outputs on, at half the cost)
     const double chain = p < (1u << 29) ? 0.147 : (p < (1u << 30) ? 0.23 : 0.37);

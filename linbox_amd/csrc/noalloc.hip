@@ -89,15 +89,19 @@ extern "C" lbx_status lbx_polymat_mul_u32_noalloc(lbx_ctx *ctx, uint32_t p, lbx_
             base = ctx->device >= 0 && ctx->device < kMaxDevices ? g_scratch[ctx->device] : nullptr;
         }
         if (!base) return LBX_ERR_HIP;
-        ArenaWorkspace ws(base, kNoAllocBytes);
         hipStream_t s = (hipStream_t)stream;
         const DevView da = devview(a, a->data), db = devview(b, b->data), dc = devview(c, c->data);
-        if (constant) {
+        const auto product = [&](int form) -> lbx_status {
+            ArenaWorkspace ws(base, kNoAllocBytes);
+            if (!constant) return fft_prime_product(ctx, p, L, da, db, dc, m, k, n, deg + 1, form, s, nullptr, &ws);
             LBX_TRY(constant_product(ctx, p, da, db, dc, m, k, n, s, &ws));
-            if (deg > 0) LBX_TRY_HIP(launch_fill(dc, m * n, 1, deg, 0u, s));
-        } else {
-            LBX_TRY(fft_prime_product(ctx, p, L, da, db, dc, m, k, n, deg + 1, method, s, nullptr, &ws));
-        }
+            return deg > 0 ? from_hip(launch_fill(dc, m * n, 1, deg, 0u, s)) : LBX_OK;
+        };
+        lbx_status st = product(method);
+        // the faster form may be the one that needs more memory (found before any product kernel
+        // is queued): AUTO then takes the other
+        if (st == LBX_ERR_WORKSPACE_TOO_SMALL && method == LBX_METHOD_AUTO) st = product(LBX_METHOD_PLAIN_U64);
+        LBX_TRY(st);
         c->size = deg + 1;
         return LBX_OK;
     });
