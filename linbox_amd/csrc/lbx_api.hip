@@ -430,7 +430,7 @@ struct Pipe {
 //   operand read by three primes' products: stride 4, 0.90-0.99; 8, 0.93-1.07; 16,
 //     0.95-1.11; above 1.05-1.39, from 3 2^20 words on
 //   their recombined result: stride 8, 0.93-1.02; 16 and more at 6 2^20 words 0.97-1.02
-//     (1.11 at 2^16 points), at 2^24 1.07-1.57
+//     (1.10 at 2^15 points, 1.11 at 2^16), at 2^24 1.07-1.57
 bool copies_to_polfirst(const DevView &v, size_t entries, size_t count, unsigned L, CopyUse use)
 {
     if (v.layout == LBX_POLFIRST || entries >= ((size_t)1 << 32) || L < 10) return false;
@@ -446,7 +446,7 @@ bool copies_to_polfirst(const DevView &v, size_t entries, size_t count, unsigned
         break;
     case CopyUse::kResult: least = L >= 12 && L <= (unsigned)kMaxLdsLog ? 8 : 16; break;
     case CopyUse::kSharedOperand: break;
-    case CopyUse::kRecombined: words = (size_t)3 << 21; break;
+    case CopyUse::kRecombined: words = L >= 15 ? words : (size_t)3 << 21; break;
     }
     return stride >= least && count >= words / entries + 1;
 }

@@ -846,11 +846,15 @@ hipError_t launch_pointwise_tiled(const uint32_t *A, const uint32_t *B, uint32_t
     // the widest tile that still gives every CU eight waves: a wide tile re-reads
     // less, a narrow one fills the chip.  Whole products, us, with the 8x8 / 4x4 /
     // 2x2 tile: 24^3 at 2^12 points 53 / 51 / 54; 64^2x32 at 2^11 95 / 81 / 98, at 2^12
-    // 147 / 150 / 186; 64^3 at 2^10 80 / 68 / 86, at 2^12 230 / 240 / 322.
+    // 147 / 150 / 186; 64^3 at 2^10 80 / 68 / 86, at 2^12 230 / 240 / 322.  No wider
+    // than the narrow side needs, whose missing rows would be computed twice: 35x7x4
+    // at 2^15 with the 8x8 tile 106, with the 4x4 one 98.
     const size_t full = 8 * (size_t)device_cus();
     const auto waves = [&](size_t T) { return ((m + T - 1) / T) * ((n + T - 1) / T) * (npts / 64) * r; };
-    if (waves(8) >= full) return tiled_launch<8>(A, B, C, m, k, n, npts, r, p, scale, s);
-    if (waves(4) >= full) return tiled_launch<4>(A, B, C, m, k, n, npts, r, p, scale, s);
+    const size_t side = m < n ? m : n;
+    if (waves(8) >= full && side > 4) return tiled_launch<8>(A, B, C, m, k, n, npts, r, p, scale, s);
+    if (waves(4) >= full && side > 2) return tiled_launch<4>(A, B, C, m, k, n, npts, r, p, scale, s);
+    if (waves(2) >= full && side <= 2) return tiled_launch<2>(A, B, C, m, k, n, npts, r, p, scale, s);
     // too few tiles: from eight steps on the inner dimension is split, 4x4 tiles
     // while that gives half the waves, 2x2 below.  Whole products, us, 2x2 unsplit /
     // split rule: 64^3 at 2^6 points 25 / 22, at 2^8 38 / 33; 64^2x32 at 2^9 40 / 34;

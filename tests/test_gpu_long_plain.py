@@ -47,3 +47,18 @@ def test_long_plain_middle_product(ctx, p, small_left):
     PolynomialMatrixMulDomain(p, ctx, lbx.METHOD_PLAIN_U64).mul(P, A, B)
     PolynomialMatrixFFTMulDomain(p, ctx, lbx.METHOD_PLAIN_U64).midproduct(C, A, B, small_left)
     assert np.array_equal(C.to_polfirst(), P.to_polfirst()[:, hdeg - 1:2 * hdeg - 1])
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 64, 64), (2, 30, 60), (60, 5, 2), (35, 7, 4), (4, 9, 70), (5, 3, 40), (60, 2, 3)])
+@pytest.mark.parametrize("p,sa,sb", [(998244353, 8193, 8000), (2013265921, 16384, 16385), (268435399, 4000, 4097)])
+def test_narrow_plain_products(ctx, p, sa, sb, m, k, n):
+    """Products of few rows or columns on transforms that fill the chip: tiles no wider
+    than the narrow side needs, whole transforms and those of several passes."""
+    rng = np.random.default_rng(m * k * n + sa)
+    a, b = rand(rng, p, m * k * sa).reshape(m * k, sa), rand(rng, p, k * n * sb).reshape(k * n, sb)
+    a[0], b[-1] = p // 2, p - 1
+    C = PolynomialMatrix(m, n, sa + sb - 1)
+    say("narrow plain product", p, m, k, n, sa, sb)
+    PolynomialMatrixMulDomain(p, ctx, lbx.METHOD_PLAIN_U64).mul(C, PolynomialMatrix.from_polfirst(a, m, k),
+                                                               PolynomialMatrix.from_polfirst(b, k, n))
+    assert check_by_evaluation(a, b, C.to_polfirst(), p, m, k, n, sa, sb, sa + sb - 1, [int(rng.integers(1, p))])
