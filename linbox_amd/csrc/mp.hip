@@ -443,7 +443,7 @@ __global__ void __launch_bounds__(128) mp_crt_kernel(const uint32_t *__restrict_
 // p), NW words of M/p; then NW words of -M; then (MOD) off, s, the reciprocal of
 // Q's top word (div21_inverse) and NW words of Q.
 // Bound by the multiply-adds: 2047 x 1024 coefficients, 14 primes, 6 words: 140 us
-// on mixed-radix digits, 47 us here (57 with the carries rebuilt from comparisons and eight words for six).
+// on mixed-radix digits, 45 us here (57 with the carries rebuilt from comparisons and eight words for six).
 struct CrtBlock {
     static constexpr int kHead = 4;
     int r, nw;
